@@ -418,6 +418,28 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         threads = 64;
         p.dv_blocks = 1;
     }
+    // Several queries per request on average (prefill, chunked prefill,
+    // drafted tokens): the tile bodies, which read a K/V row once per tile of
+    // queries instead of once per query. They take the staged bodies' shapes
+    // and any group of up to 64 query heads (a tile then holds at least two
+    // queries), count tokens in 32 bits and write 8-byte pieces.
+    const bool tile = fast && p.dk == p.dv && (p.dk == 64 || p.dk == 128) && qp % 16 == 0 &&
+                      outp % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS / 2 &&
+                      p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
+                      lay.page_size <= (1u << 24) && c.query_count / 2 >= c.request_count &&
+                      c.query_count <= SGLKV_ATTN_TILE_QUERIES_MAX &&
+                      c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
+                      SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= (unsigned)ctx->max_lds_per_block;
+    if (tile) {
+        which = p.dk == 128 ? 12 : 13;
+        lds = SGLKV_ATTN_TILE_LDS_BYTES(p.dk);
+        threads = 256;
+        p.tile_queries = SGLKV_ATTN_TILE_ROWS / p.group;
+        p.tile_recip = UINT32_MAX / p.tile_queries + 1;
+        // Queries that come request by request make at most this many tiles.
+        const uint64_t most = c.query_count / p.tile_queries + c.request_count;
+        p.tile_slots = (uint32_t)(most < c.query_count ? most : c.query_count);
+    }
     p.zero_row = ctx->zero_row;
     p.page_stride32 = (uint32_t)lay.page_stride_bytes;
     p.key_token_stride32 = (uint32_t)p.key_token_stride;
@@ -431,9 +453,9 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     const bool wide = which >= 4 && which <= 6;  // the wide and latent bodies (7, 8, 10, 11: staged)
     const uint64_t hblocks = which == 6 ? ceil_div(p.group, SGLKV_ATTN_LATENT_HEADS)
                                         : (p.head_groups + SGLKV_ATTN_WIDE_GROUPS - 1) / SGLKV_ATTN_WIDE_GROUPS;
-    uint64_t base = c.query_count;
+    uint64_t base = tile ? p.tile_slots : c.query_count;
     if (mul_ovf(base, p.kv_heads, &base) || (wide && mul_ovf(base, hblocks, &base)) ||
-        (!wide && (mul_ovf(base, p.head_groups, &base) || mul_ovf(base, p.dv_blocks, &base))) ||
+        (!wide && !tile && (mul_ovf(base, p.head_groups, &base) || mul_ovf(base, p.dv_blocks, &base))) ||
         base > UINT32_MAX / threads)  // a dispatch counts its work-items in 32 bits
         return too_large_dim("workgroups", base, UINT32_MAX / threads);
     // The latent body has two functions: hi + lo weights (the default, as
@@ -448,7 +470,21 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     }
     const uint64_t target =
         (uint64_t)ctx->attention_occupancy[fn] * (uint64_t)(ctx->cu_count > 0 ? ctx->cu_count : 256);
-    const uint64_t want = base >= target ? 1 : target / base;
+    uint64_t live = base;
+    if (tile) {
+        // The tiles of requests that share the queries evenly (the grid
+        // leaves room for one more per request).
+        const uint64_t per_request = ceil_div(ceil_div(c.query_count, c.request_count), p.tile_queries);
+        if (per_request * c.request_count < p.tile_slots) live = per_request * c.request_count * p.kv_heads;
+    }
+    uint64_t want = live >= target ? 1 : target / live;
+    if (tile && workspace) {
+        // Never more split records than the fixed workspace holds: fewer,
+        // longer splits instead (the tile bodies take chunks of any length).
+        const uint64_t record = 4ull * (SGLKV_ATTN_OPAD(p.dv) + 2);
+        const uint64_t room = workspace_bytes / record / (c.query_count * c.query_head_count);
+        if (want > room) want = room ? room : 1;
+    }
     uint64_t chunk = ceil_div(max_len, want);
     // The shortest chunk a split takes. Small batches split further when
     // the combine merges many splits per memory round (both combines spread
@@ -465,19 +501,21 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     //    before splitting, 128 for two or three (1 query 40.0 -> 33.2 us,
     //    2 queries 41.0 -> 35.2 us), 256 from four on (best there);
     //  - the other bodies keep 256 (not measured otherwise).
-    const uint64_t min_chunk = which == 11                 ? 128
+    const uint64_t min_chunk = tile                        ? 256
+                               : which == 11               ? 128
                                : which >= 7                ? 64
                                : which == 6 && base < 4    ? (base <= 1 ? 64 : 128)
                                                            : 256;
-    chunk = ceil_div(chunk < min_chunk ? min_chunk : chunk, SGLKV_ATTN_TOKENS) * SGLKV_ATTN_TOKENS;
+    const uint64_t block = tile ? SGLKV_ATTN_TILE_BLOCK : SGLKV_ATTN_TOKENS;  // splits are whole blocks
+    chunk = ceil_div(chunk < min_chunk ? min_chunk : chunk, block) * block;
     uint64_t splits = ceil_div(max_len, chunk);
-    const uint64_t table = wide ? SGLKV_ATTN_WIDE_SLOTS : which >= 7 ? SGLKV_ATTN_STAGED_SLOTS : 0;
+    const uint64_t table = tile ? 0 : wide ? SGLKV_ATTN_WIDE_SLOTS : which >= 7 ? SGLKV_ATTN_STAGED_SLOTS : 0;
     if (table && chunk > table) {  // the slot table of the wide, latent and staged bodies
         chunk = table;
         splits = ceil_div(max_len, chunk);
     }
     if (splits > 65535) {  // grid y limit
-        chunk = ceil_div(ceil_div(max_len, 65535), SGLKV_ATTN_TOKENS) * SGLKV_ATTN_TOKENS;
+        chunk = ceil_div(ceil_div(max_len, 65535), block) * block;
         splits = ceil_div(max_len, chunk);
     }
     p.chunk_tokens = chunk;

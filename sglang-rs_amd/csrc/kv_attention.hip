@@ -24,7 +24,8 @@
 //  - long sequences are split over gridDim.y (flash-decoding): each split
 //    writes (max, sum, unnormalised output) and a combine kernel merges
 //    them, so a small batch still fills 256 CUs.
-// Five bodies share this math. The staged one (head dims 128 or 64, up to
+// Five bodies here share this math (kv_attention_tile.hip has the one for
+// launches with several queries per request). The staged one (head dims 128 or 64, up to
 // 16 query heads per KV head, 16-byte rows, power-of-two pages: every
 // Llama/Qwen-style decode) loads each block's rows straight into LDS two
 // blocks deep; the pipelined one (the other head dims up to 128 on such

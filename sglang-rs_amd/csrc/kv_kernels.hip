@@ -764,3 +764,4 @@ extern "C" __global__ __launch_bounds__(SGLKV_BLOCK_THREADS) void sglkv_stream_w
 
 // The paged-attention reader of the same pools shares this code object.
 #include "kv_attention.hip"
+#include "kv_attention_tile.hip"

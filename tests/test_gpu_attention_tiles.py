@@ -1,0 +1,133 @@
+"""GPU tests of the paged attention's tile bodies (launches with at least two
+queries per request on average: prefill, chunked prefill, drafted tokens)
+against the float64 oracle, under the bound that tests/test_gpu_attention.py
+derives: the outputs' own bf16 rounding plus 2^-12 sum_i w_i |v_i| for the
+fp32 sums (the tile bodies keep hi + lo weights and fp32 split records).
+
+A tile holds up to 128 (query, query head) rows of one request, its tokens
+come in blocks of 64, and the slot table covers 2,048 (dims 64) or 4,096
+tokens, so the sizes below sit at those edges.
+"""
+import math
+
+import numpy as np
+import pytest
+
+import sgl_rocm_kv as kv
+from sgl_rocm_kv import hip
+from test_gpu_attention import _bf16_normal, _Case, _check, _say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def k():
+    if hip.device_count() == 0:
+        pytest.fail("no GPU visible: the gpu tests need an MI355X")
+    ctx = kv.RocmKvPairCopyKernels(0)
+    yield ctx
+    ctx.close()
+
+
+def _requests(rng, spans, slot_count):
+    """Metadata of requests given as (cached tokens, queries): query j of a
+    request attends cached + j + 1 tokens."""
+    lens = np.array([c + n for c, n in spans])
+    rso = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    slots = rng.choice(slot_count, size=int(rso[-1]), replace=False).astype(np.uint64)
+    qri = np.repeat(np.arange(len(spans)), [n for _, n in spans])
+    qsl = np.concatenate([c + 1 + np.arange(n) for c, n in spans])
+    return qri, qsl, rso, slots
+
+
+@pytest.mark.parametrize("H,qh,d,P,hnd,spans", [
+    (2, 8, 128, 16, False, [(0, 1), (0, 2), (0, 31), (0, 32), (0, 33), (0, 63), (0, 64), (0, 65)]),
+    (2, 8, 128, 64, True, [(0, 300), (127, 3), (64, 64), (63, 66)]),
+    (8, 32, 128, 64, False, [(700, 5), (40, 5), (1999, 5), (3, 5)]),     # drafted tokens
+    (2, 14, 64, 16, False, [(0, 129), (2000, 150), (5, 2)]),              # groups of 7, past the slot table
+    (2, 14, 64, 1, True, [(0, 40), (0, 18), (0, 19), (1, 1)]),
+    (1, 64, 128, 64, False, [(4090, 9), (0, 3)]),                         # groups of 64: two queries a tile
+    (4, 4, 64, 64, False, [(0, 200), (0, 128), (77, 127)]),               # one head a group: 128 queries a tile
+    (2, 8, 256, 64, False, [(0, 70), (500, 5), (31, 33)]),
+    (1, 16, 256, 16, True, [(100, 40), (0, 9)]),
+    (1, 48, 128, 1, False, [(0, 21), (64, 2)]),                           # two queries a tile, 32 idle rows
+])
+def test_causal_queries(k, H, qh, d, P, hnd, spans):
+    rng = np.random.default_rng(d + qh + len(spans))
+    pages = -(-sum(c + n for c, n in spans) // P) + 3
+    c = _Case(rng, P=P, L=2, H=H, dk=d, dv=d, qh=qh, pages=pages, layer=1, hnd=hnd)
+    qri, qsl, rso, slots = _requests(rng, spans, c.layout.slot_count)
+    q = _bf16_normal(rng, len(qri) * qh * d).reshape(len(qri), qh, d)
+    _say(f"tiles H={H} qh={qh} d={d} P={P} hnd={hnd} queries={len(qri)}")
+    got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=int(qsl.max()))
+    _check(got, want, c)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_queries_in_any_order(k, d):
+    """Runs of one request cut by others, decreasing and repeated lengths,
+    and far more tiles than queries that come request by request make."""
+    rng = np.random.default_rng(d)
+    c = _Case(rng, P=16, L=1, H=2, dk=d, dv=d, qh=8, pages=120, layer=0)
+    lens = np.array([900, 333, 64])
+    rso = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    slots = rng.choice(c.layout.slot_count, size=int(rso[-1]), replace=False).astype(np.uint64)
+    qri = np.concatenate([np.arange(90) % 3, np.zeros(70, int), rng.integers(0, 3, 64), np.full(3, 2)])
+    qsl = np.array([rng.integers(1, lens[r] + 1) for r in qri])
+    qsl[90:160] = np.sort(qsl[90:160])[::-1]
+    q = _bf16_normal(rng, len(qri) * 8 * d).reshape(len(qri), 8, d)
+    _say(f"tiles in any order, d={d}, {len(qri)} queries")
+    got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=900)
+    _check(got, want, c)
+
+
+@pytest.mark.parametrize("bits", [0x7F80, 0xFF80, 0x7FC0])  # inf, -inf, NaN
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_values_past_a_query_are_not_seen(k, d, bits):
+    """Tokens 50 and 180 of a causal prompt hold infinite or NaN keys and
+    values: queries that do not attend them are as without them."""
+    rng = np.random.default_rng(d + bits)
+    c = _Case(rng, P=16, L=1, H=1, dk=d, dv=d, qh=4, pages=20, layer=0)
+    qri, qsl, rso, slots = _requests(rng, [(0, 200)], c.layout.slot_count)
+    pool16 = c.pool_h.view(np.uint16)
+    for token in (50, 180):
+        for tensor in (0, 1):
+            page, pos = divmod(int(slots[token]), 16)
+            at, end = c.layout.tensor_token_byte_range(page, 0, tensor, pos)
+            pool16[at // 2 + (token % 7):end // 2:5] = bits
+    c.pool.upload(c.pool_h)
+    q = _bf16_normal(rng, 200 * 4 * d).reshape(200, 4, d)
+    _say(f"tiles with values of 0x{bits:x} past some queries, d={d}")
+    with np.errstate(all="ignore"):
+        got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=200)
+    c.absw = c.absw[:50]
+    assert np.isfinite(got[:50]).all()
+    _check(got[:50], want[:50], c)
+
+
+@pytest.mark.parametrize("qri,qsl,flag", [([0] * 40 + [7] + [1] * 40, None, 1), (None, 0, 2), (None, 1000, 2)])
+def test_bad_metadata_is_reported(k, qri, qsl, flag):
+    """A request index past the requests, and lengths of 0 or past the
+    request's slots, raise the reference's flag bits from inside a tile."""
+    rng = np.random.default_rng(9)
+    c = _Case(rng, P=16, L=1, H=2, dk=128, dv=128, qh=8, pages=20, layer=0)
+    slots = rng.choice(c.layout.slot_count, size=200, replace=False).astype(np.uint64)
+    index = np.array(qri if qri else [0] * 40 + [1] * 41)
+    lengths = np.full(81, 60)
+    if qsl is not None:
+        lengths[33] = qsl
+    q = _bf16_normal(rng, 81 * 8 * 128).reshape(81, 8, 128)
+    with pytest.raises(kv.KvError) as e:
+        c.run(k, q, index, lengths, [0, 100, 200], slots, 0.1, max_len=2000)
+    assert e.value.variant == "DeviceMetadataInvalid" and e.value.fields[0] == flag
+
+
+def test_bad_slot_is_reported(k):
+    rng = np.random.default_rng(10)
+    c = _Case(rng, P=16, L=1, H=2, dk=128, dv=128, qh=8, pages=20, layer=0)
+    slots = rng.choice(c.layout.slot_count, size=200, replace=False).astype(np.uint64)
+    slots[70] = c.layout.slot_count
+    q = _bf16_normal(rng, 64 * 8 * 128).reshape(64, 8, 128)
+    with pytest.raises(kv.KvError) as e:
+        c.run(k, q, np.zeros(64, int), 100 + np.arange(64), [0, 200], slots, 0.1, max_len=200)
+    assert e.value.variant == "DeviceMetadataInvalid" and e.value.fields[0] == 4
