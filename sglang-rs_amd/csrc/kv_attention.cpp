@@ -552,13 +552,15 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         }
         p.partial = static_cast<float *>(workspace ? workspace : ctx->attention_partial);
     }
-    // The combine pass: one workgroup per (query, head); the fp16 one in
-    // blocks of 64 per 8 groups of 8 heads (its XCD map), padded.
+    // The combine pass: the workgroup's sets of threads, SGLKV_ATTN_COMBINE_PER
+    // to a (query, head); the fp16 one in blocks of 64 per 8 groups of 8 heads
+    // (its XCD map), padded.
     uint64_t combine_grid = 0;
     if (splits > 1) {
         uint64_t heads;
         if (mul_ovf(c.query_count, c.query_head_count, &heads)) return attn_overflow();
-        combine_grid = half_records ? 64 * ceil_div(c.query_count * ceil_div(c.query_head_count, 8), 8) : heads;
+        combine_grid = half_records ? 64 * ceil_div(c.query_count * ceil_div(c.query_head_count, 8), 8)
+                                    : ceil_div(heads, SGLKV_ATTN_COMBINE_SETS(p.dv) / SGLKV_ATTN_COMBINE_PER(p.dv, p.splits));
         const uint64_t limit = UINT32_MAX / (half_records ? 256 : 128);  // work-items in 32 bits
         if (heads > limit / 2 || combine_grid > limit)
             return too_large_dim("combine workgroups", heads, limit / 2);
@@ -567,7 +569,7 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     SGLKV_CHECK_HIP(hipModuleLaunchKernel(ctx->attention[fn], (unsigned)base, (unsigned)splits, 1, threads,
                                           1, 1, lds, s, args, nullptr));
     // The fp16 combine: one wave per group of eight splits, up to four.
-    const unsigned combine_threads = half_records ? 64 * (unsigned)(splits > 24 ? 4 : ceil_div(splits, 8)) : 128;
+    const unsigned combine_threads = half_records ? 64 * (unsigned)(splits > 24 ? 4 : ceil_div(splits, 8)) : SGLKV_ATTN_COMBINE_THREADS;
     if (splits > 1)
         SGLKV_CHECK_HIP(hipModuleLaunchKernel(half_records ? ctx->attention_combine_h : ctx->attention_combine,
                                               (unsigned)combine_grid, 1, 1, combine_threads, 1, 1, 0, s, args,

@@ -2276,71 +2276,80 @@ __device__ __forceinline__ void attn_combine_groups(const float2 *ml, const floa
     }
 }
 
-// Merges the split records of one (query, head): m* = max m_s,
-// out = sum_s 2^(m_s - m*) o_s / sum_s 2^(m_s - m*) l_s. Thread t handles
+// Merges the split records of each (query, head): m* = max m_s,
+// out = sum_s 2^(m_s - m*) o_s / sum_s 2^(m_s - m*) l_s. A thread handles
 // dims 4t .. 4t+3 of each split's o row (one 16-byte read; rows are
 // 128-byte aligned, dims past dv read the row's padding and are not
 // written). A row of dv < 512 dims needs only ceil(dv / 4) threads: the
-// workgroup's threads then form `sets` of that many, set i merging split
-// groups i, i + sets, ..., and set 0 merges the sets' partial (m, l, o)
-// through LDS, so a query split many ways waits for one memory latency per
-// `sets` groups of eight splits, not per group.
-extern "C" __global__ __launch_bounds__(128) void sglkv_paged_attention_combine(sglkv_attn_params p) {
-    __shared__ float part[128][6];  // m, l, o[4] of each thread of sets 1..
-    const uint64_t q = blockIdx.x / p.query_heads;
-    const uint32_t head = static_cast<uint32_t>(blockIdx.x % p.query_heads);
-    uint64_t start = 0, len = 0;
-    if (!attn_metadata(p, q, false, &start, &len)) return;  // uniform over the workgroup
-    const uint32_t used = static_cast<uint32_t>((len + p.chunk_tokens - 1) / p.chunk_tokens);
-    const uint64_t i0 = (q * p.query_heads + head) * p.splits;
-    const float2 *ml = reinterpret_cast<const float2 *>(attn_rec_ml(p, i0));
-    const float *o = attn_rec_o(p, i0);
-    const uint32_t opad = SGLKV_ATTN_OPAD(p.dv);
-    uint16_t *out = p.output + (q * p.query_heads + head) * p.dv;
-    const uint32_t pieces = (p.dv + 3) / 4;
-    const uint32_t lanes = pieces < blockDim.x ? pieces : blockDim.x;
-    const uint32_t sets = blockDim.x / lanes, set = threadIdx.x / lanes, tl = threadIdx.x % lanes;
-    auto write = [&](uint32_t d, float m, float l, const float (&acc)[4]) {
-        (void)m;
-        const float linv = 1.0f / l;
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e)
-            if (d + e < p.dv) out[d + e] = attn_to_bf16(acc[e] * linv);
-    };
-    if (sets == 1 || used <= 8) {  // (uniform over the workgroup: one query's splits)
-        for (uint32_t d = 4 * threadIdx.x; d < p.dv; d += 4 * blockDim.x) {
+// workgroup's threads then form sets of that many. A (query, head) takes
+// SGLKV_ATTN_COMBINE_PER sets, one per group of eight splits as far as they
+// go: set i merges groups i, i + per, ..., and set 0 merges the sets' partial
+// (m, l, o) through LDS, so a query split many ways waits for one memory
+// latency per `per` groups, not per group; and the sets left over take other
+// (query, head)s, so that launches of many queries split a few ways have all
+// threads at work in a fraction of the workgroups. Latency bounds it (a
+// chain of metadata, records and one store). Measured on MI355X against one
+// (query, head) per workgroup: 5,376 of dims 64 in 16 splits 10.0 -> 6.4 us;
+// per layer of a decode, 16 queries x 32 heads of dims 64 23.1 -> 21.8 us and
+// 1 query x 32 heads of dims 128 in 64 splits 14.9 -> 14.1 us.
+extern "C" __global__ __launch_bounds__(SGLKV_ATTN_COMBINE_THREADS) void sglkv_paged_attention_combine(
+    sglkv_attn_params p) {
+    __shared__ float part[SGLKV_ATTN_COMBINE_THREADS][6];  // m, l, o[4] of each thread
+    const uint32_t lanes = SGLKV_ATTN_COMBINE_LANES(p.dv), sets = SGLKV_ATTN_COMBINE_THREADS / lanes;
+    const uint32_t per = SGLKV_ATTN_COMBINE_PER(p.dv, p.splits), items = sets / per;
+    const uint32_t set = threadIdx.x / lanes, tl = threadIdx.x % lanes;
+    const uint32_t own = set / per, sub = set - own * per;
+    // The set's (query, head) number `item` (below 2^31: the host's limit).
+    auto merge = [&](uint32_t item, bool inside) {
+        const uint32_t q = item / p.query_heads;
+        uint64_t start = 0, len = 0;
+        const bool ok = inside && q < p.query_count && attn_metadata(p, q, false, &start, &len);
+        const uint32_t used = static_cast<uint32_t>((len + p.chunk_tokens - 1) / p.chunk_tokens);
+        const uint64_t i0 = static_cast<uint64_t>(item) * p.splits;
+        const float2 *ml = reinterpret_cast<const float2 *>(attn_rec_ml(p, i0));
+        const float *o = attn_rec_o(p, i0);
+        const uint32_t opad = SGLKV_ATTN_OPAD(p.dv);
+        uint16_t *out = p.output + static_cast<uint64_t>(item) * p.dv;
+        for (uint32_t d0 = 0; d0 < p.dv; d0 += 4 * lanes) {  // (one pass where lanes cover dv: always if sets > 1)
+            const uint32_t d = d0 + 4 * tl;
+            // A set with no group keeps m = -FLT_MAX, l = 0, o = 0, which the
+            // merge weighs 0.
             float m = -3.402823466e+38f, l = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            attn_combine_groups(ml, o, opad, d, used, 0, 8, m, l, acc);
-            write(d, m, l, acc);
+            if (ok && d < p.dv) attn_combine_groups(ml, o, opad, d, used, 8 * sub, 8 * per, m, l, acc);
+            if (per > 1) {  // (uniform)
+                float *pw = part[threadIdx.x];
+                if (sub > 0) {
+                    pw[0] = m;
+                    pw[1] = l;
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) pw[2 + e] = acc[e];
+                }
+                __syncthreads();
+                if (sub == 0) {
+                    for (uint32_t k = 1; k < per; ++k) {
+                        const float *pk = pw + 6 * k * lanes;
+                        const float m_new = fmaxf(m, pk[0]);
+                        const float a = exp2f(m - m_new), b = exp2f(pk[0] - m_new);
+                        l = l * a + pk[1] * b;
+#pragma unroll
+                        for (uint32_t e = 0; e < 4; ++e) acc[e] = acc[e] * a + pk[2 + e] * b;
+                        m = m_new;
+                    }
+                }
+            }
+            if (!ok || sub != 0) continue;
+            const float linv = 1.0f / l;
+#pragma unroll
+            for (uint32_t e = 0; e < 4; ++e)
+                if (d + e < p.dv) out[d + e] = attn_to_bf16(acc[e] * linv);
         }
-        return;
-    }
-    // One 4-dim piece per thread (4 * lanes >= dv); threads past the last
-    // whole set (blockDim.x % lanes of them) only join the barrier. A set
-    // with no group keeps m = -FLT_MAX, l = 0, o = 0, which the merge
-    // weighs 0.
-    const uint32_t d = 4 * tl;
-    float m = -3.402823466e+38f, l = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (set < sets) attn_combine_groups(ml, o, opad, d, used, 8 * set, 8 * sets, m, l, acc);
-    if (set > 0 && set < sets) {
-        float *pw = part[threadIdx.x];
-        pw[0] = m;
-        pw[1] = l;
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) pw[2 + e] = acc[e];
-    }
-    __syncthreads();
-    if (set != 0) return;
-    for (uint32_t k = 1; k < sets; ++k) {
-        const float *pw = part[k * lanes + tl];
-        const float m_new = fmaxf(m, pw[0]);
-        const float a = exp2f(m - m_new), b = exp2f(pw[0] - m_new);
-        l = l * a + pw[1] * b;
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) acc[e] = acc[e] * a + pw[2 + e] * b;
-        m = m_new;
-    }
-    write(d, m, l, acc);
+    };
+    // One (query, head) a workgroup (long splits: a small launch, where the
+    // latency counts): its metadata in scalar registers.
+    if (items == 1)
+        merge(blockIdx.x, own == 0);
+    else
+        merge(blockIdx.x * items + own, own < items);
 }
 
 // The latent body's records (scaled fp16, SGLKV_ATTN_HPAD): the merge

@@ -215,6 +215,14 @@ typedef struct sglkv_request_params {
  * (rows padded to whole 128-byte lines, so that the writes fill every line
  * they touch) and its m, l at partial + records * SGLKV_ATTN_OPAD(dv) + 2 i. */
 #define SGLKV_ATTN_OPAD(dv) (((dv) + 31u) & ~31u)
+/* The combine kernel: threads of a workgroup, threads of a set (one 4-dim
+ * piece of a row each) and sets per (query, head). */
+#define SGLKV_ATTN_COMBINE_THREADS 128u
+#define SGLKV_ATTN_COMBINE_LANES(dv)                                                               \
+    (((dv) + 3u) / 4u < SGLKV_ATTN_COMBINE_THREADS ? ((dv) + 3u) / 4u : SGLKV_ATTN_COMBINE_THREADS)
+#define SGLKV_ATTN_COMBINE_SETS(dv) (SGLKV_ATTN_COMBINE_THREADS / SGLKV_ATTN_COMBINE_LANES(dv))
+#define SGLKV_ATTN_COMBINE_PER(dv, splits)                                                         \
+    (((splits) + 7u) / 8u < SGLKV_ATTN_COMBINE_SETS(dv) ? ((splits) + 7u) / 8u : SGLKV_ATTN_COMBINE_SETS(dv))
 /* The latent body's split records are scaled fp16: record i keeps
  * y[dv] = o / a at partial + i * SGLKV_ATTN_HPAD(dv) halves (rows of whole
  * 128-byte lines), a = max |o| over the record (so |y| <= 1), and
