@@ -421,20 +421,20 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     // Several queries per request on average (prefill, chunked prefill,
     // drafted tokens): the tile bodies, which read a K/V row once per tile of
     // queries instead of once per query. They take the staged bodies' shapes
-    // and any group of up to 64 query heads (a tile then holds at least two
+    // and any group of up to 64 query heads, 32 at dims 256 (a tile then holds at least two
     // queries), count tokens in 32 bits and write 8-byte pieces.
-    const bool tile = fast && p.dk == p.dv && (p.dk == 64 || p.dk == 128) && qp % 16 == 0 &&
-                      outp % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS / 2 &&
+    const bool tile = fast && p.dk == p.dv && (p.dk == 64 || p.dk == 128 || p.dk == 256) && qp % 16 == 0 &&
+                      outp % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) / 2 &&
                       p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
                       lay.page_size <= (1u << 24) && c.query_count / 2 >= c.request_count &&
                       c.query_count <= SGLKV_ATTN_TILE_QUERIES_MAX &&
                       c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
                       SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= (unsigned)ctx->max_lds_per_block;
     if (tile) {
-        which = p.dk == 128 ? 12 : 13;
+        which = p.dk == 128 ? 12 : p.dk == 64 ? 13 : 14;
         lds = SGLKV_ATTN_TILE_LDS_BYTES(p.dk);
         threads = 256;
-        p.tile_queries = SGLKV_ATTN_TILE_ROWS / p.group;
+        p.tile_queries = SGLKV_ATTN_TILE_ROWS(p.dk) / p.group;
         p.tile_recip = UINT32_MAX / p.tile_queries + 1;
         // Queries that come request by request make at most this many tiles.
         const uint64_t most = c.query_count / p.tile_queries + c.request_count;
@@ -485,6 +485,7 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         const uint64_t room = workspace_bytes / record / (c.query_count * c.query_head_count);
         if (want > room) want = room ? room : 1;
     }
+    if (tile && want > max_len / 256) want = max_len >= 512 ? max_len / 256 : 1;  // splits of 256 tokens or more
     uint64_t chunk = ceil_div(max_len, want);
     // The shortest chunk a split takes. Small batches split further when
     // the combine merges many splits per memory round (both combines spread
@@ -501,12 +502,12 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     //    before splitting, 128 for two or three (1 query 40.0 -> 33.2 us,
     //    2 queries 41.0 -> 35.2 us), 256 from four on (best there);
     //  - the other bodies keep 256 (not measured otherwise).
-    const uint64_t min_chunk = tile                        ? 256
+    const uint64_t min_chunk = tile                        ? 0
                                : which == 11               ? 128
                                : which >= 7                ? 64
                                : which == 6 && base < 4    ? (base <= 1 ? 64 : 128)
                                                            : 256;
-    const uint64_t block = tile ? SGLKV_ATTN_TILE_BLOCK : SGLKV_ATTN_TOKENS;  // splits are whole blocks
+    const uint64_t block = tile ? SGLKV_ATTN_TILE_BLOCK(p.dk) : SGLKV_ATTN_TOKENS;  // splits are whole blocks
     chunk = ceil_div(chunk < min_chunk ? min_chunk : chunk, block) * block;
     uint64_t splits = ceil_div(max_len, chunk);
     const uint64_t table = tile ? 0 : wide ? SGLKV_ATTN_WIDE_SLOTS : which >= 7 ? SGLKV_ATTN_STAGED_SLOTS : 0;

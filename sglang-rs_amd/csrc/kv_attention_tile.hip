@@ -7,13 +7,14 @@
 // fills only `group` of the 16 columns of its matrix products. Here a
 // workgroup of four waves owns a tile: up to tile_queries consecutive queries
 // of one request, whose query heads of one KV head are the tile's rows
-// (row = query * group + head, at most 128, 32 per wave). Every K and V row is
-// staged in LDS once per tile.
+// (row = query * group + head, at most 128, 32 per wave; at dims 256, whose
+// outputs of 32 rows are too many registers for one wave, 64 rows, 32 per pair
+// of waves: both compute the scores, each has half the value dims). Every K and
+// V row is staged in LDS once per tile.
 //  - Tiles. A run is a maximal stretch of consecutive queries of one request;
 //    it is cut into tiles of tile_queries from its start, and tiles are
 //    numbered over all runs. Which queries tile t holds is found from
-//    query_request_indices by every wave on its own (64 queries a step,
-//    ballots and scalar arithmetic), so queries of different requests never
+//    query_request_indices by the workgroup itself (attn_tile_find), so queries of different requests never
 //    share a tile whatever their order, and no planning launch or device list
 //    is needed. The host launches tile_slots tiles per KV head, enough for
 //    queries that come request by request; workgroups step by tile_slots, so
@@ -39,91 +40,143 @@
 //    pc ^ vswz(t), chosen so that the 16 tokens of a q.k read, and the four
 //    tokens of a half-wave's transposing read, land in distinct banks.
 // What bounds it: the matrix products (48 per 64-token block and wave at dims
-// 128, 32 of them p.v's, hi and lo) and the softmax between them, on two waves
-// per SIMD. Measured on MI355X, per layer: causal prompts of 300..2,048 tokens
-// (5,206 queries, 32 heads over 8, dims 128) 1,744 -> 206 us, 322 TFLOP/s of
-// q.k and p.v; 384 queries over 6,144 tokens (14 heads over 2, dims 64)
-// 112 -> 41 us.
+// 128, 32 of them p.v's, hi and lo) and the softmax's vector instructions (about
+// as long), on two waves per SIMD; for short prompts the chain of loads before
+// the first block (about 6 us). Measured on MI355X, per layer, against the
+// per-query bodies:
+//   causal prompts of 300..2,048 tokens (5,206 queries, 32 heads over 8, dims
+//   128): 1,744 -> 129 us (517 TFLOP/s of q.k and p.v; 688 where 2,048 queries
+//   each attend 6,144..8,192 tokens);
+//   384 queries over 6,144 tokens (14 heads over 2, dims 64): 112 -> 36 us;
+//   5 queries of each of 24 requests of 200..3,000 tokens (8 heads over 2, dims
+//   256): 109 -> 45 us.
+// Of these, the search for the tile's queries in one step of 4,096 (not 128
+// at a time) took the prompts from 185 to 135 us, and products at raised wave
+// priority with the next step's weights scheduled between them 388 -> 350 us on
+// the 8,192-token shape.
 
 namespace {
+
+constexpr uint32_t kTileAhead = 4;  // products that the K reads run ahead
 
 template <uint32_t D>
 struct attn_tl {
     static constexpr uint32_t ROW = 2 * D;                // bytes of one token's head slice
     static constexpr uint32_t PIECES = D / 8;             // 16-byte pieces per row
     static constexpr uint32_t TPL = 1024 / ROW;           // tokens per load
-    static constexpr uint32_t B = SGLKV_ATTN_TILE_BLOCK;  // tokens per block
+    static constexpr uint32_t B = SGLKV_ATTN_TILE_BLOCK(D);  // tokens per block
     static constexpr uint32_t LPW = B / TPL / 4;          // K loads (and V loads) of a wave per block
     static constexpr uint32_t V = B * ROW;                // V rows' offset in a stage
     static constexpr uint32_t STAGE = 2 * V;
     static constexpr uint32_t TABLE = SGLKV_ATTN_TILE_SLOTS(D);  // slot table entries (whole blocks)
     static constexpr uint32_t KC = D / 16;                // q.k steps
-    static constexpr uint32_t NT = D / 32;                // 32-dim output tiles
+    static constexpr uint32_t ROWS = SGLKV_ATTN_TILE_ROWS(D);  // (query, head) rows per tile
+    static constexpr uint32_t SHARE = 4 * 32 / ROWS;      // waves that share 32 rows, each with D / SHARE outputs
+    static constexpr uint32_t NT = D / SHARE / 32;        // 32-dim output tiles of a wave
     static constexpr uint32_t TB = B / 32;                // 32-token score tiles
-    static_assert(D == 64 || D == 128, "head dims");
+    static_assert(D == 64 || D == 128 || D == 256, "head dims");
     static_assert(2 * STAGE + 4 * TABLE == SGLKV_ATTN_TILE_LDS_BYTES(D), "the host sizes the same LDS");
     static_assert(LPW * TPL * 4 == B && TABLE % B == 0, "whole loads and blocks");
-    // K: 256-byte rows start on a bank period, so 16 tokens need 16
+    // K: 256- and 512-byte rows start on a bank period, so 16 tokens need 16
     // positions; 128-byte rows leave t & 1 apart already.
-    static __device__ __forceinline__ uint32_t kswz(uint32_t t) { return D == 128 ? t & 15 : (t >> 1) & 7; }
+    static __device__ __forceinline__ uint32_t kswz(uint32_t t) { return D >= 128 ? t & 15 : (t >> 1) & 7; }
     // V: four tokens' 64-byte spans in the four quarters of a bank period.
-    static __device__ __forceinline__ uint32_t vswz(uint32_t t) { return D == 128 ? (t & 3) << 2 : (t & 2) << 1; }
+    static __device__ __forceinline__ uint32_t vswz(uint32_t t) { return D >= 128 ? (t & 3) << 2 : (t & 2) << 1; }
 };
 
-// Queries [q0, q0 + nq) of tile `want`, or false if there are fewer tiles.
-// Uniform over the wave; every wave of a workgroup finds the same answer.
-__device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint32_t want, uint32_t lane,
-                                               uint32_t *q0, uint32_t *nq) {
-    constexpr uint32_t U = 2;  // 64-query steps whose loads are issued together
+// Queries [q0, q0 + nq) of tile `want`, or false if there are fewer tiles
+// (uniform over the workgroup). `masks`: 512 bytes of LDS. 4,096 queries a
+// step: each wave ballots where runs start in 16 stretches of 64 queries (its
+// loads all in flight at once: stepping through 128 queries at a time by one
+// wave, each step a memory latency, took most of a short tile's time), then
+// lane l of every wave takes stretch l, counts the tiles that start in it and
+// sums over the lanes.
+__device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint32_t want, uint32_t w, uint32_t lane,
+                                               uint64_t *masks, uint32_t *q0, uint32_t *nq, uint32_t *request) {
+    constexpr uint32_t U = 16, STEP = 4 * U * 64;
     const uint32_t count = static_cast<uint32_t>(p.query_count);  // host: at most SGLKV_ATTN_TILE_QUERIES_MAX
     const uint32_t *req = p.query_request_indices;
-    // ceil(x / tile_queries) for x below 2^24 (the host's reciprocal is exact there)
+    // ceil(x / tile_queries) for x up to 2^24 (the host's reciprocal is exact there)
     auto tiles_to = [&](uint32_t x) { return __umulhi(x + p.tile_queries - 1, p.tile_recip); };
-    uint32_t seen = 0, run = 0;
+    // Walks the runs of one stretch: queries [from, from + n), `starts` its
+    // run starts, `run` the start of the run that it begins in. Counts the
+    // tiles that start there; the k-th (from 0) starts at *at.
+    auto walk = [&](uint32_t from, uint32_t n, uint64_t starts, uint32_t run, uint32_t k, uint32_t *at) {
+        uint32_t tiles = 0;
+        for (uint32_t pos = 0; pos < n;) {
+            if ((starts >> pos) & 1) run = from + pos;
+            const uint64_t rest = starts & ~((2ull << pos) - 1);
+            const uint32_t next = rest ? static_cast<uint32_t>(__builtin_ctzll(rest)) : n;
+            const uint32_t a = tiles_to(from + pos - run), b = tiles_to(from + next - run);
+            if (k - tiles < b - a) *at = run + (a + k - tiles) * p.tile_queries;
+            tiles += b - a;
+            pos = next;
+        }
+        return tiles;
+    };
+    uint32_t seen = 0, run = 0, first = 0;
     bool found = false;
-    uint32_t first = 0;
-    for (uint32_t base = 0; base < count && !found; base += 64 * U) {
+    for (uint32_t base = 0; base < count && !found; base += STEP) {
         uint32_t cur[U], before[U];
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
-            const uint32_t i = base + 64 * u + lane, at = i < count ? i : count - 1;
-            cur[u] = req[at];
-            before[u] = req[at ? at - 1 : 0];
+            // (Past the last query both are that query: no start.)
+            const uint32_t i = base + 64 * (U * w + u) + lane, at = i < count ? i : count;
+            cur[u] = req[i < count - 1 ? i : count - 1];
+            before[u] = req[(at > 1 ? at : 1) - 1];
         }
+        __syncthreads();  // the table that the masks overlay is no longer read
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
-            const uint32_t c0 = base + 64 * u;
-            if (c0 >= count || found) break;
-            const uint32_t n = count - c0 < 64 ? count - c0 : 64;
-            uint64_t starts = __ballot(lane < n && (c0 + lane == 0 || cur[u] != before[u]));
-            for (uint32_t pos = 0; pos < n;) {
-                if ((starts >> pos) & 1) run = c0 + pos;
-                starts &= ~(1ull << pos);
-                const uint32_t next = starts ? static_cast<uint32_t>(__builtin_ctzll(starts)) : n;
-                const uint32_t a = tiles_to(c0 + pos - run), b = tiles_to(c0 + next - run);
-                if (want - seen < b - a) {
-                    first = run + (a + want - seen) * p.tile_queries;
-                    found = true;
-                    break;
-                }
-                seen += b - a;
-                pos = next;
-            }
+            const uint64_t starts = __ballot(cur[u] != before[u]) | (base + w + u == 0 ? 1 : 0);
+            if (lane == 0) masks[U * w + u] = starts;
         }
+        __syncthreads();
+        const uint64_t starts = masks[lane];
+        const uint32_t from = base + 64 * lane;
+        const uint32_t n = from >= count ? 0 : (count - from < 64 ? count - from : 64);
+        // Start of the last run at or before the stretch's end: a running
+        // maximum over the lanes (and what came before).
+        uint32_t last = starts ? from + 63 - static_cast<uint32_t>(__builtin_clzll(starts)) : run;
+#pragma unroll
+        for (uint32_t d = 1; d < 64; d <<= 1) {
+            const uint32_t x = __shfl_up(last, d);
+            last = lane >= d && x > last ? x : last;
+        }
+        const uint32_t x = __shfl_up(last, 1), in = lane ? x : run;
+        uint32_t unused;
+        const uint32_t mine = walk(from, n, starts, in, 0xFFFFFFFFu, &unused);
+        uint32_t sum = mine;
+#pragma unroll
+        for (uint32_t d = 1; d < 64; d <<= 1) {
+            const uint32_t x = __shfl_up(sum, d);
+            sum += lane >= d ? x : 0u;
+        }
+        const uint64_t here = __ballot(want - seen < sum);  // (want >= seen)
+        if (here) {
+            const int l = __builtin_ctzll(here);
+            const uint32_t k = want - seen - __shfl(sum - mine, l);
+            const uint64_t bits = static_cast<uint64_t>(__shfl(static_cast<uint32_t>(starts >> 32), l)) << 32 |
+                                  __shfl(static_cast<uint32_t>(starts), l);
+            walk(base + 64 * l, __shfl(n, l), bits, __shfl(in, l), k, &first);
+            found = true;
+        }
+        seen += __shfl(sum, 63);
+        run = __shfl(last, 63);
     }
     if (!found) return false;
     first = __builtin_amdgcn_readfirstlane(first);
-    // The tile ends with its run or after tile_queries (at most 128).
-    const uint32_t own = req[first];
-    auto leading = [&](uint32_t from) {  // queries from `from` on that are own's, up to 64
-        const uint32_t i = from + lane;
-        const uint64_t other = ~__ballot(i < count && req[i < count ? i : count - 1] == own);
-        return other ? static_cast<uint32_t>(__builtin_ctzll(other)) : 64u;
-    };
-    uint32_t len = leading(first);
-    if (len == 64 && p.tile_queries > 64) len += leading(first + 64);
+    // The tile ends with its run or after tile_queries (at most 128): how
+    // many of the queries from `first` on are of its request.
+    const uint32_t i = first + lane, j = i + 64;
+    const uint32_t ri = req[i < count ? i : count - 1], rj = req[j < count ? j : count - 1];
+    const uint32_t own = __builtin_amdgcn_readfirstlane(ri);
+    const uint64_t oi = ~__ballot(i < count && ri == own), oj = ~__ballot(j < count && rj == own);
+    const uint32_t len = oi ? static_cast<uint32_t>(__builtin_ctzll(oi))
+                            : 64 + (oj ? static_cast<uint32_t>(__builtin_ctzll(oj)) : 64u);
     *q0 = first;
     *nq = len < p.tile_queries ? len : p.tile_queries;
+    *request = own;
     return true;
 }
 
@@ -190,32 +243,57 @@ __device__ __forceinline__ void attn_tile_issue(const sglkv_attn_params &p, uint
     }
 }
 
+// Two floats rounded to bf16 (to nearest even), the first in the low half:
+// one instruction for what element by element takes two and a pack.
+__device__ __forceinline__ uint32_t attn_pack_bf16(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
+__device__ __forceinline__ float attn_max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
+
 template <uint32_t D>
 struct attn_tile_state {
     float m_run, l_part;              // row l % 32 (both half-waves hold the same m; l is this half's share)
-    sglkv_f32x16 o[attn_tl<D>::NT];   // o[n][i]: dim 32n + 8(i/4) + 4(l/32) + i%4 of the row
+    sglkv_f32x16 o[attn_tl<D>::NT];   // o[n][i]: dim 32n + 8(i/4) + 4(l/32) + i%4 of the wave's dims of the row
 };
 
 // One block from its stage: scores, softmax, o += p.v. `left`: the row's
 // tokens from the block's first on (signed); masked: some row of the wave
-// ends inside the block.
+// ends inside the block. part: which of the SHARE waves of these rows.
 template <uint32_t D>
 __device__ __forceinline__ void attn_tile_block(const sglkv_attn_params &p, const uint8_t *st_lds,
                                                 const sglkv_u16x8 (&qf)[attn_tl<D>::KC], int32_t left, bool masked,
-                                                uint32_t lane, attn_tile_state<D> &st) {
+                                                uint32_t lane, uint32_t part, attn_tile_state<D> &st) {
     typedef attn_tl<D> T;
     const uint32_t t = lane & 31, h = lane >> 5;
     sglkv_f32x16 s[T::TB];
 #pragma unroll
     for (uint32_t b = 0; b < T::TB; ++b) s[b] = sglkv_f32x16{};
+    // The K reads run kTileAhead products ahead (sched_barrier keeps the
+    // order: the scheduler would sink each read next to its product, which
+    // then waits for the LDS).
+    auto kread = [&](uint32_t i) {
+        return *reinterpret_cast<const sglkv_u16x8 *>(st_lds + T::ROW * (32 * (i % T::TB) + t) +
+                                                      16 * ((2 * (i / T::TB) + h) ^ T::kswz(t)));
+    };
+    // Products run at raised wave priority, the softmax between them at the
+    // normal one: otherwise the older of a SIMD's two waves, in its softmax,
+    // takes every issue slot and the matrix cores of the other wait.
+    __builtin_amdgcn_s_setprio(1);
+    sglkv_u16x8 kf[kTileAhead];
 #pragma unroll
-    for (uint32_t c = 0; c < T::KC; ++c)
+    for (uint32_t i = 0; i < kTileAhead; ++i) kf[i] = kread(i);
 #pragma unroll
-        for (uint32_t b = 0; b < T::TB; ++b) {
-            const sglkv_u16x8 kf = *reinterpret_cast<const sglkv_u16x8 *>(
-                st_lds + T::ROW * (32 * b + t) + 16 * ((2 * c + h) ^ T::kswz(t)));
-            s[b] = attn_mfma32(kf, qf[c], s[b]);
-        }
+    for (uint32_t i = 0; i < T::KC * T::TB; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        const sglkv_u16x8 a = kf[i % kTileAhead];
+        s[i % T::TB] = attn_mfma32(a, qf[i / T::TB], s[i % T::TB]);
+        if (i + kTileAhead < T::KC * T::TB) kf[i % kTileAhead] = kread(i + kTileAhead);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
     if (masked) {
         // Bitwise selects (all ones where the token is below `left`): a
         // compare per element would hold 32 lane masks in scalar registers.
@@ -232,7 +310,7 @@ __device__ __forceinline__ void attn_tile_block(const sglkv_attn_params &p, cons
 #pragma unroll
     for (uint32_t b = 0; b < T::TB; ++b)
 #pragma unroll
-        for (uint32_t i = 0; i < 16; ++i) mx = fmaxf(mx, s[b][i]);
+        for (uint32_t i = 0; i < 16; i += 2) mx = attn_max3(mx, s[b][i], s[b][i + 1]);
     mx = fmaxf(mx, attn_xor32(mx)) * p.scale_log2;
     if (__builtin_amdgcn_readfirstlane(__ballot(mx > st.m_run + 8.0f) != 0 ? 1u : 0u)) {
         const float m_new = fmaxf(st.m_run, mx);
@@ -248,30 +326,64 @@ __device__ __forceinline__ void attn_tile_block(const sglkv_attn_params &p, cons
     // 4h + L/4 and + 8 (the same vswz), dims 32n + 16c + 4(L%4).
     const uint32_t L = lane & 15, c = (lane >> 4) & 1, t0 = 4 * h + (L >> 2);
     auto vread = [&](uint32_t n, uint32_t step) {
-        const uint32_t pc = (4 * n + 2 * c + ((L & 3) >> 1)) ^ T::vswz(t0);
+        const uint32_t pc = (4 * (T::NT * part + n) + 2 * c + ((L & 3) >> 1)) ^ T::vswz(t0);
         const uint8_t *at = st_lds + T::V + T::ROW * (16 * step + t0) + 16 * pc + 8 * (L & 1);
         const attn_i16x4 lo = attn_lat_vtr(at), hi = attn_lat_vtr(at + 8 * T::ROW);
         return sglkv_u16x8{(uint16_t)lo[0], (uint16_t)lo[1], (uint16_t)lo[2], (uint16_t)lo[3],
                            (uint16_t)hi[0], (uint16_t)hi[1], (uint16_t)hi[2], (uint16_t)hi[3]};
     };
+    // Step `step`'s weights, hi and lo.
     float psum = 0.0f;
+    auto weights = [&](uint32_t step, sglkv_u16x8 &phi, sglkv_u16x8 &plo) {
+        attn_u32x4 hi, lo;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t e = 8 * (step & 1) + 2 * i;
+            const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(s[step >> 1][e], p.scale_log2, -st.m_run));
+            const float b = __builtin_amdgcn_exp2f(__builtin_fmaf(s[step >> 1][e + 1], p.scale_log2, -st.m_run));
+            psum += a;
+            psum += b;
+            hi[i] = attn_pack_bf16(a, b);
+            lo[i] = attn_pack_bf16(a - __uint_as_float(hi[i] << 16), b - __uint_as_float(hi[i] & 0xFFFF0000u));
+        }
+        phi = __builtin_bit_cast(sglkv_u16x8, hi);
+        plo = __builtin_bit_cast(sglkv_u16x8, lo);
+    };
+    // (Dims 256 have no registers for two steps' values.)
+    constexpr uint32_t VBUF = D > 128 ? 1 : 2;
+    sglkv_u16x8 phi[2], plo[2], v[VBUF][T::NT];
+    if (VBUF == 2) {
+#pragma unroll
+        for (uint32_t n = 0; n < T::NT; ++n) v[0][n] = vread(n, 0);
+    }
+    weights(0, phi[0], plo[0]);
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (uint32_t step = 0; step < 2 * T::TB; ++step) {
-        sglkv_u16x8 phi, plo;
+        // A step's products, with the next step's value reads and weights
+        // scheduled between them (one read and a share of the vector
+        // instructions behind each product).
+        const uint32_t x = step & 1;
+        __builtin_amdgcn_sched_barrier(0);
+        if (VBUF == 1 || step + 1 < 2 * T::TB) {
 #pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) {
-            const float pr =
-                __builtin_amdgcn_exp2f(__builtin_fmaf(s[step >> 1][8 * (step & 1) + i], p.scale_log2, -st.m_run));
-            psum += pr;
-            attn_split_bf16(pr, phi, plo, i);
+            for (uint32_t n = 0; n < T::NT; ++n) v[(x + 1) % VBUF][n] = vread(n, VBUF == 2 ? step + 1 : step);
         }
 #pragma unroll
-        for (uint32_t n = 0; n < T::NT; ++n) {
-            const sglkv_u16x8 v = vread(n, step);
-            st.o[n] = attn_mfma32(v, phi, st.o[n]);
-            st.o[n] = attn_mfma32(v, plo, st.o[n]);
+        for (uint32_t n = 0; n < T::NT; ++n) st.o[n] = attn_mfma32(v[x % VBUF][n], phi[x], st.o[n]);
+#pragma unroll
+        for (uint32_t n = 0; n < T::NT; ++n) st.o[n] = attn_mfma32(v[x % VBUF][n], plo[x], st.o[n]);
+        if (step + 1 < 2 * T::TB) {
+            weights(step + 1, phi[x ^ 1], plo[x ^ 1]);
+#pragma unroll
+            for (uint32_t n = 0; n < 2 * T::NT; ++n) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                      // a product
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                      // an LDS read
+                __builtin_amdgcn_sched_group_barrier(0x402, T::NT == 4 ? 8 : 16, 0);  // vector and exp instructions
+            }
         }
     }
+    __builtin_amdgcn_s_setprio(0);
     st.l_part += psum;
 }
 
@@ -298,41 +410,51 @@ __device__ __forceinline__ void attn_tile_pass(const sglkv_attn_params &p, uint6
     };
     fill(0);
     __syncthreads();
+    // The queries' loads are complete here, so that the compiler puts no wait
+    // for them (which would be one for the rows in flight) into the loop.
+    __builtin_amdgcn_s_waitcnt(0x0F70);
     attn_tile_issue<D>(p, kbase, vbase, table, w, lane, lds_at);
     st.m_run = -3.402823466e+38f;
     st.l_part = 0.0f;
 #pragma unroll
     for (uint32_t n = 0; n < T::NT; ++n) st.o[n] = sglkv_f32x16{};
-    for (uint32_t k = 0; k < nb; ++k) {
-        // Block k's rows have landed (every wave waits for its own, then
-        // meets the others), and nobody reads block k-1's stage any more.
+    // Block k's rows have landed (every wave waits for its own, then meets
+    // the others), and nobody reads block k-1's stage any more: block k+1's
+    // rows go there.
+    auto next = [&](uint32_t k) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (k + 1 < nb) {
-            if ((k + 1) % TBLOCKS == 0) {
-                fill(k + 1);
-                __syncthreads();
-            }
-            attn_tile_issue<D>(p, kbase, vbase, table + ((k + 1) % TBLOCKS) * T::B, w, lane,
-                               lds_at + ((k + 1) & 1) * T::STAGE);
+        if (k + 1 >= nb) return;
+        if ((k + 1) % TBLOCKS == 0) {
+            fill(k + 1);
+            __syncthreads();
         }
+        attn_tile_issue<D>(p, kbase, vbase, table + ((k + 1) % TBLOCKS) * T::B, w, lane,
+                           lds_at + ((k + 1) & 1) * T::STAGE);
+    };
+    // The blocks that the wave's rows attend, then those it only loads for
+    // the others (a branch around the block instead would have the compiler
+    // copy the outputs every block).
+    const uint32_t mine = wave_max <= t0 ? 0 : (wave_max < t1 ? wave_max - t0 + T::B - 1 : nb * T::B) / T::B;
+    for (uint32_t k = 0; k < mine; ++k) {
+        next(k);
         const uint32_t tb = t0 + k * T::B;
-        if (tb < wave_max)
-            attn_tile_block<D>(p, attn_tile_lds + (k & 1) * T::STAGE, qf, static_cast<int32_t>(len - tb),
-                                        tb + T::B > wave_min, lane, st);
+        attn_tile_block<D>(p, attn_tile_lds + (k & 1) * T::STAGE, qf, static_cast<int32_t>(len - tb),
+                           tb + T::B > wave_min, lane, w % T::SHARE, st);
     }
+    for (uint32_t k = mine; k < nb; ++k) next(k);
 }
 
 // The row's output (one split), or its split record (rows of the combine
 // kernel's layout). Lanes l and l + 32 hold the row's dims 8i + 4h .. +3.
 // Plain stores: the two lanes' pieces of a line meet in L2.
 template <uint32_t D>
-__device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint64_t qrow, uint32_t split, uint32_t h,
+__device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint64_t qrow, uint32_t split, uint32_t part, uint32_t h,
                                                 const attn_tile_state<D> &st) {
     typedef attn_tl<D> T;
     const float l_tot = st.l_part + __shfl_xor(st.l_part, 32);
     if (p.splits == 1) {
         const float linv = 1.0f / l_tot;
-        uint16_t *out = p.output + qrow * D + 4 * h;
+        uint16_t *out = p.output + qrow * D + D / T::SHARE * part + 4 * h;
 #pragma unroll
         for (uint32_t n = 0; n < T::NT; ++n)
 #pragma unroll
@@ -345,12 +467,12 @@ __device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint
         return;
     }
     const uint64_t rec = qrow * p.splits + split;
-    if (h == 0) {
+    if (h == 0 && part == 0) {
         float *pr = attn_rec_ml(p, rec);
         pr[0] = st.m_run;
         pr[1] = l_tot;
     }
-    float *out = attn_rec_o(p, rec) + 4 * h;
+    float *out = attn_rec_o(p, rec) + D / T::SHARE * part + 4 * h;
 #pragma unroll
     for (uint32_t n = 0; n < T::NT; ++n)
 #pragma unroll
@@ -372,42 +494,34 @@ __device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
     const uint64_t vbase = pool + p.value_offset + kvh * p.value_head_stride;
     const uint32_t lds_at = attn_lat_lds_at(attn_tile_lds);
     // The lane's row of a tile.
-    const uint32_t row = 32 * w + (lane & 31), rq = row / p.group, rh = row - rq * p.group;
+    const uint32_t row = 32 * (w / T::SHARE) + (lane & 31), rq = row / p.group, rh = row - rq * p.group;
 
-    uint32_t q0, nq;
-    for (uint32_t tile = p.tile_slots - 1 - blockIdx.x / p.kv_heads; attn_tile_find(p, tile, lane, &q0, &nq);
-         tile += p.tile_slots) {
-        // Metadata of the tile's request (uniform), then of the lane's query.
-        const bool report = split == 0 && kvh == 0;
-        const uint32_t req = p.query_request_indices[q0];
-        if (req >= p.request_count) {
-            if (report && tid == 0) atomicOr(p.flag, SGLKV_FLAG_ATTN_REQUEST);
-            continue;
-        }
-        const uint64_t start = p.request_slot_offsets[req], end = p.request_slot_offsets[req + 1];
-        if (start > end || end > p.sequence_slot_count) {
-            if (report && tid == 0) atomicOr(p.flag, SGLKV_FLAG_ATTN_SEQUENCE);
-            continue;
-        }
+    uint32_t q0, nq, req;
+    for (uint32_t tile = p.tile_slots - 1 - blockIdx.x / p.kv_heads;
+         attn_tile_find(p, tile, w, lane, reinterpret_cast<uint64_t *>(table), &q0, &nq, &req); tile += p.tile_slots) {
+        // The tile's request (uniform) and the lane's query: everything that
+        // depends on the tile alone is loaded at once (from request 0 and
+        // the tile's first query where the lane or the request has none).
         const bool mine = rq < nq;
-        uint32_t len = 0;  // the row's tokens (0: no row, or a query that fails its checks)
-        if (mine) {
-            const uint64_t n = p.query_sequence_lengths[q0 + rq];
-            if (n == 0 || n > end - start || n > p.chunk_tokens * static_cast<uint64_t>(p.splits)) {
-                if (report) atomicOr(p.flag, SGLKV_FLAG_ATTN_SEQUENCE);
-            } else {
-                len = static_cast<uint32_t>(n);  // host: chunk_tokens * splits < 2^31
-            }
-        }
-        const uint32_t chunk = static_cast<uint32_t>(p.chunk_tokens), t0 = split * chunk;
+        const uint64_t qrow = (static_cast<uint64_t>(q0) + (mine ? rq : 0)) * p.query_heads + kvh * p.group + rh;
+        const uint32_t known = req < p.request_count ? req : 0;
+        const uint64_t start = p.request_slot_offsets[known], end = p.request_slot_offsets[known + 1];
+        const uint64_t n = p.query_sequence_lengths[q0 + (mine ? rq : 0)];
         // Queries (B operand of q.k): row l % 32, dims 16c + 8(l/32).
-        const uint64_t qrow = (static_cast<uint64_t>(q0) + rq) * p.query_heads + kvh * p.group + rh;
         sglkv_u16x8 qf[T::KC];
 #pragma unroll
-        for (uint32_t c = 0; c < T::KC; ++c) {
-            qf[c] = sglkv_u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (mine) qf[c] = *reinterpret_cast<const sglkv_u16x8 *>(p.queries + qrow * D + 16 * c + 8 * (lane >> 5));
-        }
+        for (uint32_t c = 0; c < T::KC; ++c)
+            qf[c] = *reinterpret_cast<const sglkv_u16x8 *>(p.queries + qrow * D + 16 * c + 8 * (lane >> 5));
+        // The reference's checks; one workgroup per tile reports.
+        const uint32_t quiet = split | kvh, chunk = static_cast<uint32_t>(p.chunk_tokens), t0 = split * chunk;
+        uint32_t bad = 0;
+        if (req >= p.request_count)
+            bad = SGLKV_FLAG_ATTN_REQUEST;
+        else if (start > end || end > p.sequence_slot_count || n == 0 || n > end - start || n > chunk * p.splits)
+            bad = SGLKV_FLAG_ATTN_SEQUENCE;  // (host: chunk * splits below 2^31)
+        if (mine && bad && quiet == 0) atomicOr(p.flag, bad);
+        // The row's tokens (0: no row, or a query that fails its checks).
+        const uint32_t len = mine && !bad ? static_cast<uint32_t>(n) : 0;
         // One round with every row; the tile is done unless its values are
         // not finite. A token that one row attends and another does not has
         // weight 0 in the other's product, and 0 times an infinite or NaN
@@ -459,7 +573,7 @@ __device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
                     continue;
                 }
             }
-            if (own > t0) attn_tile_write<D>(p, qrow, split, lane >> 5, st);
+            if (own > t0) attn_tile_write<D>(p, qrow, split, w % T::SHARE, lane >> 5, st);
             if (!apart) break;
         }
     }
@@ -472,7 +586,12 @@ sglkv_paged_attention_tile128(sglkv_attn_params p) {
     attn_tile_body<128>(p);
 }
 
-extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
+extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void
 sglkv_paged_attention_tile64(sglkv_attn_params p) {
     attn_tile_body<64>(p);
+}
+
+extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
+sglkv_paged_attention_tile256(sglkv_attn_params p) {
+    attn_tile_body<256>(p);
 }

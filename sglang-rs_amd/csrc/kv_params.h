@@ -266,15 +266,15 @@ typedef struct sglkv_request_params {
 /* The dims-128 staged body keeps K in registers: two stages of V rows only
  * (64 d bytes each) and the slot table. */
 #define SGLKV_ATTN_KREG_LDS_BYTES(d) (SGLKV_ATTN_STAGED_STAGES * 64u * (d) + 4u * SGLKV_ATTN_STAGED_SLOTS)
-/* The tile bodies (several queries per request; K and V head dims d = 64 or
- * 128): a workgroup of four waves owns a tile of up to
+/* The tile bodies (several queries per request; K and V head dims d = 64,
+ * 128 or 256): a workgroup of four waves owns a tile of up to
  * SGLKV_ATTN_TILE_ROWS (query, query head) rows of one request and KV head. Its
  * LDS: two stages of a block's K and V rows and a table of the slots of the
- * next SGLKV_ATTN_TILE_SLOTS tokens: 40 and 80 KiB. */
-#define SGLKV_ATTN_TILE_ROWS 128u
-#define SGLKV_ATTN_TILE_BLOCK 64u /* tokens per block */
+ * next SGLKV_ATTN_TILE_SLOTS tokens: 40, 80 and 80 KiB. */
+#define SGLKV_ATTN_TILE_ROWS(d) ((d) > 128u ? 64u : 128u)
+#define SGLKV_ATTN_TILE_BLOCK(d) ((d) > 128u ? 32u : 64u) /* tokens per block */
 #define SGLKV_ATTN_TILE_SLOTS(d) ((d) > 64u ? 4096u : 2048u)
-#define SGLKV_ATTN_TILE_LDS_BYTES(d) (8u * (d) * SGLKV_ATTN_TILE_BLOCK + 4u * SGLKV_ATTN_TILE_SLOTS(d))
+#define SGLKV_ATTN_TILE_LDS_BYTES(d) (8u * (d) * SGLKV_ATTN_TILE_BLOCK(d) + 4u * SGLKV_ATTN_TILE_SLOTS(d))
 #define SGLKV_ATTN_TILE_QUERIES_MAX (1u << 24) /* queries the tile search indexes */
 
 typedef struct sglkv_attn_params {

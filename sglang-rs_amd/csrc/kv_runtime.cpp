@@ -524,6 +524,8 @@ extern "C" int32_t sgl_rocm_kv_init(int32_t device, const char *code_object_path
     if (err == hipSuccess)
         err = hipModuleGetFunction(&ctx->attention[13], ctx->module, "sglkv_paged_attention_tile64");
     if (err == hipSuccess)
+        err = hipModuleGetFunction(&ctx->attention[14], ctx->module, "sglkv_paged_attention_tile256");
+    if (err == hipSuccess)
         err = hipDeviceGetAttribute(&ctx->max_lds_per_block, hipDeviceAttributeMaxSharedMemoryPerBlock, device);
     if (err == hipSuccess)
         err = hipModuleGetFunction(&ctx->attention_combine, ctx->module, "sglkv_paged_attention_combine");
