@@ -515,7 +515,54 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         chunk = table;
         splits = ceil_div(max_len, chunk);
     }
+    // Ragged batches (the average request below two thirds of the longest):
+    // the split above is sized for equal lengths, so most queries leave their
+    // last splits empty and the chip part idle. With enough work (96 tokens a
+    // resident slot: below that the search for the live splits costs what it
+    // gives) the launch numbers the splits that have tokens first (compact).
+    // Its chunk is the shortest whose live workgroups, at most total / chunk +
+    // queries of each query's, fit the resident slots in one round (seventeen
+    // twentieths of the staged bodies'): at least 64 tokens (128 for long
+    // sequences, whose merge grows) and at most the equal-length chunk for
+    // the latent body, between 192 and 512 for the staged ones, whose larger
+    // batches take several rounds anyway.
+    // Measured on MI355X, per layer, before -> after:
+    //  - latent, 32 queries of 1,000..8,192 tokens (1,024 -> 672 a split) 125
+    //    -> 102 us, 23 of 955..7,643 93 -> 78, 7 of 100..900 (256 -> 64) 43 ->
+    //    30, 30 of 80..300 46 -> 33;
+    //  - dims 128, 64 queries of 100..4,096 (1,024 -> 512) 132 -> 115, 40 of
+    //    300..4,096 111 -> 83, 8 of 500..4,000 29 -> 26; head-major 140 -> 116;
+    //  - dims 64, 64 of 100..4,096 73 -> 63; dims 256, 32 of 500..4,000 45 -> 40.
+    // Batches nearer one length keep the split above (33 queries of 500..1,300:
+    // 33 us either way, 34 with this one; 128 of 2,000..3,000: 239, 250).
+    const uint64_t mean = ceil_div(c.sequence_slot_count, c.request_count);
+    uint64_t total;  // tokens times the workgroups that share them
+    if (splits > 1 && (which == 6 || which == 7 || which == 8 || which == 10 || which == 11) &&
+        c.query_count <= SGLKV_ATTN_COMPACT_QUERIES && mean < max_len - max_len / 3 && !mul_ovf(mean, base, &total)) {
+        const bool worth = total / target >= 96;
+        const uint64_t room = which == 6 ? target : target / 20 * 17;
+        uint64_t balanced = room > base ? ceil_div(total, room - base) : chunk;
+        const uint64_t least = which == 6 ? (max_len > 4096 ? 128 : 64) : (chunk < 192 ? chunk : 192);
+        const uint64_t most = which == 6 ? chunk : 512;
+        balanced = balanced < least ? least : (balanced > most ? most : balanced);
+        balanced = ceil_div(balanced, block) * block;
+        // (Never more records than the fixed workspace holds.)
+        uint64_t bytes;
+        const bool fits = !workspace ||
+                          (!mul_ovf(c.query_count * c.query_head_count, ceil_div(max_len, balanced), &bytes) &&
+                           !mul_ovf(bytes, which == 6 ? 2ull * SGLKV_ATTN_HPAD(p.dv) + 16 : 4ull * (SGLKV_ATTN_OPAD(p.dv) + 2),
+                                    &bytes) &&
+                           bytes <= workspace_bytes);
+        if (balanced < chunk && fits && (worth || which == 6)) {
+            chunk = balanced;
+            splits = ceil_div(max_len, chunk);
+        }
+        if (worth && max_len <= (1u << 30) && base * splits <= UINT32_MAX)
+            p.compact = lay.head_layout == SGL_KV_HND || base == c.query_count ? SGLKV_ATTN_COMPACT_HEADS_FIRST
+                                                                               : SGLKV_ATTN_COMPACT_QUERY_FIRST;
+    }
     if (splits > 65535) {  // grid y limit
+        p.compact = 0;
         chunk = ceil_div(ceil_div(max_len, 65535), block) * block;
         splits = ceil_div(max_len, chunk);
     }

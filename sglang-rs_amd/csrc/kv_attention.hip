@@ -132,19 +132,96 @@ struct attn_work {
     uint32_t dblk;
 };
 
+// The workgroup's query, split and number among the `inners` workgroups (KV
+// heads, head groups, value blocks) of that split, in a launch of queries *
+// inners (x) by splits (y). False: it has none.
+//
+// Workgroups go round-robin over the 8 XCDs and start in order. In a plain
+// launch a grid row of a multiple of 8 gives one XCD all of a query's splits,
+// so in a ragged batch the XCDs with the longest queries finish last. Compact
+// launches (ragged batches of at most SGLKV_ATTN_COMPACT_QUERIES queries)
+// number the splits that have tokens, every query's first split first: the
+// empty workgroups of the grid come last, every XCD gets the same number of
+// live ones, and the host can size the chunk so that they fill the chip in one
+// round. Each wave finds its place from the query lengths alone; a length that
+// the metadata checks refuse counts as one within the launch's splits. Within
+// a split the queries vary first on token-major pages (neighbours then read
+// different rows; with one query's heads adjacent 64 queries took 119 us at
+// dims 128 and 69 at dims 64, where this takes 115 and 63), the inners first
+// on head-major ones (116 against 119 us).
+// Only the bodies with COMPACT take compact launches (the host's rule).
+template <bool COMPACT>
+__device__ __forceinline__ bool attn_find_place(const sglkv_attn_params &p, uint32_t lane, uint32_t inners,
+                                                uint32_t &q, uint32_t &split, uint32_t &inner) {
+    const uint32_t queries = gridDim.x / inners;
+    if (!COMPACT || !p.compact) {
+        q = blockIdx.x % queries;
+        inner = blockIdx.x / queries;
+        split = blockIdx.y;
+        return true;
+    }
+    uint32_t n = blockIdx.y * gridDim.x + blockIdx.x;
+    constexpr uint32_t U = SGLKV_ATTN_COMPACT_QUERIES / 64;
+    const uint32_t chunk = static_cast<uint32_t>(p.chunk_tokens), covered = chunk * p.splits;  // (host: below 2^31)
+    uint32_t own[U];  // splits of query 64 u + lane
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t i = 64 * u + lane;
+        const uint64_t len = p.query_sequence_lengths[i < queries ? i : queries - 1];
+        const uint32_t l = len < covered ? static_cast<uint32_t>(len) : covered;
+        own[u] = i < queries ? (l ? (l + chunk - 1) / chunk : 1) : 0;
+    }
+    // Past the splits whose live queries the workgroups before this one take.
+    uint64_t live[U];
+    uint32_t queries_here;
+    for (split = 0;; ++split) {
+        queries_here = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            live[u] = __ballot(own[u] > split);
+            queries_here += __popcll(live[u]);
+        }
+        if (n < queries_here * inners) break;
+        if (queries_here == 0) return false;
+        n -= queries_here * inners;
+    }
+    // The n-th live query of the split.
+    if (p.compact == SGLKV_ATTN_COMPACT_QUERY_FIRST) {
+        inner = n / queries_here;
+        n -= inner * queries_here;
+    } else {
+        const uint32_t k = n / inners;
+        inner = n - k * inners;
+        n = k;
+    }
+    q = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t here = __popcll(live[u]);
+        if (n < here) {
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(live[u] >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(live[u]), 0));
+            q = 64 * u + __builtin_ctzll(__ballot(below == n && ((live[u] >> lane) & 1)));
+            break;
+        }
+        n -= here;
+    }
+    return true;
+}
+
+template <bool COMPACT = false>
 __device__ __forceinline__ bool attn_decode(const sglkv_attn_params &p, uint32_t lane, attn_work *w) {
-    // The KV head varies slowest: workgroups are dispatched round-robin
-    // over the 8 XCDs, so (with query_count * head_groups * dv_blocks a
-    // multiple of 8) every KV head of a query runs on one XCD, and the
-    // slices of one token row meet in one L2 rather than eight.
-    uint64_t bx = blockIdx.x;
-    const uint32_t dblk = static_cast<uint32_t>(bx % p.dv_blocks);
-    bx /= p.dv_blocks;
-    const uint32_t hg = static_cast<uint32_t>(bx % p.head_groups);
-    bx /= p.head_groups;
-    const uint64_t q = bx % p.query_count;
-    const uint32_t kvh = static_cast<uint32_t>(bx / p.query_count);
-    const uint32_t split = blockIdx.y;
+    // The KV head varies slowest: with query_count * head_groups * dv_blocks
+    // a multiple of 8 every KV head of a (query, split) of a plain launch runs
+    // on one XCD, and the slices of one token row meet in one L2 rather than
+    // eight.
+    uint32_t qi, split, inner;
+    if (!attn_find_place<COMPACT>(p, lane, p.kv_heads * p.head_groups * p.dv_blocks, qi, split, inner)) return false;
+    const uint32_t dblk = inner % p.dv_blocks;
+    inner /= p.dv_blocks;
+    const uint32_t hg = inner % p.head_groups;
+    const uint32_t kvh = inner / p.head_groups;
+    const uint64_t q = qi;
 
     uint64_t start = 0, len = 0;
     const bool report = lane == 0 && split == 0 && hg == 0 && dblk == 0 && kvh == 0;
@@ -339,7 +416,7 @@ __device__ __forceinline__ void attn_body(const sglkv_attn_params &p) {
     const uint32_t lane = threadIdx.x;
     const uint32_t g = lane >> 4, r = lane & 15;
     attn_work w;
-    if (!attn_decode(p, lane, &w)) return;
+    if (!attn_decode<>(p, lane, &w)) return;
     const uint32_t qstride = p.dk_pad + 8;
     uint16_t *qs = attn_lds;
     uint16_t *vt = attn_lds + SGLKV_ATTN_HEADS * qstride;
@@ -559,7 +636,7 @@ __device__ __forceinline__ void attn_pipe_body(const sglkv_attn_params &p) {
     const uint32_t g = lane >> 4, r = lane & 15;
     const uint32_t tg = lane & 7, dg = lane >> 3;
     attn_work w;
-    if (!attn_decode(p, lane, &w)) return;
+    if (!attn_decode<>(p, lane, &w)) return;
     const uint32_t qstride = p.dk_pad + 8;
     uint16_t *qs = attn_lds;
     uint16_t *vt = attn_lds + SGLKV_ATTN_HEADS * qstride;
@@ -966,12 +1043,11 @@ __device__ __forceinline__ void attn_wide_body(const sglkv_attn_params &p) {
     // same rows run on one XCD when query_count * kv_heads is a multiple
     // of 8.
     const uint32_t hblocks = (p.head_groups + G::GROUPS - 1) / G::GROUPS;
-    uint64_t bx = blockIdx.x;
-    const uint64_t q = bx % p.query_count;
-    bx /= p.query_count;
-    const uint32_t kvh = static_cast<uint32_t>(bx % p.kv_heads);
-    const uint32_t hb = static_cast<uint32_t>(bx / p.kv_heads);
-    const uint32_t split = blockIdx.y;
+    uint32_t qi, split, inner;
+    if (!attn_find_place<false>(p, lane, p.kv_heads * hblocks, qi, split, inner)) return;
+    const uint64_t q = qi;
+    const uint32_t kvh = inner % p.kv_heads;
+    const uint32_t hb = inner / p.kv_heads;
     uint64_t start = 0, len = 0;
     if (!attn_metadata(p, q, tid == 0 && split == 0 && hb == 0 && kvh == 0, &start, &len)) return;
     const uint64_t t0 = static_cast<uint64_t>(split) * p.chunk_tokens;
@@ -1501,12 +1577,11 @@ __device__ __forceinline__ void attn_latent_body(const sglkv_attn_params &p) {
 
     // Workgroup -> (query, KV head, block of 128 query heads), split.
     const uint32_t hblocks = (p.group + SGLKV_ATTN_LATENT_HEADS - 1) / SGLKV_ATTN_LATENT_HEADS;
-    uint64_t bx = blockIdx.x;
-    const uint64_t q = bx % p.query_count;
-    bx /= p.query_count;
-    const uint32_t kvh = static_cast<uint32_t>(bx % p.kv_heads);
-    const uint32_t hb = static_cast<uint32_t>(bx / p.kv_heads);
-    const uint32_t split = blockIdx.y;
+    uint32_t qi, split, inner;
+    if (!attn_find_place<true>(p, lane, p.kv_heads * hblocks, qi, split, inner)) return;
+    const uint64_t q = qi;
+    const uint32_t kvh = inner % p.kv_heads;
+    const uint32_t hb = inner / p.kv_heads;
     uint64_t start = 0, len = 0;
     if (!attn_metadata(p, q, tid == 0 && split == 0 && hb == 0 && kvh == 0, &start, &len)) return;
     const uint64_t t0 = static_cast<uint64_t>(split) * p.chunk_tokens;
@@ -1914,7 +1989,7 @@ __device__ __forceinline__ void attn_staged_body(const sglkv_attn_params &p) {
     const uint32_t lane = threadIdx.x;
     const uint32_t g = lane >> 4, r = lane & 15;
     attn_work w;
-    if (!attn_decode(p, lane, &w)) return;
+    if (!attn_decode<true>(p, lane, &w)) return;
     const uint32_t nb = static_cast<uint32_t>((w.t1 - w.t0 + kLatB - 1) / kLatB);  // <= SLOTS / 32 (host bound)
 
     // Queries (B operand of q.k): head r, dims 32c + 8g.
@@ -2115,7 +2190,7 @@ __device__ __forceinline__ void attn_kreg_body(const sglkv_attn_params &p) {
     const uint32_t lane = threadIdx.x;
     const uint32_t g = lane >> 4, r = lane & 15;
     attn_work w;
-    if (!attn_decode(p, lane, &w)) return;
+    if (!attn_decode<true>(p, lane, &w)) return;
     const uint32_t nb = static_cast<uint32_t>((w.t1 - w.t0 + kLatB - 1) / kLatB);
 
     sglkv_u16x8 qf[S::KC];

@@ -215,6 +215,11 @@ typedef struct sglkv_request_params {
  * (rows padded to whole 128-byte lines, so that the writes fill every line
  * they touch) and its m, l at partial + records * SGLKV_ATTN_OPAD(dv) + 2 i. */
 #define SGLKV_ATTN_OPAD(dv) (((dv) + 31u) & ~31u)
+/* Compact launches: at most this many queries; within a split the KV heads
+ * vary first, or the queries do. */
+#define SGLKV_ATTN_COMPACT_QUERIES 256u
+#define SGLKV_ATTN_COMPACT_HEADS_FIRST 1u
+#define SGLKV_ATTN_COMPACT_QUERY_FIRST 2u
 /* The combine kernel: threads of a workgroup, threads of a set (one 4-dim
  * piece of a row each) and sets per (query, head). */
 #define SGLKV_ATTN_COMBINE_THREADS 128u
@@ -305,7 +310,7 @@ typedef struct sglkv_attn_params {
     uint32_t splits;
     uint32_t page_shift;                  /* log2(page_size) if a power of two, else 32 */
     float scale_log2;                     /* scale * log2(e) */
-    float reserved_f;
+    uint32_t compact;                     /* 0, or a ragged batch's launch: splits with tokens first */
     /* Pipelined body only (page size a power of two, strides < 2^32): */
     const uint8_t *zero_row;              /* SGLKV_ZERO_ROW_BYTES of zeros (context-owned) */
     uint32_t page_stride32;
