@@ -251,6 +251,52 @@ int32_t attn_ptr(const char *name, const sgl_kv_device_buffer &b, uint64_t offse
 
 uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
+// The tiles of a launch with several queries per request, and whether they
+// are the faster way.
+struct TileShape {
+    uint64_t queries, per_request, live, max_len, dims;
+
+    TileShape(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p, uint64_t longest)
+        : queries(p.group && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) ? SGLKV_ATTN_TILE_ROWS(p.dk) / p.group : 1),
+          // (the queries shared evenly among the requests)
+          per_request(ceil_div(ceil_div(c.query_count, c.request_count), queries)),
+          live(per_request * c.request_count * p.kv_heads), max_len(longest), dims(p.dk) {}
+
+    // Splits that fill `target` resident workgroups: of 256 tokens or more,
+    // or of 128 where a request is one tile (few queries, so the records that
+    // the splits leave are few).
+    uint64_t splits(uint64_t target) const {
+        const uint64_t want = live >= target ? 1 : target / live, least = per_request > 1 ? 256 : 128;
+        return want < max_len / least ? want : (max_len >= 2 * least ? max_len / least : 1);
+    }
+
+    // Whether the tiles are estimated to take less time than the staged
+    // bodies, whose work items are one query's. Times in units of 50 ns, from
+    // measurements on MI355X: the staged bodies take about 8 us, 6 more once
+    // they split (and merge), and 50 ns for each token that a resident
+    // workgroup's share comes to (100 past 128; half of that at dims 64, whose
+    // workgroups are twice as many); a tile takes about 11 us to its first
+    // block, 5 more if split, and per block 0.8, 1.5 or 1.0 us (dims 64, 128;
+    // 256, whose blocks are half as long) where other tiles of the request
+    // have brought the rows into L2, 2.2 us where it reads them first. Tiles
+    // and staged measured: 64 queries of one prompt (dims 128) 13.9 and 12.0
+    // us, 4 x 64 12.8 and 17.9, 160 15.2 and 19.1, 4 x 160 16 and 51; 4 x 2
+    // queries of up to 1,000 tokens 22 and 15, 20 x 5 30 and 57 (over 8 KV
+    // heads; over one 27 and 18).
+    bool pays(int cu_count, uint64_t items, uint64_t mean) const {
+        const uint64_t cus = cu_count > 0 ? (uint64_t)cu_count : 256, lds = 160u * 1024u;
+        const uint64_t staged_slots = cus * (lds / SGLKV_ATTN_STAGED_LDS_BYTES(dims));
+        uint64_t share;  // tokens per resident workgroup
+        if (mul_ovf(items, mean, &share)) return true;
+        share = share / staged_slots / (dims == 64 ? 2 : 1);
+        const uint64_t staged = 160 + (max_len > 64 ? 120 : 0) + share + (share > 128 ? share - 128 : 0);
+        const uint64_t cut = splits(cus * (lds / SGLKV_ATTN_TILE_LDS_BYTES(dims)));
+        const uint64_t blocks = ceil_div(ceil_div(max_len, cut), SGLKV_ATTN_TILE_BLOCK(dims));
+        const uint64_t block = per_request == 1 ? 44 : dims == 64 ? 16 : dims == 128 ? 30 : 20;
+        return 220 + blocks * block + (cut > 1 ? 100 : 0) < staged;
+    }
+};
+
 // Validates, sizes the split and launches the attention (and, with
 // several splits, the combine pass) on `stream`; nothing waits. Metadata
 // errors raise `flag_word`. `workspace` (fixed, `workspace_bytes` long)
@@ -421,20 +467,23 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     // Several queries per request on average (prefill, chunked prefill,
     // drafted tokens): the tile bodies, which read a K/V row once per tile of
     // queries instead of once per query. They take the staged bodies' shapes
-    // and any group of up to 64 query heads, 32 at dims 256 (a tile then holds at least two
-    // queries), count tokens in 32 bits and write 8-byte pieces.
-    const bool tile = fast && p.dk == p.dv && (p.dk == 64 || p.dk == 128 || p.dk == 256) && qp % 16 == 0 &&
-                      outp % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) / 2 &&
-                      p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
-                      lay.page_size <= (1u << 24) && c.query_count / 2 >= c.request_count &&
-                      c.query_count <= SGLKV_ATTN_TILE_QUERIES_MAX &&
-                      c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
-                      SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= (unsigned)ctx->max_lds_per_block;
+    // and any group of up to 64 query heads, 32 at dims 256 (a tile then holds
+    // at least two queries), count tokens in 32 bits and write 8-byte pieces.
+    const bool tileable = fast && p.dk == p.dv && (p.dk == 64 || p.dk == 128 || p.dk == 256) && qp % 16 == 0 &&
+                          outp % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) / 2 &&
+                          p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
+                          lay.page_size <= (1u << 24) && c.query_count / 2 >= c.request_count &&
+                          c.query_count <= SGLKV_ATTN_TILE_QUERIES_MAX &&
+                          c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
+                          SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= (unsigned)ctx->max_lds_per_block;
+    const TileShape shape(c, p, tileable ? max_len : 1);
+    const bool tile = tileable && (which < 7 || shape.pays(ctx->cu_count, c.query_count * p.kv_heads,
+                                                           ceil_div(c.sequence_slot_count, c.request_count)));
     if (tile) {
         which = p.dk == 128 ? 12 : p.dk == 64 ? 13 : 14;
         lds = SGLKV_ATTN_TILE_LDS_BYTES(p.dk);
         threads = 256;
-        p.tile_queries = SGLKV_ATTN_TILE_ROWS(p.dk) / p.group;
+        p.tile_queries = (uint32_t)shape.queries;
         p.tile_recip = UINT32_MAX / p.tile_queries + 1;
         // Queries that come request by request make at most this many tiles.
         const uint64_t most = c.query_count / p.tile_queries + c.request_count;
@@ -470,14 +519,7 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     }
     const uint64_t target =
         (uint64_t)ctx->attention_occupancy[fn] * (uint64_t)(ctx->cu_count > 0 ? ctx->cu_count : 256);
-    uint64_t live = base;
-    if (tile) {
-        // The tiles of requests that share the queries evenly (the grid
-        // leaves room for one more per request).
-        const uint64_t per_request = ceil_div(ceil_div(c.query_count, c.request_count), p.tile_queries);
-        if (per_request * c.request_count < p.tile_slots) live = per_request * c.request_count * p.kv_heads;
-    }
-    uint64_t want = live >= target ? 1 : target / live;
+    uint64_t want = tile ? shape.splits(target) : base >= target ? 1 : target / base;
     if (tile && workspace) {
         // Never more split records than the fixed workspace holds: fewer,
         // longer splits instead (the tile bodies take chunks of any length).
@@ -485,7 +527,6 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         const uint64_t room = workspace_bytes / record / (c.query_count * c.query_head_count);
         if (want > room) want = room ? room : 1;
     }
-    if (tile && want > max_len / 256) want = max_len >= 512 ? max_len / 256 : 1;  // splits of 256 tokens or more
     uint64_t chunk = ceil_div(max_len, want);
     // The shortest chunk a split takes. Small batches split further when
     // the combine merges many splits per memory round (both combines spread
