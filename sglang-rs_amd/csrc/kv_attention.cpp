@@ -558,9 +558,9 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     }
     // Ragged batches (the average request below two thirds of the longest):
     // the split above is sized for equal lengths, so most queries leave their
-    // last splits empty and the chip part idle. With enough work (96 tokens a
-    // resident slot: below that the search for the live splits costs what it
-    // gives) the launch numbers the splits that have tokens first (compact).
+    // last splits empty and the chip part idle. With enough work (128 tokens a
+    // resident slot, 96 of the shorter dims-64 ones: 24 queries of 62..999 at
+    // dims 128, 100 a slot, took 21.1 us so and 20.5 without) the launch numbers the splits that have tokens first (compact).
     // Its chunk is the shortest whose live workgroups, at most total / chunk +
     // queries of each query's, fit the resident slots in one round (seventeen
     // twentieths of the staged bodies'): at least 64 tokens (128 for long
@@ -580,7 +580,7 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     uint64_t total;  // tokens times the workgroups that share them
     if (splits > 1 && (which == 6 || which == 7 || which == 8 || which == 10 || which == 11) &&
         c.query_count <= SGLKV_ATTN_COMPACT_QUERIES && mean < max_len - max_len / 3 && !mul_ovf(mean, base, &total)) {
-        const bool worth = total / target >= 96;
+        const bool worth = total / target >= (which == 8 ? 96 : 128);
         const uint64_t room = which == 6 ? target : target / 20 * 17;
         uint64_t balanced = room > base ? ceil_div(total, room - base) : chunk;
         const uint64_t least = which == 6 ? (max_len > 4096 ? 128 : 64) : (chunk < 192 ? chunk : 192);
@@ -683,11 +683,13 @@ extern "C" int32_t sgl_rocm_kv_paged_attention(sgl_rocm_kv_ctx *ctx, const sgl_k
     if (rc) return rc;
     DeviceScope scope(ctx->device);
     if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
+    // The word is read and cleared on the stream, into a pinned host word (a
+    // blocking copy after the wait costs more than the launch).
+    uint32_t *out = ctx->host_attn(), *word = ctx->sync_attn_flag;
+    void *args[] = {&word, &word, &out};
+    SGLKV_CHECK_HIP(hipModuleLaunchKernel(ctx->take_flags, 1, 1, 1, 64, 1, 1, 0, s, args, nullptr));
     SGLKV_CHECK_HIP(hipStreamSynchronize(s));
-    uint32_t flag = 0;
-    SGLKV_CHECK_HIP(hipMemcpy(&flag, ctx->sync_attn_flag, sizeof flag, hipMemcpyDeviceToHost));
-    if (flag) SGLKV_CHECK_HIP(hipMemset(ctx->sync_attn_flag, 0, sizeof(uint32_t)));
-    return attention_flag_status(flag);
+    return attention_flag_status(__atomic_load_n(out, __ATOMIC_ACQUIRE) | __atomic_load_n(out + 1, __ATOMIC_ACQUIRE));
 }
 
 extern "C" int32_t sgl_rocm_kv_paged_attention_async(sgl_rocm_kv_ctx *ctx,

@@ -57,9 +57,11 @@ struct Launch {
 
 // Replaces the device error word a validated launch raises (default: the
 // context's copy word).
-inline void set_launch_flag(Launch &l, uint32_t *flag) {
+inline void set_launch_flag(Launch &l, uint32_t *flag, uint32_t *host_flag = nullptr) {
     l.params.flag = flag;
     l.realign.flag = flag;
+    l.params.host_flag = host_flag;
+    l.realign.host_flag = host_flag;
 }
 
 // Layer span of a multi-layer launch: `count` layers, each side's data
@@ -155,6 +157,15 @@ struct sgl_rocm_kv_ctx {
     uint32_t *attn_flag;            // asynchronous paged attention
     uint32_t *pair_flag;            // the synchronous pair scatter/gather drop-ins
     uint32_t *sync_attn_flag;       // the synchronous paged attention
+    // Pinned host words that the device writes (separate lines), so that a
+    // synchronous call reads its result after the stream's wait instead of
+    // through a blocking copy: a bad slot of the pair scatter/gather, and two
+    // words each that sglkv_take_flags hands check_errors and the synchronous
+    // attention.
+    uint32_t *host_words;
+    uint32_t *host_pair() const { return host_words; }
+    uint32_t *host_errors() const { return host_words + 16; }
+    uint32_t *host_attn() const { return host_words + 32; }
     const uint8_t *zero_row;        // SGLKV_ZERO_ROW_BYTES of zeros inside that block
     void *attention_partial;        // split records, grown on demand
     uint64_t attention_partial_bytes;

@@ -114,10 +114,14 @@ template <> struct sglkv_vec<1> { typedef uint8_t type; };
 // SGLKV_INVALID_OFFSET for both after flagging a slot outside the pool. The
 // host guarantees slot_count < 2^32, so the page split runs in 32 bits.
 __device__ __forceinline__ void sglkv_pool_row(const sglkv_side &s, uint32_t row, uint32_t *flag,
-                                               uint64_t *off0, uint64_t *off1) {
+                                               uint32_t *host_flag, uint64_t *off0, uint64_t *off1) {
     const uint64_t slot = s.slots[row];
     if (slot >= s.slot_count) {
         atomicOr(flag, SGLKV_FLAG_SLOT);
+        // (A plain store: the only bit that a copy raises, and an atomic on
+        // host memory would need the host link's support.)
+        if (host_flag)
+            __hip_atomic_store(host_flag, SGLKV_FLAG_SLOT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         *off0 = *off1 = SGLKV_INVALID_OFFSET;
         return;
     }
@@ -134,7 +138,7 @@ __device__ __forceinline__ void sglkv_pool_row(const sglkv_side &s, uint32_t row
 // every one of its rows exists and resolved to a valid slot.
 template <uint32_t SK, uint32_t DK>
 __device__ __forceinline__ bool sglkv_stage_tile(const sglkv_side &src, const sglkv_side &dst, uint32_t *flag,
-                                                 uint64_t row0, uint32_t tile, uint32_t rows, uint64_t *s_src0,
+                                                 uint32_t *host_flag, uint64_t row0, uint32_t tile, uint32_t rows, uint64_t *s_src0,
                                                  uint64_t *s_src1, uint64_t *s_dst0, uint64_t *s_dst1) {
     const uint32_t nthreads = blockDim.x * blockDim.y;
     const uint32_t tid = threadIdx.y * blockDim.x + threadIdx.x;
@@ -145,11 +149,11 @@ __device__ __forceinline__ bool sglkv_stage_tile(const sglkv_side &src, const sg
             const uint64_t r = row0 + i;
             if (r < rows) {
                 if (SK == SGLKV_SIDE_POOL) {
-                    sglkv_pool_row(src, static_cast<uint32_t>(r), flag, &s_src0[i], &s_src1[i]);
+                    sglkv_pool_row(src, static_cast<uint32_t>(r), flag, host_flag, &s_src0[i], &s_src1[i]);
                     bad |= s_src0[i] == SGLKV_INVALID_OFFSET;
                 }
                 if (DK == SGLKV_SIDE_POOL) {
-                    sglkv_pool_row(dst, static_cast<uint32_t>(r), flag, &s_dst0[i], &s_dst1[i]);
+                    sglkv_pool_row(dst, static_cast<uint32_t>(r), flag, host_flag, &s_dst0[i], &s_dst1[i]);
                     bad |= s_dst0[i] == SGLKV_INVALID_OFFSET;
                 }
             }
@@ -180,7 +184,7 @@ __device__ __forceinline__ void sglkv_copy_rows(const sglkv_copy_params &p) {
     // Clean tiles (all but the last tile, unless a slot is bad) copy without
     // per-row predicates, so the compiler can pipeline the stores behind the
     // loads instead of draining the memory counter at every branch.
-    const bool clean = sglkv_stage_tile<SK, DK>(p.src, p.dst, p.flag, row0, tile, p.rows, s_src[0], s_src[1],
+    const bool clean = sglkv_stage_tile<SK, DK>(p.src, p.dst, p.flag, p.host_flag, row0, tile, p.rows, s_src[0], s_src[1],
                                                 s_dst[0], s_dst[1]);
     sglkv_copy_scales(p.scale_src, p.scale_dst, p.scale_count);
     const uint32_t layer = blockIdx.y;
@@ -311,7 +315,7 @@ __device__ __forceinline__ void sglkv_realign_rows(const sglkv_realign_params &p
     uint8_t *data = reinterpret_cast<uint8_t *>(s_dst1 + tile) + 16;
 
     const uint64_t row0 = static_cast<uint64_t>(sglkv_tile_index<REMAP>()) * tile;
-    sglkv_stage_tile<SK, DK>(p.src, p.dst, p.flag, row0, tile, p.rows, s_src0, s_src1, s_dst0, s_dst1);
+    sglkv_stage_tile<SK, DK>(p.src, p.dst, p.flag, p.host_flag, row0, tile, p.rows, s_src0, s_src1, s_dst0, s_dst1);
     sglkv_copy_scales(p.scale_src, p.scale_dst, p.scale_count);
     const uint32_t layer = blockIdx.y;
 

@@ -83,6 +83,7 @@ typedef struct sglkv_copy_params {
     sglkv_side src;
     sglkv_side dst;
     uint32_t *flag;         /* device error word (OR of SGLKV_FLAG_*) */
+    uint32_t *host_flag;    /* or null: a bad slot sets this host word too */
     float *scale_src;       /* optional per-layer scales copied bit-exactly; layer y's */
     float *scale_dst;       /* scale_count floats follow layer y - 1's */
     uint32_t scale_count;   /* floats to copy per layer (0: none) */
@@ -112,6 +113,7 @@ typedef struct sglkv_realign_params {
     sglkv_side src;
     sglkv_side dst;
     uint32_t *flag;
+    uint32_t *host_flag;
     float *scale_src;
     float *scale_dst;
     uint32_t scale_count;
