@@ -254,17 +254,20 @@ uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 // The tiles of a launch with several queries per request, and whether they
 // are the faster way.
 struct TileShape {
-    uint64_t queries, per_request, live, max_len, dims;
+    uint64_t queries, per_request, live, max_len, dims, mean;
 
     TileShape(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p, uint64_t longest)
         : queries(p.group && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) ? SGLKV_ATTN_TILE_ROWS(p.dk) / p.group : 1),
           // (the queries shared evenly among the requests)
           per_request(ceil_div(ceil_div(c.query_count, c.request_count), queries)),
-          live(per_request * c.request_count * p.kv_heads), max_len(longest), dims(p.dk) {}
+          live(per_request * c.request_count * p.kv_heads), max_len(longest), dims(p.dk),
+          mean(ceil_div(c.sequence_slot_count, c.request_count)) {}
 
     // Splits that fill `target` resident workgroups: of 256 tokens or more,
     // or of 128 where a request is one tile (few queries, so the records that
-    // the splits leave are few).
+    // the splits leave are few). They are counted for the longest sequence
+    // also where most are shorter: with as many more as the average leaves
+    // room for, 24 requests of 200..3,000 tokens (dims 256) took 49 us, not 38.
     uint64_t splits(uint64_t target) const {
         const uint64_t want = live >= target ? 1 : target / live, least = per_request > 1 ? 256 : 128;
         return want < max_len / least ? want : (max_len >= 2 * least ? max_len / least : 1);
@@ -283,7 +286,7 @@ struct TileShape {
     // us, 4 x 64 12.8 and 17.9, 160 15.2 and 19.1, 4 x 160 16 and 51; 4 x 2
     // queries of up to 1,000 tokens 22 and 15, 20 x 5 30 and 57 (over 8 KV
     // heads; over one 27 and 18).
-    bool pays(int cu_count, uint64_t items, uint64_t mean) const {
+    bool pays(int cu_count, uint64_t items) const {
         const uint64_t cus = cu_count > 0 ? (uint64_t)cu_count : 256, lds = 160u * 1024u;
         const uint64_t staged_slots = cus * (lds / SGLKV_ATTN_STAGED_LDS_BYTES(dims));
         uint64_t share;  // tokens per resident workgroup
@@ -477,8 +480,7 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
                           c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
                           SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= (unsigned)ctx->max_lds_per_block;
     const TileShape shape(c, p, tileable ? max_len : 1);
-    const bool tile = tileable && (which < 7 || shape.pays(ctx->cu_count, c.query_count * p.kv_heads,
-                                                           ceil_div(c.sequence_slot_count, c.request_count)));
+    const bool tile = tileable && (which < 7 || shape.pays(ctx->cu_count, c.query_count * p.kv_heads));
     if (tile) {
         which = p.dk == 128 ? 12 : p.dk == 64 ? 13 : 14;
         lds = SGLKV_ATTN_TILE_LDS_BYTES(p.dk);
@@ -488,6 +490,9 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         // Queries that come request by request make at most this many tiles.
         const uint64_t most = c.query_count / p.tile_queries + c.request_count;
         p.tile_slots = (uint32_t)(most < c.query_count ? most : c.query_count);
+        // The last tiles first, except where each request is one tile.
+        p.tile_first = shape.per_request > 1 ? p.tile_slots - 1 : 0;
+        p.tile_step = shape.per_request > 1 ? ~0u : 1u;
     }
     p.zero_row = ctx->zero_row;
     p.page_stride32 = (uint32_t)lay.page_stride_bytes;

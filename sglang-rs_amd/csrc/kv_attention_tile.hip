@@ -57,7 +57,7 @@
 
 namespace {
 
-constexpr uint32_t kTileAhead = 4;  // products that the K reads run ahead
+constexpr uint32_t kTileRaw = 1;    // slots per thread that are loaded ahead of the row lengths
 
 template <uint32_t D>
 struct attn_tl {
@@ -74,6 +74,7 @@ struct attn_tl {
     static constexpr uint32_t SHARE = 4 * 32 / ROWS;      // waves that share 32 rows, each with D / SHARE outputs
     static constexpr uint32_t NT = D / SHARE / 32;        // 32-dim output tiles of a wave
     static constexpr uint32_t TB = B / 32;                // 32-token score tiles
+    static constexpr uint32_t AHEAD = 4;                  // products that the K reads run ahead
     static_assert(D == 64 || D == 128 || D == 256, "head dims");
     static_assert(2 * STAGE + 4 * TABLE == SGLKV_ATTN_TILE_LDS_BYTES(D), "the host sizes the same LDS");
     static_assert(LPW * TPL * 4 == B && TABLE % B == 0, "whole loads and blocks");
@@ -84,16 +85,30 @@ struct attn_tl {
     static __device__ __forceinline__ uint32_t vswz(uint32_t t) { return D >= 128 ? (t & 3) << 2 : (t & 2) << 1; }
 };
 
+// The kernel's parameters, read again by whoever asks: the address passes
+// through an empty asm, so what one part of the kernel needs (the search, a
+// tile's set-up, its loop, its stores) is not held in scalar registers by all
+// of them.
+__device__ __forceinline__ const sglkv_attn_params &attn_tile_params() {
+    typedef const __attribute__((address_space(4))) sglkv_attn_params kernarg;
+    kernarg *k = (kernarg *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    return *(const sglkv_attn_params *)k;
+}
+
 // Queries [q0, q0 + nq) of tile `want`, or false if there are fewer tiles
-// (uniform over the workgroup). `masks`: 512 bytes of LDS. 4,096 queries a
-// step: each wave ballots where runs start in 16 stretches of 64 queries (its
-// loads all in flight at once: stepping through 128 queries at a time by one
-// wave, each step a memory latency, took most of a short tile's time), then
-// lane l of every wave takes stretch l, counts the tiles that start in it and
-// sums over the lanes.
+// (uniform over the workgroup). `masks`: 256 bytes of LDS; `seen_requests`: 8
+// KiB, the step's request indices, from which the tile's own request and end
+// are read without another memory latency. 2,048 queries a step: each wave
+// ballots where runs start in 8 stretches of 64 queries (its loads all in
+// flight at once: stepping through 128 queries at a time by one wave, each
+// step a memory latency, took most of a short tile's time), then lane l of
+// every wave takes stretch l, counts the tiles that start in it and sums over
+// the lanes.
 __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint32_t want, uint32_t w, uint32_t lane,
-                                               uint64_t *masks, uint32_t *q0, uint32_t *nq, uint32_t *request) {
-    constexpr uint32_t U = 16, STEP = 4 * U * 64;
+                                               uint64_t *masks, uint32_t *seen_requests, uint32_t *q0, uint32_t *nq,
+                                               uint32_t *request) {
+    constexpr uint32_t U = 8, STEP = 4 * U * 64;
     const uint32_t count = static_cast<uint32_t>(p.query_count);  // host: at most SGLKV_ATTN_TILE_QUERIES_MAX
     const uint32_t *req = p.query_request_indices;
     // ceil(x / tile_queries) for x up to 2^24 (the host's reciprocal is exact there)
@@ -114,9 +129,9 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
         }
         return tiles;
     };
-    uint32_t seen = 0, run = 0, first = 0;
+    uint32_t seen = 0, run = 0, first = 0, base = 0;
     bool found = false;
-    for (uint32_t base = 0; base < count && !found; base += STEP) {
+    for (; base < count; base += STEP) {
         uint32_t cur[U], before[U];
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
@@ -125,16 +140,17 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
             cur[u] = req[i < count - 1 ? i : count - 1];
             before[u] = req[(at > 1 ? at : 1) - 1];
         }
-        __syncthreads();  // the table that the masks overlay is no longer read
+        __syncthreads();  // the table and stage that the masks and indices overlay are no longer read
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
             const uint64_t starts = __ballot(cur[u] != before[u]) | (base + w + u == 0 ? 1 : 0);
+            seen_requests[64 * (U * w + u) + lane] = cur[u];
             if (lane == 0) masks[U * w + u] = starts;
         }
         __syncthreads();
-        const uint64_t starts = masks[lane];
+        const uint64_t starts = lane < 4 * U ? masks[lane] : 0;
         const uint32_t from = base + 64 * lane;
-        const uint32_t n = from >= count ? 0 : (count - from < 64 ? count - from : 64);
+        const uint32_t n = lane >= 4 * U || from >= count ? 0 : (count - from < 64 ? count - from : 64);
         // Start of the last run at or before the stretch's end: a running
         // maximum over the lanes (and what came before).
         uint32_t last = starts ? from + 63 - static_cast<uint32_t>(__builtin_clzll(starts)) : run;
@@ -160,6 +176,7 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
                                   __shfl(static_cast<uint32_t>(starts), l);
             walk(base + 64 * l, __shfl(n, l), bits, __shfl(in, l), k, &first);
             found = true;
+            break;
         }
         seen += __shfl(sum, 63);
         run = __shfl(last, 63);
@@ -169,7 +186,14 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
     // The tile ends with its run or after tile_queries (at most 128): how
     // many of the queries from `first` on are of its request.
     const uint32_t i = first + lane, j = i + 64;
-    const uint32_t ri = req[i < count ? i : count - 1], rj = req[j < count ? j : count - 1];
+    uint32_t ri, rj;
+    if (first + 128 <= base + STEP) {
+        ri = seen_requests[i - base];
+        rj = seen_requests[j - base];
+    } else {
+        ri = req[i < count ? i : count - 1];
+        rj = req[j < count ? j : count - 1];
+    }
     const uint32_t own = __builtin_amdgcn_readfirstlane(ri);
     const uint64_t oi = ~__ballot(i < count && ri == own), oj = ~__ballot(j < count && rj == own);
     const uint32_t len = oi ? static_cast<uint32_t>(__builtin_ctzll(oi))
@@ -271,7 +295,7 @@ __device__ __forceinline__ void attn_tile_block(const sglkv_attn_params &p, cons
     sglkv_f32x16 s[T::TB];
 #pragma unroll
     for (uint32_t b = 0; b < T::TB; ++b) s[b] = sglkv_f32x16{};
-    // The K reads run kTileAhead products ahead (sched_barrier keeps the
+    // The K reads run AHEAD products ahead (sched_barrier keeps the
     // order: the scheduler would sink each read next to its product, which
     // then waits for the LDS).
     auto kread = [&](uint32_t i) {
@@ -282,15 +306,15 @@ __device__ __forceinline__ void attn_tile_block(const sglkv_attn_params &p, cons
     // normal one: otherwise the older of a SIMD's two waves, in its softmax,
     // takes every issue slot and the matrix cores of the other wait.
     __builtin_amdgcn_s_setprio(1);
-    sglkv_u16x8 kf[kTileAhead];
+    sglkv_u16x8 kf[T::AHEAD];
 #pragma unroll
-    for (uint32_t i = 0; i < kTileAhead; ++i) kf[i] = kread(i);
+    for (uint32_t i = 0; i < T::AHEAD; ++i) kf[i] = kread(i);
 #pragma unroll
     for (uint32_t i = 0; i < T::KC * T::TB; ++i) {
         __builtin_amdgcn_sched_barrier(0);
-        const sglkv_u16x8 a = kf[i % kTileAhead];
+        const sglkv_u16x8 a = kf[i % T::AHEAD];
         s[i % T::TB] = attn_mfma32(a, qf[i / T::TB], s[i % T::TB]);
-        if (i + kTileAhead < T::KC * T::TB) kf[i % kTileAhead] = kread(i + kTileAhead);
+        if (i + T::AHEAD < T::KC * T::TB) kf[i % T::AHEAD] = kread(i + T::AHEAD);
     }
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(0);
@@ -387,7 +411,39 @@ __device__ __forceinline__ void attn_tile_block(const sglkv_attn_params &p, cons
     st.l_part += psum;
 }
 
-// Tokens [t0, t1) of the tile's request for the wave's 32 rows.
+// The slot table from token `from` on, up to the end of the split's last
+// block, each slot checked once; the first kTileRaw per thread from raw, if
+// the caller has them.
+template <uint32_t D, uint32_t N = 0>
+__device__ __forceinline__ void attn_tile_slots(const sglkv_attn_params &p, uint64_t start, uint32_t t0, uint32_t t1,
+                                                uint32_t from, uint32_t tid, uint32_t *table, const uint64_t *raw) {
+    typedef attn_tl<D> T;
+    asm volatile("" : "+v"(tid));  // (its table addresses are not held across the loop)
+    const uint32_t left = t0 + (t1 - t0 + T::B - 1) / T::B * T::B - from, n = left < T::TABLE ? left : T::TABLE;
+#pragma unroll
+    for (uint32_t j = 0; j < N; ++j) {
+        const uint32_t i = tid + 256 * j;
+        if (i < n) table[i] = attn_wide_slot(p, raw[j], from + i, t1);
+    }
+    for (uint32_t i = tid + 256 * N; i < n; i += 256) {
+        const uint32_t tok = from + i;
+        table[i] = attn_wide_slot(p, tok < t1 ? p.sequence_slots[start + tok] : 0, tok, t1);
+    }
+}
+template <uint32_t D>
+__device__ __forceinline__ void attn_tile_fill(const sglkv_attn_params &p, uint64_t start, uint32_t t0, uint32_t t1,
+                                               uint32_t from, uint32_t tid, uint32_t *table) {
+    attn_tile_slots<D>(p, start, t0, t1, from, tid, table, nullptr);
+}
+template <uint32_t D>
+__device__ __forceinline__ void attn_tile_fill(const sglkv_attn_params &p, uint64_t start, uint32_t t0, uint32_t t1,
+                                               uint32_t from, uint32_t tid, uint32_t *table,
+                                               const uint64_t (&raw)[kTileRaw]) {
+    attn_tile_slots<D, kTileRaw>(p, start, t0, t1, from, tid, table, raw);
+}
+
+// Tokens [t0, t1) of the tile's request for the wave's 32 rows, the first
+// blocks' slots in the table.
 template <uint32_t D>
 __device__ __forceinline__ void attn_tile_pass(const sglkv_attn_params &p, uint64_t start, uint32_t t0, uint32_t t1,
                                                uint64_t kbase, uint64_t vbase, uint32_t w, uint32_t tid,
@@ -399,16 +455,6 @@ __device__ __forceinline__ void attn_tile_pass(const sglkv_attn_params &p, uint6
     uint32_t *table = reinterpret_cast<uint32_t *>(attn_tile_lds + 2 * T::STAGE);
     constexpr uint32_t TBLOCKS = T::TABLE / T::B;
     const uint32_t nb = (t1 - t0 + T::B - 1) / T::B;
-    // The slots of blocks [b, b + TBLOCKS), checked once.
-    auto fill = [&](uint32_t b) {
-        const uint32_t from = t0 + b * T::B;
-        const uint32_t left = (nb - b) * T::B, n = left < T::TABLE ? left : T::TABLE;
-        for (uint32_t i = tid; i < n; i += 256) {
-            const uint32_t tok = from + i;
-            table[i] = attn_wide_slot(p, tok < t1 ? p.sequence_slots[start + tok] : 0, tok, t1);
-        }
-    };
-    fill(0);
     __syncthreads();
     // The queries' loads are complete here, so that the compiler puts no wait
     // for them (which would be one for the rows in flight) into the loop.
@@ -425,7 +471,7 @@ __device__ __forceinline__ void attn_tile_pass(const sglkv_attn_params &p, uint6
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (k + 1 >= nb) return;
         if ((k + 1) % TBLOCKS == 0) {
-            fill(k + 1);
+            attn_tile_fill<D>(p, start, t0, t1, t0 + (k + 1) * T::B, tid, table);
             __syncthreads();
         }
         attn_tile_issue<D>(p, kbase, vbase, table + ((k + 1) % TBLOCKS) * T::B, w, lane,
@@ -444,13 +490,29 @@ __device__ __forceinline__ void attn_tile_pass(const sglkv_attn_params &p, uint6
     for (uint32_t k = mine; k < nb; ++k) next(k);
 }
 
+// The lane's row of a tile: query and head within the group. Worked out anew
+// (the lane passes through an empty asm) where it is needed, rather than held
+// across the loop.
+template <uint32_t D>
+__device__ __forceinline__ void attn_tile_row(const sglkv_attn_params &p, uint32_t w, uint32_t lane, uint32_t *query,
+                                              uint32_t *head) {
+    asm volatile("" : "+v"(lane));
+    const uint32_t row = 32 * (w / attn_tl<D>::SHARE) + (lane & 31);
+    *query = row / p.group;
+    *head = row - *query * p.group;
+}
+
 // The row's output (one split), or its split record (rows of the combine
 // kernel's layout). Lanes l and l + 32 hold the row's dims 8i + 4h .. +3.
 // Plain stores: the two lanes' pieces of a line meet in L2.
 template <uint32_t D>
-__device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint64_t qrow, uint32_t split, uint32_t part, uint32_t h,
-                                                const attn_tile_state<D> &st) {
+__device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint32_t q0, uint32_t kvh, uint32_t split, uint32_t w,
+                                                uint32_t lane, const attn_tile_state<D> &st) {
     typedef attn_tl<D> T;
+    uint32_t rq, rh;
+    attn_tile_row<D>(p, w, lane, &rq, &rh);
+    const uint64_t qrow = (static_cast<uint64_t>(q0) + rq) * p.query_heads + kvh * p.group + rh;
+    const uint32_t part = w % T::SHARE, h = lane >> 5;
     const float l_tot = st.l_part + __shfl_xor(st.l_part, 32);
     if (p.splits == 1) {
         const float linv = 1.0f / l_tot;
@@ -483,8 +545,9 @@ __device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint
 }
 
 template <uint32_t D>
-__device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
+__device__ __forceinline__ void attn_tile_body() {
     typedef attn_tl<D> T;
+    const sglkv_attn_params &p = attn_tile_params();
     extern __shared__ __attribute__((aligned(16))) uint8_t attn_tile_lds[];
     uint32_t *table = reinterpret_cast<uint32_t *>(attn_tile_lds + 2 * T::STAGE);
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -493,12 +556,26 @@ __device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
     const uint64_t kbase = pool + p.key_offset + kvh * p.key_head_stride;
     const uint64_t vbase = pool + p.value_offset + kvh * p.value_head_stride;
     const uint32_t lds_at = attn_lat_lds_at(attn_tile_lds);
-    // The lane's row of a tile.
-    const uint32_t row = 32 * (w / T::SHARE) + (lane & 31), rq = row / p.group, rh = row - rq * p.group;
-
+    // Plans of one request take their queries in tiles as they come (a query
+    // of any other index is refused row by row): no search. Otherwise the
+    // tiles of each request's run.
+    const uint32_t count = static_cast<uint32_t>(p.query_count);
+    auto find = [&](uint32_t tile, uint32_t *q0, uint32_t *nq, uint32_t *req) {
+        const sglkv_attn_params &p = attn_tile_params();
+        if (p.request_count > 1)
+            return attn_tile_find(p, tile, w, lane, reinterpret_cast<uint64_t *>(table),
+                                  reinterpret_cast<uint32_t *>(attn_tile_lds), q0, nq, req);
+        *q0 = tile * p.tile_queries;
+        *nq = *q0 < count && count - *q0 < p.tile_queries ? count - *q0 : p.tile_queries;
+        *req = 0;
+        return *q0 < count;
+    };
     uint32_t q0, nq, req;
-    for (uint32_t tile = p.tile_slots - 1 - blockIdx.x / p.kv_heads;
-         attn_tile_find(p, tile, w, lane, reinterpret_cast<uint64_t *>(table), &q0, &nq, &req); tile += p.tile_slots) {
+    for (uint32_t tile = p.tile_first + p.tile_step * (blockIdx.x / p.kv_heads); find(tile, &q0, &nq, &req);
+         tile += p.tile_slots) {
+        const sglkv_attn_params &p = attn_tile_params();
+        uint32_t rq, rh;
+        attn_tile_row<D>(p, w, lane, &rq, &rh);
         // The tile's request (uniform) and the lane's query: everything that
         // depends on the tile alone is loaded at once (from request 0 and
         // the tile's first query where the lane or the request has none).
@@ -507,6 +584,7 @@ __device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
         const uint32_t known = req < p.request_count ? req : 0;
         const uint64_t start = p.request_slot_offsets[known], end = p.request_slot_offsets[known + 1];
         const uint64_t n = p.query_sequence_lengths[q0 + (mine ? rq : 0)];
+        const uint32_t own_req = p.query_request_indices[q0 + (mine ? rq : 0)];
         // Queries (B operand of q.k): row l % 32, dims 16c + 8(l/32).
         sglkv_u16x8 qf[T::KC];
 #pragma unroll
@@ -515,13 +593,22 @@ __device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
         // The reference's checks; one workgroup per tile reports.
         const uint32_t quiet = split | kvh, chunk = static_cast<uint32_t>(p.chunk_tokens), t0 = split * chunk;
         uint32_t bad = 0;
-        if (req >= p.request_count)
+        if (own_req >= p.request_count)
             bad = SGLKV_FLAG_ATTN_REQUEST;
         else if (start > end || end > p.sequence_slot_count || n == 0 || n > end - start || n > chunk * p.splits)
             bad = SGLKV_FLAG_ATTN_SEQUENCE;  // (host: chunk * splits below 2^31)
         if (mine && bad && quiet == 0) atomicOr(p.flag, bad);
         // The row's tokens (0: no row, or a query that fails its checks).
         const uint32_t len = mine && !bad ? static_cast<uint32_t>(n) : 0;
+        // The split's first slots, ahead of the rows' lengths (which tokens
+        // are attended, and so checked, is decided at use).
+        uint64_t raw[kTileRaw];
+        const bool ranged = start < end && end <= p.sequence_slot_count;
+#pragma unroll
+        for (uint32_t j = 0; j < kTileRaw; ++j) {
+            const uint64_t tok = start + t0 + tid + 256 * j;
+            raw[j] = ranged ? p.sequence_slots[tok < end ? tok : end - 1] : 0;
+        }
         // One round with every row; the tile is done unless its values are
         // not finite. A token that one row attends and another does not has
         // weight 0 in the other's product, and 0 times an infinite or NaN
@@ -529,35 +616,38 @@ __device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
         // length. So when a wave whose rows end apart holds an output that is
         // not finite, the rows are done again, one length a round from the
         // longest down: no row then meets a token that it does not attend.
+        auto wave_reduce = [&](uint32_t v, bool most) {
+#pragma unroll
+            for (uint32_t d = 1; d < 32; d <<= 1) {
+                const uint32_t x = __shfl_xor(v, d);
+                v = (x > v) == most ? x : v;
+            }
+            return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v));
+        };
+        // The longest of the tile's rows that are shorter than `below`
+        // (through the slot table's first words).
+        auto tile_longest = [&](uint32_t below) {
+            const uint32_t most = wave_reduce(len < below ? len : 0, true);
+            __syncthreads();  // the table and stages are no longer read
+            if (lane == 0) table[w] = most;
+            __syncthreads();
+            uint32_t x = table[0];
+#pragma unroll
+            for (uint32_t i = 1; i < 4; ++i) x = table[i] > x ? table[i] : x;
+            __syncthreads();
+            return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(x));
+        };
+        uint32_t longest = tile_longest(0xFFFFFFFFu);
+        if (t0 >= longest) continue;
+        uint32_t t1 = longest - t0 < chunk ? longest : t0 + chunk;
+        attn_tile_fill<D>(p, start, t0, t1, t0, tid, table, raw);
         bool apart = false;
-        for (uint32_t below = 0xFFFFFFFFu;;) {
-            // The round's longest row over the tile (through the slot
-            // table's first words), and the wave's longest and shortest.
-            auto wave_reduce = [&](uint32_t v, bool most) {
-#pragma unroll
-                for (uint32_t d = 1; d < 32; d <<= 1) {
-                    const uint32_t x = __shfl_xor(v, d);
-                    v = (x > v) == most ? x : v;
-                }
-                return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v));
-            };
-            uint32_t wave_max = wave_reduce(len < below ? len : 0, true);
-            __syncthreads();  // the previous round's table and stages are no longer read
-            if (lane == 0) table[w] = wave_max;
-            __syncthreads();
-            uint32_t longest = table[0];
-#pragma unroll
-            for (uint32_t i = 1; i < 4; ++i) longest = table[i] > longest ? table[i] : longest;
-            longest = __builtin_amdgcn_readfirstlane(longest);
-            __syncthreads();
-            if (t0 >= longest) break;
-            below = longest;
+        for (;;) {
             const uint32_t own = apart && len != longest ? 0 : len;
-            if (apart) wave_max = wave_reduce(own, true);
+            const uint32_t wave_max = wave_reduce(own, true);
             const uint32_t wave_min = wave_reduce(own ? own : 0xFFFFFFFFu, false);
-            const uint32_t t1 = longest - t0 < chunk ? longest : t0 + chunk;
             attn_tile_state<D> st;
-            attn_tile_pass<D>(p, start, t0, t1, kbase, vbase, w, tid, lane, lds_at, own, wave_min, wave_max, qf, st);
+            attn_tile_pass<D>(attn_tile_params(), start, t0, t1, kbase, vbase, w, tid, lane, lds_at, own, wave_min, wave_max, qf, st);
             if (!apart) {
                 float odd = 0.0f;
 #pragma unroll
@@ -568,13 +658,18 @@ __device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
                 if (lane == 0) table[w] = redo ? 1u : 0u;  // (the table is not read past the last block's issue)
                 __syncthreads();
                 apart = __builtin_amdgcn_readfirstlane(table[0] | table[1] | table[2] | table[3]) != 0;
-                if (apart) {
-                    below = 0xFFFFFFFFu;
-                    continue;
+                if (!apart) {
+                    if (own > t0) attn_tile_write<D>(attn_tile_params(), q0, kvh, split, w, lane, st);
+                    break;
                 }
+                longest = 0xFFFFFFFFu;
+            } else if (own > t0) {
+                attn_tile_write<D>(attn_tile_params(), q0, kvh, split, w, lane, st);
             }
-            if (own > t0) attn_tile_write<D>(p, qrow, split, w % T::SHARE, lane >> 5, st);
-            if (!apart) break;
+            longest = tile_longest(longest);
+            if (t0 >= longest) break;
+            t1 = longest - t0 < chunk ? longest : t0 + chunk;
+            attn_tile_fill<D>(p, start, t0, t1, t0, tid, table);
         }
     }
 }
@@ -582,16 +677,16 @@ __device__ __forceinline__ void attn_tile_body(const sglkv_attn_params &p) {
 }  // namespace
 
 extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
-sglkv_paged_attention_tile128(sglkv_attn_params p) {
-    attn_tile_body<128>(p);
+sglkv_paged_attention_tile128(sglkv_attn_params) {
+    attn_tile_body<128>();
 }
 
 extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void
-sglkv_paged_attention_tile64(sglkv_attn_params p) {
-    attn_tile_body<64>(p);
+sglkv_paged_attention_tile64(sglkv_attn_params) {
+    attn_tile_body<64>();
 }
 
 extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
-sglkv_paged_attention_tile256(sglkv_attn_params p) {
-    attn_tile_body<256>(p);
+sglkv_paged_attention_tile256(sglkv_attn_params) {
+    attn_tile_body<256>();
 }
