@@ -490,9 +490,11 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         // Queries that come request by request make at most this many tiles.
         const uint64_t most = c.query_count / p.tile_queries + c.request_count;
         p.tile_slots = (uint32_t)(most < c.query_count ? most : c.query_count);
-        // The last tiles first, except where each request is one tile.
-        p.tile_first = shape.per_request > 1 ? p.tile_slots - 1 : 0;
-        p.tile_step = shape.per_request > 1 ? ~0u : 1u;
+        // Later tiles of a causal prompt attend more tokens: they start
+        // first, except where each request is one tile. (Several prompts'
+        // last tiles in turn were no faster: 4 of 2,048 tokens 266 us against
+        // 259, 4 of 300..2,048 189 against 143.)
+        p.tile_backward = shape.per_request > 1;
     }
     p.zero_row = ctx->zero_row;
     p.page_stride32 = (uint32_t)lay.page_stride_bytes;
@@ -524,6 +526,13 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     }
     const uint64_t target =
         (uint64_t)ctx->attention_occupancy[fn] * (uint64_t)(ctx->cu_count > 0 ? ctx->cu_count : 256);
+    // A launch of whole tiles that fits the chip in one round starts one
+    // workgroup on each CU and then a second: in that order the first CUs
+    // would get two long tiles, so the second ones come from the other end (a
+    // prompt of 1,500 tokens, dims 128, 55 -> 51 us, of 2,048 77 -> 74).
+    if (tile && p.tile_backward && base <= target && ctx->cu_count > 0 && base > (uint64_t)ctx->cu_count &&
+        shape.splits(target) == 1)
+        p.tile_fold = (uint32_t)ctx->cu_count / p.kv_heads;
     uint64_t want = tile ? shape.splits(target) : base >= target ? 1 : target / base;
     if (tile && workspace) {
         // Never more split records than the fixed workspace holds: fewer,

@@ -544,6 +544,13 @@ __device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint
         }
 }
 
+// The first tile of the x-th workgroup of a KV head and split (the host's
+// rule).
+__device__ __forceinline__ uint32_t attn_tile_order(const sglkv_attn_params &p, uint32_t x) {
+    if (p.tile_fold && x >= p.tile_fold) x = p.tile_slots - 1 - (x - p.tile_fold);
+    return p.tile_backward ? p.tile_slots - 1 - x : x;
+}
+
 template <uint32_t D>
 __device__ __forceinline__ void attn_tile_body() {
     typedef attn_tl<D> T;
@@ -571,7 +578,7 @@ __device__ __forceinline__ void attn_tile_body() {
         return *q0 < count;
     };
     uint32_t q0, nq, req;
-    for (uint32_t tile = p.tile_first + p.tile_step * (blockIdx.x / p.kv_heads); find(tile, &q0, &nq, &req);
+    for (uint32_t tile = attn_tile_order(p, blockIdx.x / p.kv_heads); find(tile, &q0, &nq, &req);
          tile += p.tile_slots) {
         const sglkv_attn_params &p = attn_tile_params();
         uint32_t rq, rh;

@@ -320,8 +320,9 @@ typedef struct sglkv_attn_params {
     /* Tile bodies only: */
     uint32_t tile_queries;                /* queries per tile (at most 128) */
     uint32_t tile_recip;                  /* ceil(2^32 / tile_queries) */
-    uint32_t tile_slots;                  /* workgroups per KV head and split; the x-th of them */
-    uint32_t tile_first, tile_step;       /* takes tile tile_first + tile_step * x first */
+    uint32_t tile_slots;                  /* workgroups per KV head and split */
+    uint32_t tile_backward;               /* they take the tiles from the last to the first */
+    uint32_t tile_fold;                   /* past this many, from the other end (0: never) */
     uint32_t reserved2;
 } sglkv_attn_params;
 
