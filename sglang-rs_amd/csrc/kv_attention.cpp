@@ -580,13 +580,16 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     // twentieths of the staged bodies'): at least 64 tokens (128 for long
     // sequences, whose merge grows) and at most the equal-length chunk for
     // the latent body, between 192 and 512 for the staged ones, whose larger
-    // batches take several rounds anyway.
+    // batches take several rounds anyway (past 32,768 tokens up to the
+    // equal-length chunk: 64 splits of the longest are enough, and more only
+    // add workgroups without tokens).
     // Measured on MI355X, per layer, before -> after:
     //  - latent, 32 queries of 1,000..8,192 tokens (1,024 -> 672 a split) 125
     //    -> 102 us, 23 of 955..7,643 93 -> 78, 7 of 100..900 (256 -> 64) 43 ->
     //    30, 30 of 80..300 46 -> 33;
     //  - dims 128, 64 queries of 100..4,096 (1,024 -> 512) 132 -> 115, 40 of
     //    300..4,096 111 -> 83, 8 of 500..4,000 29 -> 26; head-major 140 -> 116;
+    //    one of 131,072 among 63 of 1,000 1,683 -> 181, of 32,768 453 -> 96;
     //  - dims 64, 64 of 100..4,096 73 -> 63; dims 256, 32 of 500..4,000 45 -> 40.
     // Batches nearer one length keep the split above (33 queries of 500..1,300:
     // 33 us either way, 34 with this one; 128 of 2,000..3,000: 239, 250).
@@ -598,7 +601,7 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         const uint64_t room = which == 6 ? target : target / 20 * 17;
         uint64_t balanced = room > base ? ceil_div(total, room - base) : chunk;
         const uint64_t least = which == 6 ? (max_len > 4096 ? 128 : 64) : (chunk < 192 ? chunk : 192);
-        const uint64_t most = which == 6 ? chunk : 512;
+        const uint64_t most = which == 6 || max_len > 32768 ? chunk : 512;
         balanced = balanced < least ? least : (balanced > most ? most : balanced);
         balanced = ceil_div(balanced, block) * block;
         // (Never more records than the fixed workspace holds.)

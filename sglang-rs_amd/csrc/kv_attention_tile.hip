@@ -47,10 +47,10 @@
 //   causal prompts of 300..2,048 tokens (5,206 queries, 32 heads over 8, dims
 //   128): 1,744 -> 129 us (517 TFLOP/s of q.k and p.v; 688 where 2,048 queries
 //   each attend 6,144..8,192 tokens);
-//   384 queries over 6,144 tokens (14 heads over 2, dims 64): 112 -> 36 us;
+//   384 queries over 6,144 tokens (14 heads over 2, dims 64): 112 -> 33 us;
 //   5 queries of each of 24 requests of 200..3,000 tokens (8 heads over 2, dims
-//   256): 109 -> 45 us.
-// Of these, the search for the tile's queries in one step of 4,096 (not 128
+//   256): 109 -> 41 us.
+// Of these, the search for the tile's queries in steps of 2,048 (not 128
 // at a time) took the prompts from 185 to 135 us, and products at raised wave
 // priority with the next step's weights scheduled between them 388 -> 350 us on
 // the 8,192-token shape.

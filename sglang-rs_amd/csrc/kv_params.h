@@ -220,6 +220,7 @@ typedef struct sglkv_request_params {
 /* Compact launches: at most this many queries; within a split the KV heads
  * vary first, or the queries do. */
 #define SGLKV_ATTN_COMPACT_QUERIES 256u
+#define SGLKV_ATTN_COMPACT_NEAR 16u /* most splits that the search takes one by one */
 #define SGLKV_ATTN_COMPACT_HEADS_FIRST 1u
 #define SGLKV_ATTN_COMPACT_QUERY_FIRST 2u
 /* The combine kernel: threads of a workgroup, threads of a set (one 4-dim

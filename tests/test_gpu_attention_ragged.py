@@ -43,6 +43,8 @@ def _ragged(rng, queries, longest, mean):
     (21, 1, 128, 576, 512, False, 5000, 1500),
     (1, 1, 128, 576, 512, False, 700, 700),
     (9, 1, 100, 576, 512, False, 400, 90),     # short MLA batch: 64-token splits
+    (70, 8, 32, 128, 128, False, 40000, 300),  # one sequence of far more splits than the others
+    (64, 4, 8, 64, 64, True, 60000, 400),
 ])
 def test_ragged_decode(k, queries, H, qh, dk, dv, hnd, longest, mean):
     rng = np.random.default_rng(queries + dk)
