@@ -276,7 +276,8 @@ struct TileShape {
     // Whether the tiles are estimated to take less time than the staged
     // bodies, whose work items are one query's. Times in units of 50 ns, from
     // measurements on MI355X: the staged bodies take about 8 us, 6 more once
-    // they split (and merge), and 50 ns for each token that a resident
+    // they split (and merge: where twice the work items fit the resident slots,
+    // or a sequence is longer than a slot table), and 50 ns for each token that a resident
     // workgroup's share comes to (100 past 128; half of that at dims 64, whose
     // workgroups are twice as many); a tile takes about 11 us to its first
     // block, 5 more if split, and per block 0.8, 1.5 or 1.0 us (dims 64, 128;
@@ -292,7 +293,8 @@ struct TileShape {
         uint64_t share;  // tokens per resident workgroup
         if (mul_ovf(items, mean, &share)) return true;
         share = share / staged_slots / (dims == 64 ? 2 : 1);
-        const uint64_t staged = 160 + (max_len > 64 ? 120 : 0) + share + (share > 128 ? share - 128 : 0);
+        const bool cuts = (max_len > 64 && items <= staged_slots / 2) || max_len > SGLKV_ATTN_STAGED_SLOTS;
+        const uint64_t staged = 160 + (cuts ? 120 : 0) + share + (share > 128 ? share - 128 : 0);
         const uint64_t cut = splits(cus * (lds / SGLKV_ATTN_TILE_LDS_BYTES(dims)));
         const uint64_t blocks = ceil_div(ceil_div(max_len, cut), SGLKV_ATTN_TILE_BLOCK(dims));
         const uint64_t block = per_request == 1 ? 44 : dims == 64 ? 16 : dims == 128 ? 30 : 20;
@@ -592,6 +594,10 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     //    300..4,096 111 -> 83, 8 of 500..4,000 29 -> 26; head-major 140 -> 116;
     //    one of 131,072 among 63 of 1,000 1,683 -> 181, of 32,768 453 -> 96;
     //  - dims 64, 64 of 100..4,096 73 -> 63; dims 256, 32 of 500..4,000 45 -> 40.
+    // The latent body's live splits are always numbered first where they are
+    // sized to one round: one workgroup a CU, an uneven share of the XCDs is a
+    // second round (15 queries of 454..3,638 tokens 72 us a layer in grid
+    // order, 48 so; 9 of 739..5,919 69 and 47).
     // Batches nearer one length keep the split above (33 queries of 500..1,300:
     // 33 us either way, 34 with this one; 128 of 2,000..3,000: 239, 250).
     const uint64_t mean = ceil_div(c.sequence_slot_count, c.request_count);
@@ -616,7 +622,7 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
             chunk = balanced;
             splits = ceil_div(max_len, chunk);
         }
-        if (worth && max_len <= (1u << 30) && base * splits <= UINT32_MAX)
+        if ((worth || (which == 6 && chunk == balanced)) && max_len <= (1u << 30) && base * splits <= UINT32_MAX)
             p.compact = lay.head_layout == SGL_KV_HND || base == c.query_count ? SGLKV_ATTN_COMPACT_HEADS_FIRST
                                                                                : SGLKV_ATTN_COMPACT_QUERY_FIRST;
     }
