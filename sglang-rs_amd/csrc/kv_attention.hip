@@ -2400,10 +2400,9 @@ __device__ __forceinline__ void attn_combine_groups(const float2 *ml, const floa
 extern "C" __global__ __launch_bounds__(SGLKV_ATTN_COMBINE_THREADS) void sglkv_paged_attention_combine(
     sglkv_attn_params p) {
     __shared__ float part[SGLKV_ATTN_COMBINE_THREADS][6];  // m, l, o[4] of each thread
-    const uint32_t lanes = SGLKV_ATTN_COMBINE_LANES(p.dv), sets = SGLKV_ATTN_COMBINE_THREADS / lanes;
-    const uint32_t per = SGLKV_ATTN_COMBINE_PER(p.dv, p.splits), items = sets / per;
-    const uint32_t set = threadIdx.x / lanes, tl = threadIdx.x % lanes;
-    const uint32_t own = set / per, sub = set - own * per;
+    const sglkv_combine_place place = sglkv_combine_place_of(threadIdx.x, p.dv, p.splits);
+    const uint32_t lanes = place.lanes, per = place.per, items = place.items, own = place.own, sub = place.sub;
+    const uint32_t tl = threadIdx.x % lanes;
     // The set's (query, head) number `item` (below 2^31: the host's limit).
     auto merge = [&](uint32_t item, bool inside) {
         const uint32_t q = item / p.query_heads;
@@ -2430,7 +2429,7 @@ extern "C" __global__ __launch_bounds__(SGLKV_ATTN_COMBINE_THREADS) void sglkv_p
                     for (uint32_t e = 0; e < 4; ++e) pw[2 + e] = acc[e];
                 }
                 __syncthreads();
-                if (sub == 0) {
+                if (place.merges) {
                     for (uint32_t k = 1; k < per; ++k) {
                         const float *pk = pw + 6 * k * lanes;
                         const float m_new = fmaxf(m, pk[0]);
@@ -2442,7 +2441,7 @@ extern "C" __global__ __launch_bounds__(SGLKV_ATTN_COMBINE_THREADS) void sglkv_p
                     }
                 }
             }
-            if (!ok || sub != 0) continue;
+            if (!ok || !place.merges) continue;
             const float linv = 1.0f / l;
 #pragma unroll
             for (uint32_t e = 0; e < 4; ++e)

@@ -231,6 +231,30 @@ typedef struct sglkv_request_params {
 #define SGLKV_ATTN_COMBINE_SETS(dv) (SGLKV_ATTN_COMBINE_THREADS / SGLKV_ATTN_COMBINE_LANES(dv))
 #define SGLKV_ATTN_COMBINE_PER(dv, splits)                                                         \
     (((splits) + 7u) / 8u < SGLKV_ATTN_COMBINE_SETS(dv) ? ((splits) + 7u) / 8u : SGLKV_ATTN_COMBINE_SETS(dv))
+/* The place of a combine thread: its set's (query, head) among the
+ * workgroup's `items`, the set's number among that one's `per`, and whether it
+ * merges the other sets' shares, which thread t + k * lanes left in LDS for
+ * set k. The SETS % per sets (and the threads past the last whole set) that
+ * have no (query, head) merge nothing: shares past the workgroup's threads
+ * would be asked for. */
+typedef struct sglkv_combine_place {
+    uint32_t lanes, per, items, own, sub;
+    uint32_t merges;
+} sglkv_combine_place;
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+static inline sglkv_combine_place sglkv_combine_place_of(uint32_t thread, uint32_t dv, uint32_t splits) {
+    sglkv_combine_place c;
+    const uint32_t set = thread / SGLKV_ATTN_COMBINE_LANES(dv);
+    c.lanes = SGLKV_ATTN_COMBINE_LANES(dv);
+    c.per = SGLKV_ATTN_COMBINE_PER(dv, splits);
+    c.items = SGLKV_ATTN_COMBINE_SETS(dv) / c.per;
+    c.own = set / c.per;
+    c.sub = set - c.own * c.per;
+    c.merges = c.sub == 0 && c.own < c.items;
+    return c;
+}
 /* The latent body's split records are scaled fp16: record i keeps
  * y[dv] = o / a at partial + i * SGLKV_ATTN_HPAD(dv) halves (rows of whole
  * 128-byte lines), a = max |o| over the record (so |y| <= 1), and

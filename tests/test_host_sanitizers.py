@@ -3,7 +3,8 @@ UndefinedBehaviorSanitizer: tests/native/layout_fuzz.cpp replays reference
 goldens and fuzzes every group-1 entry point (small, boundary and
 overflowing values), the page allocator under random traffic and the
 checksum; tests/native/bootstrap_fuzz.cpp round-trips and mutates bootstrap
-frames through the wire-format decoder. Any out-of-bounds access, overflow
+frames through the wire-format decoder; tests/native/attention_rules.cpp
+walks the index rules that the attention kernels share with the host. Any out-of-bounds access, overflow
 UB or violated invariant fails the run. Host code only (g++, no device
 code)."""
 import os
@@ -47,3 +48,15 @@ def test_bootstrap_fuzz_under_asan_ubsan(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=240, env=env)
     assert r.returncode == 0, r.stderr[-4000:]
     assert "bootstrap fuzz ok" in r.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_attention_index_rules(tmp_path):
+    exe = tmp_path / "attention_rules"
+    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-Wextra", "-Werror", "-fsanitize=address,undefined",
+           "-fno-sanitize-recover=all", "-I" + CSRC,
+           os.path.join(ROOT, "tests", "native", "attention_rules.cpp"), "-o", str(exe)]
+    subprocess.run(cmd, check=True, capture_output=True, timeout=240)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0, r.stderr[-4000:]
+    assert "attention rules ok" in r.stdout
