@@ -309,8 +309,8 @@ __device__ __forceinline__ void attn_state_init(attn_state_n<NJ> &st) {
 // the validity ballots of the rows, and vt the block's values transposed
 // in LDS (vt[dim][position]). Updates the softmax state and o += p.v.
 // vt rows are VTS elements apart.
-template <bool FULL_DV = false, int NJ = SGLKV_ATTN_DV / 16, int VTS = SGLKV_ATTN_VT_STRIDE>
-__device__ __forceinline__ void attn_softmax_pv(const sglkv_attn_params &p, uint32_t g, uint32_t d0,
+template <int NJ = SGLKV_ATTN_DV / 16, int VTS = SGLKV_ATTN_VT_STRIDE>
+__device__ __forceinline__ void attn_softmax_pv(const sglkv_attn_params &p, uint32_t g,
                                                 const sglkv_f32x4 (&sc)[2], uint64_t vb0, uint64_t vb1,
                                                 const uint16_t *vt, uint32_t r, attn_state_n<NJ> &st) {
     float x[8];
@@ -350,9 +350,12 @@ __device__ __forceinline__ void attn_softmax_pv(const sglkv_attn_params &p, uint
 
     __builtin_amdgcn_wave_barrier();
     // o[head 4g+e][dim 16j + r] += sum_t p[head][t] * v[t][dim], p = hi + lo.
+    // Every block of dims, also those past dv (whose values are zeros): leaving
+    // the loop at dv put a branch between a block's products and the reads of
+    // their results, and the compiler counted the wait that these need wrongly
+    // where seven blocks are used (97 to 112 dims): dims 97.. came out wrong.
 #pragma unroll
     for (uint32_t j = 0; j < NJ; ++j) {
-        if (!FULL_DV && d0 + 16 * j >= p.dv) break;
         const sglkv_u16x8 vv = *reinterpret_cast<const sglkv_u16x8 *>(vt + (16 * j + r) * VTS + 8 * g);
         st.o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(attn_as_bf16(phi), attn_as_bf16(vv), st.o[j], 0, 0, 0);
         st.o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(attn_as_bf16(plo), attn_as_bf16(vv), st.o[j], 0, 0, 0);
@@ -526,7 +529,7 @@ __device__ __forceinline__ void attn_body(const sglkv_attn_params &p) {
                     vt[(8 * (g + 4 * s) + e) * SGLKV_ATTN_VT_STRIDE + tl] = vpiece[b][s][e];
         }
         const uint64_t vb0 = __ballot(valid[0]), vb1 = __ballot(valid[1]);
-        attn_softmax_pv(p, g, w.d0, sc, vb0, vb1, vt, r, st);
+        attn_softmax_pv(p, g, sc, vb0, vb1, vt, r, st);
     }
     attn_finish(p, w, g, r, st);
 }
@@ -650,7 +653,7 @@ __device__ __forceinline__ void attn_pipe_block(const sglkv_attn_params &p, uint
                                                             sc[b], 0, 0, 0);
     }
     const uint64_t vb0 = __ballot(rw.kvalid & 1), vb1 = __ballot((rw.kvalid >> 1) & 1);
-    attn_softmax_pv<FULL>(p, g, 0, sc, vb0, vb1, vt, r, st);
+    attn_softmax_pv(p, g, sc, vb0, vb1, vt, r, st);
 }
 
 #ifndef SGLKV_ATTN_PIPE_DEPTH

@@ -302,6 +302,22 @@ def test_shapes(k, H, qh, dk, dv, hnd):
     _check(got, want, c)
 
 
+@pytest.mark.parametrize("dk,dv,qh,H,hnd,max_len", [
+    (112, 112, 16, 4, False, 700), (104, 104, 8, 2, True, 90), (128, 98, 8, 2, False, 300),
+    (112, 112, 24, 1, False, 200), (240, 240, 8, 2, False, 300), (96, 120, 4, 2, False, 500),
+])
+def test_seven_blocks_of_value_dims(k, dk, dv, qh, H, hnd, max_len):
+    """Value dims that end in or beside the seventh 16-dim block of a
+    workgroup's 128, on the pipelined and the generic bodies."""
+    rng = np.random.default_rng(dk + dv + qh)
+    c = _Case(rng, P=16, L=2, H=H, dk=dk, dv=dv, qh=qh, pages=5 * max_len // 16 + 4, layer=1, hnd=hnd)
+    lens, rso, slots = _random_batch(rng, 5, max_len, c.layout.slot_count)
+    q = _bf16_normal(rng, 5 * qh * dk).reshape(5, qh, dk)
+    _say(f"value dims dk={dk} dv={dv} qh={qh} H={H} hnd={hnd} tokens={int(rso[-1])}")
+    got, want = c.run(k, q, np.arange(5), lens, rso, slots, 1.0 / math.sqrt(dk), max_len=max_len)
+    _check(got, want, c)
+
+
 @pytest.mark.parametrize("dk,dv,P,hnd", [(128, 128, 64, False), (128, 128, 64, True), (64, 64, 16, False),
                                          (256, 256, 64, False), (576, 512, 16, False)])
 def test_slots_outside_the_sequences_hold_nan(k, dk, dv, P, hnd):
