@@ -916,6 +916,40 @@ int32_t sgl_rocm_kv_paged_attention_async(sgl_rocm_kv_ctx *ctx, const sgl_kv_att
                                           const sgl_kv_attention_buffers *buffers,
                                           uint64_t max_sequence_length, void *stream);
 
+/* What sgl_rocm_kv_paged_attention_async launches for the same arguments, for
+ * profiles and tests; nothing is enqueued and nothing allocated. `body` is an
+ * SGL_KV_ATTN_BODY_*; a query's tokens are split into pieces of chunk_tokens,
+ * `splits` of them for one of max_sequence_length tokens; record_bytes is the
+ * size of the split records (0 with one split). */
+enum {
+    SGL_KV_ATTN_BODY_VECTOR = 0,       /* generic, 16-byte pieces */
+    SGL_KV_ATTN_BODY_ELEMENT = 1,      /* generic, element by element */
+    SGL_KV_ATTN_BODY_PIPE128 = 2,      /* pipelined: dims 128 */
+    SGL_KV_ATTN_BODY_PIPE = 3,         /* pipelined: dims up to 128 */
+    SGL_KV_ATTN_BODY_WIDE576 = 4,      /* many heads or wide values: K up to 576, V up to 512 */
+    SGL_KV_ATTN_BODY_WIDE128 = 5,      /* many heads: dims up to 128 */
+    SGL_KV_ATTN_BODY_LATENT = 6,       /* MLA: K 576, V 512, bf16 weights */
+    SGL_KV_ATTN_BODY_STAGED128 = 7,    /* rows staged in LDS: dims 128 */
+    SGL_KV_ATTN_BODY_STAGED64 = 8,
+    SGL_KV_ATTN_BODY_LATENT_EXACT = 9, /* MLA, hi + lo weights */
+    SGL_KV_ATTN_BODY_STAGED256 = 10,
+    SGL_KV_ATTN_BODY_STAGED128K = 11,  /* dims 128 on head-major pages: K in registers */
+    SGL_KV_ATTN_BODY_TILE128 = 12,     /* tiles of several queries of a request */
+    SGL_KV_ATTN_BODY_TILE64 = 13,
+    SGL_KV_ATTN_BODY_TILE256 = 14
+};
+typedef struct sgl_kv_attention_route {
+    uint32_t body;
+    uint32_t live_splits_first;  /* a ragged batch's splits are numbered, live ones first */
+    uint64_t splits;
+    uint64_t chunk_tokens;
+    uint64_t workgroups;
+    uint64_t record_bytes;
+} sgl_kv_attention_route;
+int32_t sgl_rocm_kv_attention_route(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *plan,
+                                    const sgl_kv_attention_buffers *buffers, uint64_t max_sequence_length,
+                                    sgl_kv_attention_route *out);
+
 /* No counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). sgl_rocm_kv_paged_attention_async with

@@ -320,6 +320,27 @@ class _AttentionBuffers(ctypes.Structure):
     _fields_ = [f for n in _ATTENTION_BUFFERS for f in ((n, _DeviceBuffer), (n + "_offset", _u64))]
 
 
+class _AttentionRoute(ctypes.Structure):
+    _fields_ = [("body", ctypes.c_uint32), ("live_splits_first", ctypes.c_uint32), ("splits", _u64),
+                ("chunk_tokens", _u64), ("workgroups", _u64), ("record_bytes", _u64)]
+
+
+# SGL_KV_ATTN_BODY_*, by value
+ATTENTION_BODIES = ("vector", "element", "pipe128", "pipe", "wide576", "wide128", "latent", "staged128", "staged64",
+                    "latent_exact", "staged256", "staged128k", "tile128", "tile64", "tile256")
+
+
+@dataclass(frozen=True)
+class AttentionRoute:
+    """sgl_kv_attention_route: what a paged-attention call launches."""
+    body: str
+    live_splits_first: bool
+    splits: int
+    chunk_tokens: int
+    workgroups: int
+    record_bytes: int
+
+
 PAGE_REQUEST_DTYPE = np.dtype([("source", "<u8"), ("target_offset", "<u8"), ("length", "<u8")])
 
 
@@ -506,6 +527,9 @@ _EXPORTS = {
                                                            ctypes.POINTER(_AttentionPlan),
                                                            ctypes.POINTER(_AttentionBuffers), _u64,
                                                            ctypes.c_void_p]),
+    "sgl_rocm_kv_attention_route": (ctypes.c_int32, [ctypes.c_void_p, ctypes.POINTER(_AttentionPlan),
+                                                     ctypes.POINTER(_AttentionBuffers), _u64,
+                                                     ctypes.POINTER(_AttentionRoute)]),
     "sgl_rocm_kv_paged_attention_async_noalloc": (ctypes.c_int32, [ctypes.c_void_p,
                                                                    ctypes.POINTER(_AttentionPlan),
                                                                    ctypes.POINTER(_AttentionBuffers), _u64,
@@ -1289,6 +1313,16 @@ class RocmKvPairCopyKernels:
         _paged_attention(lib().sgl_rocm_kv_paged_attention_async, self, plan, buffers,
                          max_sequence_length, stream)
 
+    def attention_route(self, plan: "PagedAttentionPlan", *, max_sequence_length: int = 0,
+                        **buffers) -> AttentionRoute:
+        """What paged_attention_async launches for these arguments (nothing
+        is enqueued). Buffers as for paged_attention."""
+        r = _AttentionRoute()
+        _call(lib().sgl_rocm_kv_attention_route, self._h, ctypes.byref(plan._c),
+              ctypes.byref(_attention_buffers(buffers)), max_sequence_length, ctypes.byref(r))
+        return AttentionRoute(ATTENTION_BODIES[r.body], bool(r.live_splits_first), r.splits, r.chunk_tokens,
+                              r.workgroups, r.record_bytes)
+
     def paged_attention_async_noalloc(self, plan: "PagedAttentionPlan", *, max_sequence_length: int = 0,
                                       stream=None, **buffers):
         """paged_attention_async with the split records in the library's
@@ -1863,14 +1897,18 @@ class PagedAttentionPlan:
                 lay.value_in_page_offset, lay.key_row_bytes, lay.value_row_bytes)
 
 
-def _paged_attention(fn, kernels, plan: PagedAttentionPlan, buffers: dict, max_sequence_length: int,
-                     stream):
+def _attention_buffers(buffers: dict) -> _AttentionBuffers:
     b = _AttentionBuffers()
     for n in _ATTENTION_BUFFERS:
         buf = buffers[n]
         setattr(b, n, _DeviceBuffer(buf.ptr, buf.nbytes) if hasattr(buf, "nbytes") else buf)
         setattr(b, n + "_offset", buffers.get(n + "_offset", 0))
-    _call(fn, kernels._h, ctypes.byref(plan._c), ctypes.byref(b), max_sequence_length,
+    return b
+
+
+def _paged_attention(fn, kernels, plan: PagedAttentionPlan, buffers: dict, max_sequence_length: int,
+                     stream):
+    _call(fn, kernels._h, ctypes.byref(plan._c), ctypes.byref(_attention_buffers(buffers)), max_sequence_length,
           _stream(stream))
 
 

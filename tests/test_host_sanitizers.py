@@ -4,7 +4,8 @@ goldens and fuzzes every group-1 entry point (small, boundary and
 overflowing values), the page allocator under random traffic and the
 checksum; tests/native/bootstrap_fuzz.cpp round-trips and mutates bootstrap
 frames through the wire-format decoder; tests/native/attention_rules.cpp
-walks the index rules that the attention kernels share with the host. Any out-of-bounds access, overflow
+walks the index rules that the attention kernels share with the host and
+tests/native/attention_route.cpp the choice of kernel and splits. Any out-of-bounds access, overflow
 UB or violated invariant fails the run. Host code only (g++, no device
 code)."""
 import os
@@ -60,3 +61,17 @@ def test_attention_index_rules(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=240)
     assert r.returncode == 0, r.stderr[-4000:]
     assert "attention rules ok" in r.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_attention_route(tmp_path):
+    exe = tmp_path / "attention_route"
+    cmd = ["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-fsanitize=address,undefined",
+           "-fno-sanitize-recover=all", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
+           os.path.join(ROOT, "tests", "native", "attention_route.cpp"),
+           os.path.join(CSRC, "kv_attention_route.cpp"), os.path.join(CSRC, "kv_layout.cpp"), "-o", str(exe)]
+    subprocess.run(cmd, check=True, capture_output=True, timeout=240)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0, r.stderr[-4000:]
+    assert "attention route ok" in r.stdout
