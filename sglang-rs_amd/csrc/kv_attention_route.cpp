@@ -18,6 +18,10 @@ int32_t sglkv::attention_overflow() {
 
 namespace {
 
+// (A plan edited after it was made may have no request: its queries are
+// refused one by one on the device.)
+uint64_t requests(const sgl_kv_attention_plan_config &c) { return c.request_count ? c.request_count : 1; }
+
 // The tiles of a launch with several queries per request, and whether they
 // are the faster way.
 struct TileShape {
@@ -26,9 +30,9 @@ struct TileShape {
     TileShape(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p, uint64_t longest)
         : queries(p.group && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) ? SGLKV_ATTN_TILE_ROWS(p.dk) / p.group : 1),
           // (the queries shared evenly among the requests)
-          per_request(ceil_div(ceil_div(c.query_count, c.request_count), queries)),
-          live(per_request * c.request_count * p.kv_heads), max_len(longest), dims(p.dk),
-          mean(ceil_div(c.sequence_slot_count, c.request_count)) {}
+          per_request(ceil_div(ceil_div(c.query_count, requests(c)), queries)),
+          live(per_request * requests(c) * p.kv_heads), max_len(longest), dims(p.dk),
+          mean(ceil_div(c.sequence_slot_count, requests(c))) {}
 
     // Splits that fill `target` resident workgroups: of 256 tokens or more,
     // or of 128 where a request is one tile (few queries, so the records that
@@ -153,7 +157,7 @@ int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_atten
     const bool tileable = fast && p.dk == p.dv && (p.dk == 64 || p.dk == 128 || p.dk == 256) && qp % 16 == 0 &&
                           outp % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) / 2 &&
                           p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
-                          lay.page_size <= (1u << 24) && c.query_count / 2 >= c.request_count &&
+                          lay.page_size <= (1u << 24) && c.request_count > 0 && c.query_count / 2 >= c.request_count &&
                           c.query_count <= SGLKV_ATTN_TILE_QUERIES_MAX &&
                           c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
                           SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= device.max_lds;
@@ -266,7 +270,7 @@ int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_atten
     // order, 48 so; 9 of 739..5,919 69 and 47).
     // Batches nearer one length keep the split above (33 queries of 500..1,300:
     // 33 us either way, 34 with this one; 128 of 2,000..3,000: 239, 250).
-    const uint64_t mean = ceil_div(c.sequence_slot_count, c.request_count);
+    const uint64_t mean = ceil_div(c.sequence_slot_count, requests(c));
     uint64_t total;  // tokens times the workgroups that share them
     if (splits > 1 && (which == 6 || which == 7 || which == 8 || which == 10 || which == 11) &&
         c.query_count <= SGLKV_ATTN_COMPACT_QUERIES && mean < max_len - max_len / 3 && !mul_ovf(mean, base, &total)) {

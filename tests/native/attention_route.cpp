@@ -154,9 +154,22 @@ void random_calls() {
     }
 }
 
+// A plan is a plain struct: one whose request_count was set to 0 after it was
+// made still launches, and its queries are refused on the device.
+void no_requests() {
+    for (const Shape &s : kShapes)
+        for (uint64_t queries : {1, 7, 500}) {
+            const Call x = {queries, 0, 1000, 1000, s.qheads, s.heads, s.dk, s.dv, false};
+            const Routed o = route(x);
+            check(x, o);
+            if (is_tile(o.r.body)) fail_call("a tile of no request", x, o);
+        }
+}
+
 }  // namespace
 
 int main() {
+    no_requests();
     random_calls();
     std::puts("attention route ok");
     return 0;
