@@ -18,9 +18,221 @@ int32_t sglkv::attention_overflow() {
 
 namespace {
 
+uint64_t whole_blocks(uint64_t tokens, uint64_t block) { return ceil_div(tokens, block) * block; }
+
+// Rows of K and V that 16-byte accesses read.
+bool rows16(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p) {
+    const sgl_kv_attention_layout &lay = c.layout;
+    const uint64_t poolp = reinterpret_cast<uint64_t>(p.pool);
+    return (p.dk % 8 == 0) && (p.dv % 8 == 0) && ((poolp + lay.key_in_page_offset) % 16 == 0) &&
+           ((poolp + lay.value_in_page_offset) % 16 == 0) &&
+           ((lay.page_stride_bytes | p.key_head_stride | p.key_token_stride | p.value_head_stride |
+             p.value_token_stride) % 16 == 0);
+}
+
+// 16-byte rows, power-of-two pages and strides that fit 32 bits admit the
+// pipelined, wide, staged and tile bodies (32-bit slots, shift-and-mask pages).
+bool fast_rows(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p) {
+    return rows16(c, p) && p.page_shift < 32 && c.slot_count < (1ull << 32) &&
+           c.layout.page_stride_bytes <= UINT32_MAX && p.key_token_stride <= UINT32_MAX &&
+           p.value_token_stride <= UINT32_MAX;
+}
+
+struct Body {
+    int which;
+    unsigned threads, lds;
+    // The latent body has two functions: hi + lo weights (the default, as
+    // precise as the other bodies) and, on request, bf16 weights.
+    int function(const sgl_kv_attention_plan_config &c) const {
+        return which == kAttnLatent && !(c.flags & SGL_KV_ATTN_FAST_WEIGHTS) ? kAttnLatentExact : which;
+    }
+};
+
 // (A plan edited after it was made may have no request: its queries are
 // refused one by one on the device.)
 uint64_t requests(const sgl_kv_attention_plan_config &c) { return c.request_count ? c.request_count : 1; }
+
+// The body that takes each query by itself.
+Body query_body(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p,
+                uint64_t max_len) {
+    const sgl_kv_attention_layout &lay = c.layout;
+    const uint64_t qp = reinterpret_cast<uint64_t>(p.queries);
+    const bool vec = rows16(c, p), fast = fast_rows(c, p);
+    const bool pipe = fast && p.dk_pad <= 128 && p.dv <= SGLKV_ATTN_DV;
+    int which = !vec ? 1 : !pipe ? 0 : (p.dk == 128 && p.dv == 128) ? 2 : 3;
+    // Many query heads per KV head (more than one 16-head group) or wide
+    // values: the wide bodies share each K/V block among 4 head groups
+    // instead of every group and value block reading it again. They hold
+    // the queries in registers as 16-byte vectors.
+    unsigned threads = 64;
+    unsigned lds = (unsigned)((SGLKV_ATTN_HEADS * (p.dk_pad + 8) + SGLKV_ATTN_DV * SGLKV_ATTN_VT_STRIDE) *
+                              sizeof(uint16_t));
+    // (Their chunks fit the slot table, so the grid's 65535 splits bound
+    // the length they take.)
+    if (fast && qp % 16 == 0 && (p.head_groups > 1 || p.dv > SGLKV_ATTN_DV) &&
+        max_len <= 65535ull * SGLKV_ATTN_WIDE_SLOTS) {
+        const unsigned narrow = SGLKV_ATTN_WIDE_LDS_BYTES(4u, 8u), wide = SGLKV_ATTN_WIDE_LDS_BYTES(18u, 32u);
+        if (p.dk_pad <= 128 && p.dv <= 128 && narrow <= device.max_lds) {
+            which = 5;
+            lds = narrow;
+            threads = 64 * SGLKV_ATTN_WIDE_WAVES;
+        } else if (p.dk > 512 && p.dk <= 576 && p.dv == 512 &&
+                   SGLKV_ATTN_LATENT_LDS_BYTES <= device.max_lds) {
+            // MLA's latent rows (K 576 = 512 + 64 rope dims, V 512): 32 heads
+            // per wave, rows loaded straight into LDS.
+            which = 6;
+            lds = SGLKV_ATTN_LATENT_LDS_BYTES;
+            threads = 64 * SGLKV_ATTN_LATENT_WAVES;
+        } else if (p.dk_pad <= 576 && p.dv <= 512 && wide <= device.max_lds) {
+            which = 4;
+            lds = wide;
+            threads = 64 * SGLKV_ATTN_WIDE_WAVES;
+        }
+    }
+    // Dims 128 or 64 with one head group per KV head (the Llama/Qwen GQA
+    // decodes): the staged bodies, rows loaded straight into LDS. They
+    // share one in-page offset between a token's K and V rows and form it
+    // with a 24-bit multiply.
+    // Dims 256 (Qwen3.5's full-attention layers) take the staged body too,
+    // one wave covering all 256 value dims.
+    const bool d64 = which == 3 && p.dk == 64 && p.dv == 64;
+    const bool d256 = fast && p.dk == 256 && p.dv == 256;
+    if ((which == 2 || d64 || d256) && qp % 16 == 0 && p.head_groups == 1 &&
+        p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
+        lay.page_size <= (1u << 24) &&
+        max_len <= 65535ull * SGLKV_ATTN_STAGED_SLOTS &&
+        SGLKV_ATTN_STAGED_LDS_BYTES(p.dk) <= device.max_lds) {
+        which = d64 ? 8 : d256 ? 10 : 7;
+        lds = SGLKV_ATTN_STAGED_LDS_BYTES(p.dk);
+        // Head-major pages at dims 128: K in registers, V alone in LDS.
+        // (Dims 64 keep K in LDS: the same body with K in registers,
+        // 125 VGPRs, measured no faster on head-major pages.)
+        if (which == 7 && lay.head_layout == SGL_KV_HND) {
+            which = 11;
+            lds = SGLKV_ATTN_KREG_LDS_BYTES(p.dk);
+        }
+        threads = 64;
+    }
+    return {which, threads, lds};
+}
+
+// A launch's workgroups of one split, how many stay resident at once, and the
+// equal splits of its longest sequence.
+struct Split {
+    uint64_t base, target, chunk, splits;
+};
+
+// Splits each query's sequence so that a per-query body's launch fills every
+// CU with as many workgroups as stay resident at once (the kernel's occupancy
+// at this LDS size), in one round.
+int32_t split_queries(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p,
+                      const Body &body, uint64_t max_len, Split *s) {
+    const int which = body.which;
+    const bool wide = which >= kAttnWide576 && which <= kAttnLatent;  // the wide and latent bodies (7, 8, 10, 11: staged)
+    const uint64_t hblocks = which == 6 ? ceil_div(p.group, SGLKV_ATTN_LATENT_HEADS)
+                                        : (p.head_groups + SGLKV_ATTN_WIDE_GROUPS - 1) / SGLKV_ATTN_WIDE_GROUPS;
+    uint64_t base = c.query_count;
+    if (mul_ovf(base, p.kv_heads, &base) || (wide && mul_ovf(base, hblocks, &base)) ||
+        (!wide && (mul_ovf(base, p.head_groups, &base) || mul_ovf(base, p.dv_blocks, &base))) ||
+        base > UINT32_MAX / body.threads)  // a dispatch counts its work-items in 32 bits
+        return too_large_dim("workgroups", base, UINT32_MAX / body.threads);
+    s->base = base;
+    s->target = device.resident(device.context, body.function(c), body.threads, body.lds) * device.cus;
+    if (!s->target) return SGL_KV_MODULE;
+    uint64_t chunk = ceil_div(max_len, base >= s->target ? 1 : s->target / base);
+    // The shortest chunk a split takes. Small batches split further when
+    // the combine merges many splits per memory round (both combines spread
+    // a query's split groups over several waves or thread sets), which puts
+    // more CUs to work. Measured:
+    //  - staged bodies (GQA dims 128 / 64, 32 heads over 8 KV heads, 4,096
+    //    tokens): 1 query 23.3 -> 15.5 us / 16.7 -> 11.8 us at 64 tokens
+    //    against 256, 2 queries 24.6 -> 17.8 / 17.5 -> 12.2, 4 queries 26.4
+    //    -> 23.3 / 18.8 -> 15.9; from 16 queries on the split count is set
+    //    by the occupancy target, not by this minimum. The dims-128 body
+    //    with K in registers (eight waves per CU) takes 128: at 64, 4
+    //    queries took 22.4 us against 20.6;
+    //  - latent body (MLA over 8,192 tokens): 64 tokens for one workgroup
+    //    before splitting, 128 for two or three (1 query 40.0 -> 33.2 us,
+    //    2 queries 41.0 -> 35.2 us), 256 from four on (best there);
+    //  - the other bodies keep 256 (not measured otherwise).
+    const uint64_t min_chunk = which == 11               ? 128
+                               : which >= 7              ? 64
+                               : which == 6 && base < 4  ? (base <= 1 ? 64 : 128)
+                                                         : 256;
+    chunk = whole_blocks(chunk < min_chunk ? min_chunk : chunk, SGLKV_ATTN_TOKENS);
+    const uint64_t table = wide ? SGLKV_ATTN_WIDE_SLOTS : which >= 7 ? SGLKV_ATTN_STAGED_SLOTS : 0;
+    if (table && chunk > table) chunk = table;  // the slot table of the wide, latent and staged bodies
+    s->chunk = chunk;
+    s->splits = ceil_div(max_len, chunk);
+    return SGL_KV_OK;
+}
+
+// Split records of a launch; false where their bytes pass 64 bits.
+bool record_bytes(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p, bool half_records, uint64_t splits,
+                  uint64_t *bytes) {
+    const uint64_t record = half_records ? 2ull * SGLKV_ATTN_HPAD(p.dv) + 16 : 4ull * (SGLKV_ATTN_OPAD(p.dv) + 2);
+    return !mul_ovf(c.query_count, c.query_head_count, bytes) && !mul_ovf(*bytes, splits, bytes) &&
+           !mul_ovf(*bytes, record, bytes);
+}
+
+// Ragged batches (the average request below two thirds of the longest):
+// the split above is sized for equal lengths, so most queries leave their
+// last splits empty and the chip part idle. With enough work (128 tokens a
+// resident slot, 96 of the shorter dims-64 ones: 24 queries of 62..999 at
+// dims 128, 100 a slot, took 21.1 us so and 20.5 without) the launch numbers the splits that have tokens first (compact).
+// Its chunk is the shortest whose live workgroups, at most total / chunk +
+// queries of each query's, fit the resident slots in one round (seventeen
+// twentieths of the staged bodies'): at least 64 tokens (128 for long
+// sequences, whose merge grows) and at most the equal-length chunk for
+// the latent body, between 192 and 512 for the staged ones, whose larger
+// batches take several rounds anyway (past 32,768 tokens up to the
+// equal-length chunk: 64 splits of the longest are enough, and more only
+// add workgroups without tokens: one of 131,072 tokens among 63 of 1,000
+// 248 us at 512 a split, 181 so; dims 64, one of 65,536, 81 and 67).
+// Measured on MI355X, per layer, before -> after:
+//  - latent, 32 queries of 1,000..8,192 tokens (1,024 -> 672 a split) 125
+//    -> 102 us, 23 of 955..7,643 93 -> 78, 7 of 100..900 (256 -> 64) 43 ->
+//    30, 30 of 80..300 46 -> 33;
+//  - dims 128, 64 queries of 100..4,096 (1,024 -> 512) 132 -> 115, 40 of
+//    300..4,096 111 -> 83, 8 of 500..4,000 29 -> 26; head-major 140 -> 116;
+//    one of 131,072 among 63 of 1,000 1,683 -> 181, of 32,768 453 -> 96;
+//  - dims 64, 64 of 100..4,096 73 -> 63; dims 256, 32 of 500..4,000 45 -> 40.
+// The latent body's live splits are always numbered first where they are
+// sized to one round: one workgroup a CU, an uneven share of the XCDs is a
+// second round (15 queries of 454..3,638 tokens 72 us a layer in grid
+// order, 48 so; 9 of 739..5,919 69 and 47).
+// Batches nearer one length keep the split above (33 queries of 500..1,300:
+// 33 us either way, 34 with this one; 128 of 2,000..3,000: 239, 250).
+void split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint64_t max_len, uint64_t workspace_bytes,
+                  sglkv_attn_params *params, Split *s) {
+    sglkv_attn_params &p = *params;
+    const int which = body.which;
+    if (s->splits < 2 || (which != kAttnLatent && which < kAttnStaged128) ||
+        c.query_count > SGLKV_ATTN_COMPACT_QUERIES)
+        return;
+    const uint64_t mean = ceil_div(c.sequence_slot_count, requests(c)), base = s->base, target = s->target;
+    uint64_t total;  // tokens times the workgroups that share them
+    if (mean >= max_len - max_len / 3 || mul_ovf(mean, base, &total)) return;
+    const bool worth = total / target >= (which == kAttnStaged64 ? 96 : 128);
+    const uint64_t room = which == kAttnLatent ? target : target / 20 * 17;
+    uint64_t balanced = room > base ? ceil_div(total, room - base) : s->chunk;
+    const uint64_t least = which == kAttnLatent ? (max_len > 4096 ? 128 : 64) : (s->chunk < 192 ? s->chunk : 192);
+    const uint64_t most = which == kAttnLatent || max_len > 32768 ? s->chunk : 512;
+    balanced = balanced < least ? least : (balanced > most ? most : balanced);
+    balanced = whole_blocks(balanced, SGLKV_ATTN_TOKENS);
+    // (Never more records than the fixed workspace holds.)
+    uint64_t bytes;
+    const bool fits = !workspace_bytes || (record_bytes(c, p, which == kAttnLatent, ceil_div(max_len, balanced), &bytes) &&
+                                           bytes <= workspace_bytes);
+    if (balanced < s->chunk && fits && (worth || which == kAttnLatent)) {
+        s->chunk = balanced;
+        s->splits = ceil_div(max_len, s->chunk);
+    }
+    if ((worth || (which == kAttnLatent && s->chunk == balanced)) && max_len <= (1u << 30) &&
+        base * s->splits <= UINT32_MAX)
+        p.compact = c.layout.head_layout == SGL_KV_HND || base == c.query_count ? SGLKV_ATTN_COMPACT_HEADS_FIRST
+                                                                                : SGLKV_ATTN_COMPACT_QUERY_FIRST;
+}
 
 // The tiles of a launch with several queries per request, and whether they
 // are the faster way.
@@ -73,258 +285,116 @@ struct TileShape {
     }
 };
 
-}  // namespace
-
-int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, uint64_t max_len,
-                               uint64_t workspace_bytes, sglkv_attn_params *params, AttentionRoute *route) {
-    sglkv_attn_params &p = *params;
-    const sgl_kv_attention_layout &lay = c.layout;
-    const uint64_t qp = reinterpret_cast<uint64_t>(p.queries), outp = reinterpret_cast<uint64_t>(p.output),
-                   poolp = reinterpret_cast<uint64_t>(p.pool);
-    const bool vec = (p.dk % 8 == 0) && (p.dv % 8 == 0) &&
-                     ((poolp + lay.key_in_page_offset) % 16 == 0) &&
-                     ((poolp + lay.value_in_page_offset) % 16 == 0) &&
-                     ((lay.page_stride_bytes | p.key_head_stride | p.key_token_stride | p.value_head_stride |
-                       p.value_token_stride) % 16 == 0);
-    // 16-byte rows, power-of-two pages and strides that fit 32 bits admit
-    // the pipelined and wide bodies (32-bit slots, shift-and-mask pages);
-    // head dims up to 128 take the software-pipelined body.
-    const bool fast = vec && p.page_shift < 32 && c.slot_count < (1ull << 32) &&
-                      lay.page_stride_bytes <= UINT32_MAX && p.key_token_stride <= UINT32_MAX &&
-                      p.value_token_stride <= UINT32_MAX;
-    const bool pipe = fast && p.dk_pad <= 128 && p.dv <= SGLKV_ATTN_DV;
-    int which = !vec ? 1 : !pipe ? 0 : (p.dk == 128 && p.dv == 128) ? 2 : 3;
-    // Many query heads per KV head (more than one 16-head group) or wide
-    // values: the wide bodies share each K/V block among 4 head groups
-    // instead of every group and value block reading it again. They hold
-    // the queries in registers as 16-byte vectors.
-    unsigned threads = 64;
-    unsigned lds = (unsigned)((SGLKV_ATTN_HEADS * (p.dk_pad + 8) + SGLKV_ATTN_DV * SGLKV_ATTN_VT_STRIDE) *
-                              sizeof(uint16_t));
-    if (!max_len || max_len > c.sequence_slot_count) max_len = c.sequence_slot_count;
-    // (Their chunks fit the slot table, so the grid's 65535 splits bound
-    // the length they take.)
-    if (fast && qp % 16 == 0 && (p.head_groups > 1 || p.dv > SGLKV_ATTN_DV) &&
-        max_len <= 65535ull * SGLKV_ATTN_WIDE_SLOTS) {
-        const unsigned narrow = SGLKV_ATTN_WIDE_LDS_BYTES(4u, 8u), wide = SGLKV_ATTN_WIDE_LDS_BYTES(18u, 32u);
-        if (p.dk_pad <= 128 && p.dv <= 128 && narrow <= device.max_lds) {
-            which = 5;
-            lds = narrow;
-            threads = 64 * SGLKV_ATTN_WIDE_WAVES;
-        } else if (p.dk > 512 && p.dk <= 576 && p.dv == 512 &&
-                   SGLKV_ATTN_LATENT_LDS_BYTES <= device.max_lds) {
-            // MLA's latent rows (K 576 = 512 + 64 rope dims, V 512): 32 heads
-            // per wave, rows loaded straight into LDS.
-            which = 6;
-            lds = SGLKV_ATTN_LATENT_LDS_BYTES;
-            threads = 64 * SGLKV_ATTN_LATENT_WAVES;
-        } else if (p.dk_pad <= 576 && p.dv <= 512 && wide <= device.max_lds) {
-            which = 4;
-            lds = wide;
-            threads = 64 * SGLKV_ATTN_WIDE_WAVES;
-        }
-    }
-    // Dims 128 or 64 with one head group per KV head (the Llama/Qwen GQA
-    // decodes): the staged bodies, rows loaded straight into LDS. They
-    // share one in-page offset between a token's K and V rows and form it
-    // with a 24-bit multiply.
-    // Dims 256 (Qwen3.5's full-attention layers) take the staged body too,
-    // one wave covering all 256 value dims.
-    const bool d64 = which == 3 && p.dk == 64 && p.dv == 64;
-    const bool d256 = fast && p.dk == 256 && p.dv == 256;
-    if ((which == 2 || d64 || d256) && qp % 16 == 0 && p.head_groups == 1 &&
-        p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
-        lay.page_size <= (1u << 24) &&
-        max_len <= 65535ull * SGLKV_ATTN_STAGED_SLOTS &&
-        SGLKV_ATTN_STAGED_LDS_BYTES(p.dk) <= device.max_lds) {
-        which = d64 ? 8 : d256 ? 10 : 7;
-        lds = SGLKV_ATTN_STAGED_LDS_BYTES(p.dk);
-        // Head-major pages at dims 128: K in registers, V alone in LDS.
-        // (Dims 64 keep K in LDS: the same body with K in registers,
-        // 125 VGPRs, measured no faster on head-major pages.)
-        if (which == 7 && lay.head_layout == SGL_KV_HND) {
-            which = 11;
-            lds = SGLKV_ATTN_KREG_LDS_BYTES(p.dk);
-        }
-        threads = 64;
-        p.dv_blocks = 1;
-    }
-    // Several queries per request on average (prefill, chunked prefill,
-    // drafted tokens): the tile bodies, which read a K/V row once per tile of
-    // queries instead of once per query. They take the staged bodies' shapes
-    // and any group of up to 64 query heads, 32 at dims 256 (a tile then holds
-    // at least two queries), count tokens in 32 bits and write 8-byte pieces.
-    const bool tileable = fast && p.dk == p.dv && (p.dk == 64 || p.dk == 128 || p.dk == 256) && qp % 16 == 0 &&
-                          outp % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) / 2 &&
+// Whether the tile bodies can take the call: several queries per request on
+// average (prefill, chunked prefill, drafted tokens). They read a K/V row once
+// per tile of queries instead of once per query, take the staged bodies' shapes
+// and any group of up to 64 query heads, 32 at dims 256 (a tile then holds
+// at least two queries), count tokens in 32 bits and write 8-byte pieces.
+bool tiles_take(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p,
+                uint64_t max_len) {
+    return fast_rows(c, p) && p.dk == p.dv && (p.dk == 64 || p.dk == 128 || p.dk == 256) && reinterpret_cast<uint64_t>(p.queries) % 16 == 0 &&
+                          reinterpret_cast<uint64_t>(p.output) % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) / 2 &&
                           p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
-                          lay.page_size <= (1u << 24) && c.request_count > 0 && c.query_count / 2 >= c.request_count &&
+                          c.layout.page_size <= (1u << 24) && c.request_count > 0 && c.query_count / 2 >= c.request_count &&
                           c.query_count <= SGLKV_ATTN_TILE_QUERIES_MAX &&
                           c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
                           SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= device.max_lds;
-    const TileShape shape(c, p, tileable ? max_len : 1);
-    const bool tile = tileable && (which < 7 || shape.pays(device.cus, c.query_count * p.kv_heads));
-    if (tile) {
-        which = p.dk == 128 ? 12 : p.dk == 64 ? 13 : 14;
-        lds = SGLKV_ATTN_TILE_LDS_BYTES(p.dk);
-        threads = 256;
-        p.tile_queries = (uint32_t)shape.queries;
-        p.tile_recip = UINT32_MAX / p.tile_queries + 1;
-        // Queries that come request by request make at most this many tiles.
-        const uint64_t most = c.query_count / p.tile_queries + c.request_count;
-        p.tile_slots = (uint32_t)(most < c.query_count ? most : c.query_count);
-        // Later tiles of a causal prompt attend more tokens: they start
-        // first, except where each request is one tile. (Several prompts'
-        // last tiles in turn were no faster: 4 of 2,048 tokens 266 us against
-        // 259, 4 of 300..2,048 189 against 143.)
-        p.tile_backward = shape.per_request > 1;
-    }
-    p.page_stride32 = (uint32_t)lay.page_stride_bytes;
-    p.key_token_stride32 = (uint32_t)p.key_token_stride;
-    p.value_token_stride32 = (uint32_t)p.value_token_stride;
+}
 
-    // Workgroups before splitting; split each query's sequence so that the
-    // launch fills every CU with as many workgroups as stay resident at
-    // once (the kernel's occupancy at this LDS size), in one round.
-    const bool wide = which >= kAttnWide576 && which <= kAttnLatent;  // the wide and latent bodies (7, 8, 10, 11: staged)
-    const uint64_t hblocks = which == 6 ? ceil_div(p.group, SGLKV_ATTN_LATENT_HEADS)
-                                        : (p.head_groups + SGLKV_ATTN_WIDE_GROUPS - 1) / SGLKV_ATTN_WIDE_GROUPS;
-    uint64_t base = tile ? p.tile_slots : c.query_count;
-    if (mul_ovf(base, p.kv_heads, &base) || (wide && mul_ovf(base, hblocks, &base)) ||
-        (!wide && !tile && (mul_ovf(base, p.head_groups, &base) || mul_ovf(base, p.dv_blocks, &base))) ||
-        base > UINT32_MAX / threads)  // a dispatch counts its work-items in 32 bits
-        return too_large_dim("workgroups", base, UINT32_MAX / threads);
-    // The latent body has two functions: hi + lo weights (the default, as
-    // precise as the other bodies) and, on request, bf16 weights.
-    const int fn = which == 6 && !(c.flags & SGL_KV_ATTN_FAST_WEIGHTS) ? 9 : which;
-    const uint64_t target = device.resident(device.context, fn, threads, lds) * device.cus;
+// Splits for a launch of tiles.
+int32_t split_tiles(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, const TileShape &shape,
+                    const Body &body, uint64_t max_len, uint64_t workspace_bytes, sglkv_attn_params *params, Split *s) {
+    sglkv_attn_params &p = *params;
+    p.tile_queries = (uint32_t)shape.queries;
+    p.tile_recip = UINT32_MAX / p.tile_queries + 1;
+    // Queries that come request by request make at most this many tiles.
+    const uint64_t most = c.query_count / p.tile_queries + c.request_count;
+    p.tile_slots = (uint32_t)(most < c.query_count ? most : c.query_count);
+    // Later tiles of a causal prompt attend more tokens: they start
+    // first, except where each request is one tile. (Several prompts'
+    // last tiles in turn were no faster: 4 of 2,048 tokens 266 us against
+    // 259, 4 of 300..2,048 189 against 143.)
+    p.tile_backward = shape.per_request > 1;
+    const uint64_t base = s->base = (uint64_t)p.tile_slots * p.kv_heads;
+    if (base > UINT32_MAX / body.threads)  // a dispatch counts its work-items in 32 bits
+        return too_large_dim("workgroups", base, UINT32_MAX / body.threads);
+    const uint64_t target = s->target =
+        device.resident(device.context, body.which, body.threads, body.lds) * device.cus;
     if (!target) return SGL_KV_MODULE;
     // A launch of whole tiles that fits the chip in one round starts one
     // workgroup on each CU and then a second: in that order the first CUs
     // would get two long tiles, so the second ones come from the other end (a
     // prompt of 1,500 tokens, dims 128, 55 -> 51 us, of 2,048 77 -> 74).
-    if (tile && p.tile_backward && base <= target && base > device.cus &&
-        shape.splits(target) == 1)
+    if (p.tile_backward && base <= target && base > device.cus && shape.splits(target) == 1)
         p.tile_fold = (uint32_t)device.cus / p.kv_heads;
-    uint64_t want = tile ? shape.splits(target) : base >= target ? 1 : target / base;
-    if (tile && workspace_bytes) {
+    uint64_t want = shape.splits(target);
+    if (workspace_bytes) {
         // Never more split records than the fixed workspace holds: fewer,
         // longer splits instead (the tile bodies take chunks of any length).
         const uint64_t record = 4ull * (SGLKV_ATTN_OPAD(p.dv) + 2);
         const uint64_t room = workspace_bytes / record / (c.query_count * c.query_head_count);
         if (want > room) want = room ? room : 1;
     }
-    uint64_t chunk = ceil_div(max_len, want);
-    // The shortest chunk a split takes. Small batches split further when
-    // the combine merges many splits per memory round (both combines spread
-    // a query's split groups over several waves or thread sets), which puts
-    // more CUs to work. Measured:
-    //  - staged bodies (GQA dims 128 / 64, 32 heads over 8 KV heads, 4,096
-    //    tokens): 1 query 23.3 -> 15.5 us / 16.7 -> 11.8 us at 64 tokens
-    //    against 256, 2 queries 24.6 -> 17.8 / 17.5 -> 12.2, 4 queries 26.4
-    //    -> 23.3 / 18.8 -> 15.9; from 16 queries on the split count is set
-    //    by the occupancy target, not by this minimum. The dims-128 body
-    //    with K in registers (eight waves per CU) takes 128: at 64, 4
-    //    queries took 22.4 us against 20.6;
-    //  - latent body (MLA over 8,192 tokens): 64 tokens for one workgroup
-    //    before splitting, 128 for two or three (1 query 40.0 -> 33.2 us,
-    //    2 queries 41.0 -> 35.2 us), 256 from four on (best there);
-    //  - the other bodies keep 256 (not measured otherwise).
-    const uint64_t min_chunk = tile                        ? 0
-                               : which == 11               ? 128
-                               : which >= 7                ? 64
-                               : which == 6 && base < 4    ? (base <= 1 ? 64 : 128)
-                                                           : 256;
-    const uint64_t block = tile ? SGLKV_ATTN_TILE_BLOCK(p.dk) : SGLKV_ATTN_TOKENS;  // splits are whole blocks
-    chunk = ceil_div(chunk < min_chunk ? min_chunk : chunk, block) * block;
-    uint64_t splits = ceil_div(max_len, chunk);
-    const uint64_t table = tile ? 0 : wide ? SGLKV_ATTN_WIDE_SLOTS : which >= 7 ? SGLKV_ATTN_STAGED_SLOTS : 0;
-    if (table && chunk > table) {  // the slot table of the wide, latent and staged bodies
-        chunk = table;
-        splits = ceil_div(max_len, chunk);
+    s->chunk = whole_blocks(ceil_div(max_len, want), SGLKV_ATTN_TILE_BLOCK(p.dk));
+    s->splits = ceil_div(max_len, s->chunk);
+    return SGL_KV_OK;
+}
+
+}  // namespace
+
+int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, uint64_t max_len,
+                               uint64_t workspace_bytes, sglkv_attn_params *params, AttentionRoute *route) {
+    sglkv_attn_params &p = *params;
+    if (!max_len || max_len > c.sequence_slot_count) max_len = c.sequence_slot_count;
+    p.page_stride32 = (uint32_t)c.layout.page_stride_bytes;
+    p.key_token_stride32 = (uint32_t)p.key_token_stride;
+    p.value_token_stride32 = (uint32_t)p.value_token_stride;
+    Body body = query_body(device, c, p, max_len);
+    if (body.which >= kAttnStaged128) p.dv_blocks = 1;
+    Split s = {0, 0, 0, 0};
+    uint64_t block = SGLKV_ATTN_TOKENS;
+    const TileShape shape(c, p, max_len);
+    if (tiles_take(device, c, p, max_len) &&
+        (body.which < kAttnStaged128 || shape.pays(device.cus, c.query_count * p.kv_heads))) {
+        body = {p.dk == 128 ? kAttnTile128 : p.dk == 64 ? kAttnTile64 : kAttnTile256, 256,
+                SGLKV_ATTN_TILE_LDS_BYTES(p.dk)};
+        block = SGLKV_ATTN_TILE_BLOCK(p.dk);
+        const int32_t rc = split_tiles(device, c, shape, body, max_len, workspace_bytes, &p, &s);
+        if (rc) return rc;
+    } else {
+        const int32_t rc = split_queries(device, c, p, body, max_len, &s);
+        if (rc) return rc;
+        split_ragged(c, body, max_len, workspace_bytes, &p, &s);
     }
-    // Ragged batches (the average request below two thirds of the longest):
-    // the split above is sized for equal lengths, so most queries leave their
-    // last splits empty and the chip part idle. With enough work (128 tokens a
-    // resident slot, 96 of the shorter dims-64 ones: 24 queries of 62..999 at
-    // dims 128, 100 a slot, took 21.1 us so and 20.5 without) the launch numbers the splits that have tokens first (compact).
-    // Its chunk is the shortest whose live workgroups, at most total / chunk +
-    // queries of each query's, fit the resident slots in one round (seventeen
-    // twentieths of the staged bodies'): at least 64 tokens (128 for long
-    // sequences, whose merge grows) and at most the equal-length chunk for
-    // the latent body, between 192 and 512 for the staged ones, whose larger
-    // batches take several rounds anyway (past 32,768 tokens up to the
-    // equal-length chunk: 64 splits of the longest are enough, and more only
-    // add workgroups without tokens: one of 131,072 tokens among 63 of 1,000
-    // 248 us at 512 a split, 181 so; dims 64, one of 65,536, 81 and 67).
-    // Measured on MI355X, per layer, before -> after:
-    //  - latent, 32 queries of 1,000..8,192 tokens (1,024 -> 672 a split) 125
-    //    -> 102 us, 23 of 955..7,643 93 -> 78, 7 of 100..900 (256 -> 64) 43 ->
-    //    30, 30 of 80..300 46 -> 33;
-    //  - dims 128, 64 queries of 100..4,096 (1,024 -> 512) 132 -> 115, 40 of
-    //    300..4,096 111 -> 83, 8 of 500..4,000 29 -> 26; head-major 140 -> 116;
-    //    one of 131,072 among 63 of 1,000 1,683 -> 181, of 32,768 453 -> 96;
-    //  - dims 64, 64 of 100..4,096 73 -> 63; dims 256, 32 of 500..4,000 45 -> 40.
-    // The latent body's live splits are always numbered first where they are
-    // sized to one round: one workgroup a CU, an uneven share of the XCDs is a
-    // second round (15 queries of 454..3,638 tokens 72 us a layer in grid
-    // order, 48 so; 9 of 739..5,919 69 and 47).
-    // Batches nearer one length keep the split above (33 queries of 500..1,300:
-    // 33 us either way, 34 with this one; 128 of 2,000..3,000: 239, 250).
-    const uint64_t mean = ceil_div(c.sequence_slot_count, requests(c));
-    uint64_t total;  // tokens times the workgroups that share them
-    if (splits > 1 && (which == 6 || which == 7 || which == 8 || which == 10 || which == 11) &&
-        c.query_count <= SGLKV_ATTN_COMPACT_QUERIES && mean < max_len - max_len / 3 && !mul_ovf(mean, base, &total)) {
-        const bool worth = total / target >= (which == 8 ? 96 : 128);
-        const uint64_t room = which == 6 ? target : target / 20 * 17;
-        uint64_t balanced = room > base ? ceil_div(total, room - base) : chunk;
-        const uint64_t least = which == 6 ? (max_len > 4096 ? 128 : 64) : (chunk < 192 ? chunk : 192);
-        const uint64_t most = which == 6 || max_len > 32768 ? chunk : 512;
-        balanced = balanced < least ? least : (balanced > most ? most : balanced);
-        balanced = ceil_div(balanced, block) * block;
-        // (Never more records than the fixed workspace holds.)
-        uint64_t bytes;
-        const bool fits = !workspace_bytes ||
-                          (!mul_ovf(c.query_count * c.query_head_count, ceil_div(max_len, balanced), &bytes) &&
-                           !mul_ovf(bytes, which == 6 ? 2ull * SGLKV_ATTN_HPAD(p.dv) + 16 : 4ull * (SGLKV_ATTN_OPAD(p.dv) + 2),
-                                    &bytes) &&
-                           bytes <= workspace_bytes);
-        if (balanced < chunk && fits && (worth || which == 6)) {
-            chunk = balanced;
-            splits = ceil_div(max_len, chunk);
-        }
-        if ((worth || (which == 6 && chunk == balanced)) && max_len <= (1u << 30) && base * splits <= UINT32_MAX)
-            p.compact = lay.head_layout == SGL_KV_HND || base == c.query_count ? SGLKV_ATTN_COMPACT_HEADS_FIRST
-                                                                               : SGLKV_ATTN_COMPACT_QUERY_FIRST;
-    }
-    if (splits > 65535) {  // grid y limit
+    if (s.splits > 65535) {  // grid y limit
         p.compact = 0;
-        chunk = ceil_div(ceil_div(max_len, 65535), block) * block;
-        splits = ceil_div(max_len, chunk);
+        s.chunk = whole_blocks(ceil_div(max_len, 65535), block);
+        s.splits = ceil_div(max_len, s.chunk);
     }
-    p.chunk_tokens = chunk;
+    const uint64_t splits = s.splits;
+    p.chunk_tokens = s.chunk;
     p.splits = (uint32_t)splits;
 
     // The latent body writes scaled fp16 records (SGLKV_ATTN_HPAD), the
     // others fp32 ones (SGLKV_ATTN_OPAD).
-    const bool half_records = which == 6;
+    const bool half_records = body.which == kAttnLatent;
     // The fp16 records and their combine are laid out for the latent body's
     // 512-wide values (SGLKV_ATTN_HPAD); nothing else selects that body.
     if (half_records && p.dv != 512)
         return fail(SGL_KV_INVALID_ARGUMENT, "value_head_dim", p.dv, 512, 0,
                     "the latent body's fp16 split records need 512-wide values, not %u", (unsigned)p.dv);
-    route->body = fn;
-    route->threads = threads;
-    route->lds = lds;
-    route->grid = base;
+    route->body = body.function(c);
+    route->threads = body.threads;
+    route->lds = body.lds;
+    route->grid = s.base;
     route->half_records = half_records;
     route->record_bytes = 0;
     route->combine_grid = 0;
     route->combine_threads = 0;
     if (splits == 1) return SGL_KV_OK;
-    const uint64_t per_record = half_records ? 2ull * SGLKV_ATTN_HPAD(p.dv) + 16 : 4ull * (SGLKV_ATTN_OPAD(p.dv) + 2);
     uint64_t heads;
-    if (mul_ovf(c.query_count, c.query_head_count, &heads) || mul_ovf(heads, splits, &route->record_bytes) ||
-        mul_ovf(route->record_bytes, per_record, &route->record_bytes))
+    if (mul_ovf(c.query_count, c.query_head_count, &heads) ||
+        !record_bytes(c, p, half_records, splits, &route->record_bytes))
         return attention_overflow();
     // The combine pass: the workgroup's sets of threads, SGLKV_ATTN_COMBINE_PER
     // to a (query, head); the fp16 one in blocks of 64 per 8 groups of 8 heads
