@@ -909,7 +909,11 @@ int32_t sgl_rocm_kv_paged_attention(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention
  * SGL_KV_ATTN_DEVICE_METADATA_INVALID). The error word is not cleared
  * first, so an earlier unchecked error stays visible. The split workspace
  * is shared by all calls on the context: issue calls that split on one
- * stream (growing it waits for the whole device). No counterpart in the
+ * stream (growing it waits for the whole device). Calls with several queries
+ * per request whose queries alone would not be split keep their records apart,
+ * in a buffer of 64 MiB made at the first of them, and are ordered on the
+ * device among themselves, whatever their streams; under graph capture, or
+ * where there is no memory for that buffer, they are not split. No counterpart in the
  * reference, whose forward always synchronises (cuda_attention.rs:821-829);
  * it is for decode loops that check errors once per step. */
 int32_t sgl_rocm_kv_paged_attention_async(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *plan,
@@ -945,6 +949,7 @@ typedef struct sgl_kv_attention_route {
     uint64_t chunk_tokens;
     uint64_t workgroups;
     uint64_t record_bytes;
+    uint64_t records_apart;      /* 1: they go to the tile bodies' own buffer (see below) */
 } sgl_kv_attention_route;
 int32_t sgl_rocm_kv_attention_route(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *plan,
                                     const sgl_kv_attention_buffers *buffers, uint64_t max_sequence_length,

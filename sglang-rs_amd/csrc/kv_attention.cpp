@@ -417,11 +417,24 @@ AttentionDevice attention_device(sgl_rocm_kv_ctx *ctx) {
             attention_resident};
 }
 
+// The tiles' own record buffer and the event that orders the calls that use
+// it, made at the first such call. False where there is no memory for them.
+bool attention_tile_records(sgl_rocm_kv_ctx *ctx) {
+    if (ctx->tile_records) return true;
+    if (!ctx->tile_order && hipEventCreateWithFlags(&ctx->tile_order, hipEventDisableTiming) != hipSuccess)
+        ctx->tile_order = nullptr;
+    if (!ctx->tile_order || hipMalloc(&ctx->tile_records, kAttentionTileRecordBytes) != hipSuccess) {
+        ctx->tile_records = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
 // Validates, sizes the split and launches the attention (and, with
 // several splits, the combine pass) on `stream`; nothing waits. Metadata
 // errors raise `flag_word`. `workspace` (fixed, `workspace_bytes` long)
-// holds the split records when given; otherwise the context's buffer,
-// grown on demand.
+// holds the split records when given; otherwise the context's buffers.
 int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *plan,
                           const sgl_kv_attention_buffers *b, uint64_t max_sequence_length,
                           hipStream_t s, uint32_t *flag_word, void *workspace = nullptr,
@@ -432,15 +445,27 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     if (rc) return rc;
     DeviceScope scope(ctx->device);
     if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
-    if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length, workspace_bytes, &p, &r)))
-        return rc;
+    const sglkv_attn_params unrouted = p;
+    AttentionRecords records = {workspace_bytes, true};
+    if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length, records, &p, &r))) return rc;
+    if (r.apart) {
+        // (An event recorded outside a capture cannot be waited on inside it.)
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        SGLKV_CHECK_HIP(hipStreamIsCapturing(s, &capture));
+        if (capture != hipStreamCaptureStatusNone || !attention_tile_records(ctx)) {
+            records.apart = false;
+            p = unrouted;
+            if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length, records, &p, &r)))
+                return rc;
+        }
+    }
     if (workspace) {
         if (r.record_bytes > workspace_bytes)
             return fail(SGL_KV_DIMENSION_TOO_LARGE, "workspace", r.record_bytes, workspace_bytes, 0,
                         "paged attention needs %llu bytes of split records, more than the "
                         "%llu-byte workspace",
                         (unsigned long long)r.record_bytes, (unsigned long long)workspace_bytes);
-    } else if (r.record_bytes > ctx->attention_partial_bytes) {
+    } else if (!r.apart && r.record_bytes > ctx->attention_partial_bytes) {
         if (ctx->attention_partial) {
             SGLKV_CHECK_HIP(hipDeviceSynchronize());
             SGLKV_CHECK_HIP(hipFree(ctx->attention_partial));
@@ -450,15 +475,21 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         SGLKV_CHECK_HIP(hipMalloc(&ctx->attention_partial, r.record_bytes));
         ctx->attention_partial_bytes = r.record_bytes;
     }
-    if (p.splits > 1) p.partial = static_cast<float *>(workspace ? workspace : ctx->attention_partial);
-    void *args[] = {&p};
-    SGLKV_CHECK_HIP(hipModuleLaunchKernel(ctx->attention[r.body], (unsigned)r.grid, p.splits, 1, r.threads, 1, 1, r.lds,
-                                          s, args, nullptr));
     if (p.splits > 1)
-        SGLKV_CHECK_HIP(hipModuleLaunchKernel(r.half_records ? ctx->attention_combine_h : ctx->attention_combine,
-                                              (unsigned)r.combine_grid, 1, 1, r.combine_threads, 1, 1, 0, s, args,
-                                              nullptr));
-    return SGL_KV_OK;
+        p.partial = static_cast<float *>(workspace ? workspace : r.apart ? ctx->tile_records : ctx->attention_partial);
+    if (r.apart) SGLKV_CHECK_HIP(hipStreamWaitEvent(s, ctx->tile_order, 0));
+    void *args[] = {&p};
+    hipError_t err = hipModuleLaunchKernel(ctx->attention[r.body], (unsigned)r.grid, p.splits, 1, r.threads, 1, 1, r.lds,
+                                           s, args, nullptr);
+    if (err == hipSuccess && p.splits > 1)
+        err = hipModuleLaunchKernel(r.half_records ? ctx->attention_combine_h : ctx->attention_combine,
+                                    (unsigned)r.combine_grid, 1, 1, r.combine_threads, 1, 1, 0, s, args, nullptr);
+    // Recorded also after a failure: a first launch may have been made.
+    if (r.apart) {
+        const hipError_t rec = hipEventRecord(ctx->tile_order, s);
+        if (err == hipSuccess) err = rec;
+    }
+    return err == hipSuccess ? SGL_KV_OK : hip_fail(err, "paged attention launch");
 }
 
 }  // namespace
@@ -497,7 +528,7 @@ extern "C" int32_t sgl_rocm_kv_attention_route(sgl_rocm_kv_ctx *ctx, const sgl_k
     if (rc) return rc;
     DeviceScope scope(ctx->device);
     if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
-    if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length, 0, &p, &r))) return rc;
+    if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length, {0, true}, &p, &r))) return rc;
     memset(out, 0, sizeof *out);
     out->body = (uint32_t)r.body;
     out->live_splits_first = p.compact != 0;
@@ -505,6 +536,7 @@ extern "C" int32_t sgl_rocm_kv_attention_route(sgl_rocm_kv_ctx *ctx, const sgl_k
     out->chunk_tokens = p.chunk_tokens;
     out->workgroups = r.grid * p.splits;
     out->record_bytes = r.record_bytes;
+    out->records_apart = r.apart;
     return ok();
 }
 

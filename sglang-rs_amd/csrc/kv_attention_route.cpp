@@ -343,7 +343,7 @@ int32_t split_tiles(const AttentionDevice &device, const sgl_kv_attention_plan_c
 }  // namespace
 
 int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, uint64_t max_len,
-                               uint64_t workspace_bytes, sglkv_attn_params *params, AttentionRoute *route) {
+                               const AttentionRecords &records, sglkv_attn_params *params, AttentionRoute *route) {
     sglkv_attn_params &p = *params;
     if (!max_len || max_len > c.sequence_slot_count) max_len = c.sequence_slot_count;
     p.page_stride32 = (uint32_t)c.layout.page_stride_bytes;
@@ -354,17 +354,35 @@ int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_atten
     Split s = {0, 0, 0, 0};
     uint64_t block = SGLKV_ATTN_TOKENS;
     const TileShape shape(c, p, max_len);
+    route->apart = false;
     if (tiles_take(device, c, p, max_len) &&
         (body.which < kAttnStaged128 || shape.pays(device.cus, c.query_count * p.kv_heads))) {
+        const Body single = body;
         body = {p.dk == 128 ? kAttnTile128 : p.dk == 64 ? kAttnTile64 : kAttnTile256, 256,
                 SGLKV_ATTN_TILE_LDS_BYTES(p.dk)};
         block = SGLKV_ATTN_TILE_BLOCK(p.dk);
-        const int32_t rc = split_tiles(device, c, shape, body, max_len, workspace_bytes, &p, &s);
+        const int32_t rc = split_tiles(device, c, shape, body, max_len, records.workspace_bytes, &p, &s);
         if (rc) return rc;
+        // The calls of a context that split share one buffer, so a caller
+        // issues them on one stream. Where the per-query body would not split,
+        // the caller need not: those records go to the tiles' own buffer,
+        // whose calls the library orders itself, or the tiles stay whole
+        // (where there is no such buffer, and under graph capture).
+        Split alone = {0, 0, 0, 0};
+        if (s.splits > 1 && !records.workspace_bytes &&
+            (split_queries(device, c, p, single, max_len, &alone) != SGL_KV_OK || alone.splits == 1)) {
+            uint64_t bytes;
+            route->apart = records.apart && record_bytes(c, p, false, s.splits, &bytes) &&
+                           bytes <= kAttentionTileRecordBytes;
+            if (!route->apart) {
+                s.chunk = whole_blocks(max_len, block);
+                s.splits = 1;
+            }
+        }
     } else {
         const int32_t rc = split_queries(device, c, p, body, max_len, &s);
         if (rc) return rc;
-        split_ragged(c, body, max_len, workspace_bytes, &p, &s);
+        split_ragged(c, body, max_len, records.workspace_bytes, &p, &s);
     }
     if (s.splits > 65535) {  // grid y limit
         p.compact = 0;

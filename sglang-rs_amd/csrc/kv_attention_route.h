@@ -44,6 +44,7 @@ struct AttentionRoute {
     uint64_t grid;            // workgroups of one split (p->splits of them in y)
     bool half_records;        // scaled fp16 split records (SGLKV_ATTN_HPAD)
     uint64_t record_bytes;    // all split records of the launch (0: one split)
+    bool apart;               // the records go to the tiles' own buffer
     uint64_t combine_grid;
     unsigned combine_threads;
 };
@@ -51,11 +52,23 @@ struct AttentionRoute {
 // The reference's overflow error.
 int32_t attention_overflow();
 
+// Where split records can go: the caller's fixed workspace (its size, 0 if
+// there is none), else the buffer that all splitting calls of a context share,
+// or, where `apart`, the tiles' own.
+struct AttentionRecords {
+    uint64_t workspace_bytes;
+    bool apart;
+};
+// The size of the tiles' own buffer. A launch of tiles leaves at most
+// SGLKV_ATTN_TILE_ROWS records for each workgroup that it splits into, and no
+// more of these than stay resident at once: 34 MB at dims 128 and 256 and 26 MB at
+// dims 64 on 256 CUs.
+constexpr uint64_t kAttentionTileRecordBytes = 64ull << 20;
+
 // Chooses for `p`, whose pointers, sizes, strides and page_shift are set, and
-// sets its launch fields (chunk_tokens, splits, ...). `workspace_bytes`: the
-// size of the caller's fixed workspace, 0 if the records' buffer can grow.
+// sets its launch fields (chunk_tokens, splits, ...).
 int32_t attention_route(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, uint64_t max_len,
-                        uint64_t workspace_bytes, sglkv_attn_params *p, AttentionRoute *r);
+                        const AttentionRecords &records, sglkv_attn_params *p, AttentionRoute *r);
 
 }  // namespace sglkv
 

@@ -169,6 +169,8 @@ struct sgl_rocm_kv_ctx {
     const uint8_t *zero_row;        // SGLKV_ZERO_ROW_BYTES of zeros inside that block
     void *attention_partial;        // split records, grown on demand
     uint64_t attention_partial_bytes;
+    void *tile_records;             // split records of tile launches whose queries alone would not split
+    hipEvent_t tile_order;          // after the last of these, on whatever stream
     void *noalloc_workspace;        // this device's static workspace (SGL_KV_NOALLOC_WORKSPACE_BYTES)
     sglkv::NoallocOrder *noalloc_order;  // its ordering across streams and contexts
     uint32_t rows_per_thread;  // from the code object

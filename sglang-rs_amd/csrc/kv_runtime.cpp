@@ -588,6 +588,8 @@ extern "C" int32_t sgl_rocm_kv_destroy(sgl_rocm_kv_ctx *ctx) {
     if (!ctx) return ok();
     DeviceScope scope(ctx->device);
     if (ctx->attention_partial) (void)hipFree(ctx->attention_partial);
+    if (ctx->tile_records) (void)hipFree(ctx->tile_records);
+    if (ctx->tile_order) (void)hipEventDestroy(ctx->tile_order);
     (void)hipHostFree(ctx->host_words);
     hipError_t e1 = hipFree(ctx->flag);
     hipError_t e2 = hipModuleUnload(ctx->module);

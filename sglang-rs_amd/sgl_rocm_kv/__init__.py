@@ -322,7 +322,7 @@ class _AttentionBuffers(ctypes.Structure):
 
 class _AttentionRoute(ctypes.Structure):
     _fields_ = [("body", ctypes.c_uint32), ("live_splits_first", ctypes.c_uint32), ("splits", _u64),
-                ("chunk_tokens", _u64), ("workgroups", _u64), ("record_bytes", _u64)]
+                ("chunk_tokens", _u64), ("workgroups", _u64), ("record_bytes", _u64), ("records_apart", _u64)]
 
 
 # SGL_KV_ATTN_BODY_*, by value
@@ -339,6 +339,7 @@ class AttentionRoute:
     chunk_tokens: int
     workgroups: int
     record_bytes: int
+    records_apart: bool
 
 
 PAGE_REQUEST_DTYPE = np.dtype([("source", "<u8"), ("target_offset", "<u8"), ("length", "<u8")])
@@ -1321,7 +1322,7 @@ class RocmKvPairCopyKernels:
         _call(lib().sgl_rocm_kv_attention_route, self._h, ctypes.byref(plan._c),
               ctypes.byref(_attention_buffers(buffers)), max_sequence_length, ctypes.byref(r))
         return AttentionRoute(ATTENTION_BODIES[r.body], bool(r.live_splits_first), r.splits, r.chunk_tokens,
-                              r.workgroups, r.record_bytes)
+                              r.workgroups, r.record_bytes, bool(r.records_apart))
 
     def paged_attention_async_noalloc(self, plan: "PagedAttentionPlan", *, max_sequence_length: int = 0,
                                       stream=None, **buffers):

@@ -37,7 +37,7 @@ struct Routed {
     AttentionRoute r;
 };
 
-Routed route(const Call &x, uint64_t workspace = 0) {
+Routed route(const Call &x, const AttentionRecords &records = {0, true}) {
     Routed o;
     memset(&o, 0, sizeof o);
     sgl_kv_attention_plan_config c;
@@ -76,7 +76,7 @@ Routed route(const Call &x, uint64_t workspace = 0) {
     p.dv = x.dv;
     p.dv_blocks = (x.dv + SGLKV_ATTN_DV - 1) / SGLKV_ATTN_DV;
     p.page_shift = 6;
-    o.rc = attention_route(kDevice, c, x.max_len, workspace, &p, &o.r);
+    o.rc = attention_route(kDevice, c, x.max_len, records, &p, &o.r);
     return o;
 }
 
@@ -128,6 +128,25 @@ void check(const Call &x, const Routed &o) {
     if (o.r.record_bytes != (splits > 1 ? x.queries * x.qheads * splits * record : 0)) fail_call("records", x, o);
 }
 
+// Records go to the buffer that all splitting calls share only where the
+// queries one by one (as many requests, so no tiles) would be split too.
+void check_apart(const Call &x, const Routed &o) {
+    if (!is_tile(o.r.body)) {
+        if (o.r.apart) fail_call("no tiles, but records apart", x, o);
+        return;
+    }
+    Call single = x;
+    single.requests = x.queries;
+    const Routed alone = route(single);
+    const bool splits = alone.rc == SGL_KV_OK && alone.p.splits > 1;
+    if (o.r.apart != (o.p.splits > 1 && !splits)) fail_call("records in the wrong buffer", x, o);
+    if (o.r.record_bytes > kAttentionTileRecordBytes) fail_call("more records than the tiles' buffer holds", x, o);
+    // Without that buffer the call is made all the same, in whole tiles.
+    const Routed without = route(x, {0, false});
+    check(x, without);
+    if (without.r.apart || (!splits && without.p.splits != 1)) fail_call("records without a buffer", x, without);
+}
+
 struct Shape {
     uint32_t qheads, heads, dk, dv;
 };
@@ -150,7 +169,9 @@ void random_calls() {
         x.slots = mean * x.requests;
         if (x.slots < x.max_len) x.slots = x.max_len;
         if (rng() % 8 == 0) x.max_len = 0;
-        check(x, route(x));
+        const Routed o = route(x);
+        check(x, o);
+        if (o.rc == SGL_KV_OK) check_apart(x, o);
     }
 }
 

@@ -8,11 +8,13 @@ A tile holds up to 128 (query, query head) rows of one request, its tokens
 come in blocks of 64, and the slot table covers 2,048 (dims 64) or 4,096
 tokens, so the sizes below sit at those edges.
 """
+import ctypes
 import math
 
 import numpy as np
 import pytest
 
+import oracle
 import sgl_rocm_kv as kv
 from sgl_rocm_kv import hip
 from test_gpu_attention import _bf16_normal, _Case, _check, _say
@@ -131,3 +133,124 @@ def test_bad_slot_is_reported(k):
     with pytest.raises(kv.KvError) as e:
         c.run(k, q, np.zeros(64, int), 100 + np.arange(64), [0, 200], slots, 0.1, max_len=200)
     assert e.value.variant == "DeviceMetadataInvalid" and e.value.fields[0] == 4
+
+
+class _Call:
+    """Device buffers of one call, for launches into outputs of their own."""
+
+    def __init__(self, c, q, qri, qsl, rso, slots, max_len):
+        self.plan = kv.PagedAttentionPlan.for_layer(c.layout, c.layer, len(qri), len(rso) - 1, len(slots), c.qh,
+                                                    1.0 / math.sqrt(c.dk), kv.HND if c.hnd else kv.NHD)
+        arrays = dict(queries=q, query_request_indices=np.asarray(qri, np.uint32),
+                      query_sequence_lengths=np.asarray(qsl, np.uint64),
+                      request_slot_offsets=np.asarray(rso, np.uint64), sequence_slots=np.asarray(slots, np.uint64))
+        self.bufs = {n: hip.DeviceBuffer.from_array(a) for n, a in arrays.items()}
+        self.bufs["pool"], self.max_len = c.pool, max_len
+
+    def output(self):
+        out = hip.DeviceBuffer(self.plan.output_required_bytes)
+        out.fill(0xFF)
+        return out
+
+    def run(self, k, out, stream=None):
+        k.paged_attention_async(self.plan, max_sequence_length=self.max_len, stream=stream, output=out, **self.bufs)
+
+    def route(self, k):
+        out = self.output()
+        return k.attention_route(self.plan, max_sequence_length=self.max_len, output=out, **self.bufs)
+
+
+def _chunk_call(seed, H, qh, d, cached, queries):
+    rng = np.random.default_rng(seed)
+    c = _Case(rng, P=16, L=1, H=H, dk=d, dv=d, qh=qh, pages=(cached + queries) // 16 + 3, layer=0)
+    qri, qsl, rso, slots = _requests(rng, [(cached, queries)], c.layout.slot_count)
+    q = _bf16_normal(rng, queries * qh * d).reshape(queries, qh, d)
+    return _Call(c, q, qri, qsl, rso, slots, cached + queries)
+
+
+def test_calls_on_several_streams_keep_their_records_apart(k):
+    """Chunks of prompts that are split only because their tiles are few, on
+    two streams, beside a decode call on a third whose records are in the
+    context's shared buffer: each result equals that of the call alone."""
+    first, second = _chunk_call(1, 8, 32, 128, 600, 384), _chunk_call(2, 8, 32, 64, 700, 300)
+    for call, body in ((first, "tile128"), (second, "tile64")):
+        route = call.route(k)
+        assert route.body == body and route.splits > 1 and route.records_apart
+    rng = np.random.default_rng(3)
+    c = _Case(rng, P=16, L=1, H=8, dk=128, dv=128, qh=32, pages=600, layer=0)
+    decode = _Call(c, _bf16_normal(rng, 2 * 32 * 128).reshape(2, 32, 128), [0, 1], [4000, 3000], [0, 4000, 7000],
+                   rng.choice(c.layout.slot_count, size=7000, replace=False), 4000)
+    route = decode.route(k)
+    assert route.body == "staged128" and route.splits > 1 and not route.records_apart
+    calls = (first, second, decode)
+    want = []
+    for call in calls:
+        out = call.output()
+        call.run(k, out)
+        hip.synchronize()
+        want.append(out.download(dtype=np.uint16))
+        assert not np.all(want[-1] == 0xFFFF)
+    streams = [hip.Stream() for _ in calls]
+    outs = [[call.output() for call in calls] for _ in range(20)]
+    hip.synchronize()
+    _say("tiles: 60 calls on three streams")
+    for row in outs:
+        for call, out, stream in zip(calls, row, streams):
+            call.run(k, out, stream)
+    for stream in streams:
+        stream.synchronize()
+    k.check_errors()
+    for i, row in enumerate(outs):
+        for out, w in zip(row, want):
+            np.testing.assert_array_equal(out.download(dtype=np.uint16), w, err_msg=f"round {i}")
+    for stream in streams:
+        stream.destroy()
+
+
+def test_captured_call_is_not_split(k):
+    """The same chunk under graph capture, in a context that has split
+    nothing yet: it is captured (nothing is allocated, no event waited for),
+    and every replay matches the eager result up to the splits' rounding."""
+    call = _chunk_call(4, 8, 32, 128, 600, 384)
+    ctx = kv.RocmKvPairCopyKernels(0)
+    assert call.route(ctx).records_apart
+    out, stream = call.output(), hip.Stream()
+    h, vp = hip.lib(), ctypes.c_void_p
+    h.hipStreamBeginCapture.argtypes = [vp, ctypes.c_int]
+    h.hipStreamEndCapture.argtypes = [vp, ctypes.POINTER(vp)]
+    h.hipGraphInstantiate.argtypes = [ctypes.POINTER(vp), vp, vp, vp, ctypes.c_size_t]
+    h.hipGraphLaunch.argtypes = [vp, vp]
+    h.hipGraphExecDestroy.argtypes = [vp]
+    h.hipGraphDestroy.argtypes = [vp]
+    hip.synchronize()
+    graph, execution = vp(), vp()
+    _say("tiles: a chunk under graph capture")
+    hip.check(h.hipStreamBeginCapture(stream.handle, 0), "hipStreamBeginCapture")
+    call.run(ctx, out, stream)
+    hip.check(h.hipStreamEndCapture(stream.handle, ctypes.byref(graph)), "hipStreamEndCapture")
+    hip.check(h.hipGraphInstantiate(ctypes.byref(execution), graph, None, None, 0), "hipGraphInstantiate")
+    eager = call.output()
+    call.run(ctx, eager)
+    hip.synchronize()
+    want = eager.download(dtype=np.uint16)
+    replays = []
+    for i in range(3):
+        out.fill(0xFF)
+        hip.synchronize()
+        hip.check(h.hipGraphLaunch(execution, stream.handle), "hipGraphLaunch")
+        stream.synchronize()
+        replays.append(out.download(dtype=np.uint16))
+        call.run(ctx, eager)  # eager work between the replays
+        hip.synchronize()
+        np.testing.assert_array_equal(eager.download(dtype=np.uint16), want)
+    ctx.check_errors()
+    a, b = (oracle.bf16_to_f32(x).astype(np.float64) for x in (replays[0], want))
+    # Both are within the bound of _check of one exact value: a bf16 rounding
+    # each and 2^-12 of sum w|v| (|v| <= 5.5 here) each.
+    assert (np.abs(a - b) <= 2 * (2.0 ** -8 * np.abs(a) + 5.5 * 2.0 ** -12)).all()
+    for r in replays[1:]:
+        np.testing.assert_array_equal(r, replays[0])
+    hip.check(h.hipGraphExecDestroy(execution), "hipGraphExecDestroy")
+    hip.check(h.hipGraphDestroy(graph), "hipGraphDestroy")
+    stream.destroy()
+    ctx.close()
