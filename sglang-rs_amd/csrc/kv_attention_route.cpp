@@ -303,7 +303,7 @@ bool tiles_take(const AttentionDevice &device, const sgl_kv_attention_plan_confi
 
 // Splits for a launch of tiles.
 int32_t split_tiles(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, const TileShape &shape,
-                    const Body &body, uint64_t max_len, uint64_t workspace_bytes, sglkv_attn_params *params, Split *s) {
+                    const Body &body, uint64_t max_len, sglkv_attn_params *params, Split *s) {
     sglkv_attn_params &p = *params;
     p.tile_queries = (uint32_t)shape.queries;
     p.tile_recip = UINT32_MAX / p.tile_queries + 1;
@@ -327,15 +327,7 @@ int32_t split_tiles(const AttentionDevice &device, const sgl_kv_attention_plan_c
     // prompt of 1,500 tokens, dims 128, 55 -> 51 us, of 2,048 77 -> 74).
     if (p.tile_backward && base <= target && base > device.cus && shape.splits(target) == 1)
         p.tile_fold = (uint32_t)device.cus / p.kv_heads;
-    uint64_t want = shape.splits(target);
-    if (workspace_bytes) {
-        // Never more split records than the fixed workspace holds: fewer,
-        // longer splits instead (the tile bodies take chunks of any length).
-        const uint64_t record = 4ull * (SGLKV_ATTN_OPAD(p.dv) + 2);
-        const uint64_t room = workspace_bytes / record / (c.query_count * c.query_head_count);
-        if (want > room) want = room ? room : 1;
-    }
-    s->chunk = whole_blocks(ceil_div(max_len, want), SGLKV_ATTN_TILE_BLOCK(p.dk));
+    s->chunk = whole_blocks(ceil_div(max_len, shape.splits(target)), SGLKV_ATTN_TILE_BLOCK(p.dk));
     s->splits = ceil_div(max_len, s->chunk);
     return SGL_KV_OK;
 }
@@ -361,7 +353,7 @@ int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_atten
         body = {p.dk == 128 ? kAttnTile128 : p.dk == 64 ? kAttnTile64 : kAttnTile256, 256,
                 SGLKV_ATTN_TILE_LDS_BYTES(p.dk)};
         block = SGLKV_ATTN_TILE_BLOCK(p.dk);
-        const int32_t rc = split_tiles(device, c, shape, body, max_len, records.workspace_bytes, &p, &s);
+        const int32_t rc = split_tiles(device, c, shape, body, max_len, &p, &s);
         if (rc) return rc;
         // The calls of a context that split share one buffer, so a caller
         // issues them on one stream. Where the per-query body would not split,

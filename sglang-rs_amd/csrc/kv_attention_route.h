@@ -62,7 +62,7 @@ struct AttentionRecords {
 // The size of the tiles' own buffer. A launch of tiles leaves at most
 // SGLKV_ATTN_TILE_ROWS records for each workgroup that it splits into, and no
 // more of these than stay resident at once: 34 MB at dims 128 and 256 and 26 MB at
-// dims 64 on 256 CUs.
+// dims 64 on 256 CUs (well inside the no-allocation entry point's workspace, too).
 constexpr uint64_t kAttentionTileRecordBytes = 64ull << 20;
 
 // Chooses for `p`, whose pointers, sizes, strides and page_shift are set, and

@@ -141,6 +141,9 @@ void check_apart(const Call &x, const Routed &o) {
     const bool splits = alone.rc == SGL_KV_OK && alone.p.splits > 1;
     if (o.r.apart != (o.p.splits > 1 && !splits)) fail_call("records in the wrong buffer", x, o);
     if (o.r.record_bytes > kAttentionTileRecordBytes) fail_call("more records than the tiles' buffer holds", x, o);
+    const Routed fixed = route(x, {SGL_KV_NOALLOC_WORKSPACE_BYTES, true});
+    check(x, fixed);
+    if (fixed.r.record_bytes > kAttentionTileRecordBytes) fail_call("more tile records than a workspace takes", x, fixed);
     // Without that buffer the call is made all the same, in whole tiles.
     const Routed without = route(x, {0, false});
     check(x, without);
