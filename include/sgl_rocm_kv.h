@@ -900,7 +900,8 @@ int32_t sgl_kv_attention_plan_for_layer(const sgl_kv_paged_layout *layout, uint6
  * query lengths and steers how sequences are split across workgroups; a
  * query longer than it is reported as a sequence error (flag 0x2), not
  * truncated. Long sequences use a
- * context-owned workspace, grown on demand. */
+ * context-owned workspace of 128 MiB (made at the first call that splits;
+ * smaller where memory is short), grown for calls that need more. */
 int32_t sgl_rocm_kv_paged_attention(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *plan,
                                     const sgl_kv_attention_buffers *buffers,
                                     uint64_t max_sequence_length, void *stream);
@@ -976,7 +977,8 @@ int32_t sgl_rocm_kv_attention_route(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention
  * there the graph's own dependencies order the calls it holds, and the
  * caller must not replay such a graph while another call that uses the
  * workspace runs. Results equal those of sgl_rocm_kv_paged_attention_async
- * on the same arguments. */
+ * on the same arguments, bit for bit, unless that call was split otherwise for
+ * want of a record buffer (under graph capture, or where memory is short). */
 #define SGL_KV_NOALLOC_WORKSPACE_BYTES (128ull << 20)
 int32_t sgl_rocm_kv_paged_attention_async_noalloc(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *plan,
                                                   const sgl_kv_attention_buffers *buffers,

@@ -435,6 +435,36 @@ bool attention_tile_records(sgl_rocm_kv_ctx *ctx) {
     return true;
 }
 
+// Where a call's records can go.
+AttentionRecords attention_records(const sgl_rocm_kv_ctx *ctx, uint64_t workspace_bytes) {
+    const uint64_t held = workspace_bytes ? workspace_bytes : ctx->attention_partial_bytes;
+    return {workspace_bytes, held && held < kAttentionShorterBytes ? held : kAttentionShorterBytes, true};
+}
+
+// Makes the context's record buffer hold `bytes`; a new one holds
+// kAttentionShorterBytes, or `bytes` alone where memory is short.
+hipError_t attention_grow(sgl_rocm_kv_ctx *ctx, uint64_t bytes) {
+    if (ctx->attention_partial) {
+        hipError_t err = hipDeviceSynchronize();
+        if (err == hipSuccess) err = hipFree(ctx->attention_partial);
+        if (err != hipSuccess) return err;
+        ctx->attention_partial = nullptr;
+        ctx->attention_partial_bytes = 0;
+    }
+    uint64_t size = bytes < kAttentionShorterBytes ? kAttentionShorterBytes : bytes;
+    hipError_t err = hipMalloc(&ctx->attention_partial, size);
+    if (err == hipErrorOutOfMemory && size > bytes) {
+        (void)hipGetLastError();
+        size = bytes;
+        err = hipMalloc(&ctx->attention_partial, size);
+    }
+    if (err == hipSuccess)
+        ctx->attention_partial_bytes = size;
+    else
+        ctx->attention_partial = nullptr;
+    return err;
+}
+
 // Validates, sizes the split and launches the attention (and, with
 // several splits, the combine pass) on `stream`; nothing waits. Metadata
 // errors raise `flag_word`. `workspace` (fixed, `workspace_bytes` long)
@@ -450,18 +480,22 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
     DeviceScope scope(ctx->device);
     if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
     const sglkv_attn_params unrouted = p;
-    AttentionRecords records = {workspace_bytes, true};
-    if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length, records, &p, &r))) return rc;
-    if (r.apart) {
-        // (An event recorded outside a capture cannot be waited on inside it.)
+    AttentionRecords records = attention_records(ctx, workspace_bytes);
+    auto route = [&] {
+        p = unrouted;
+        return attention_route(attention_device(ctx), plan->config, max_sequence_length, records, &p, &r);
+    };
+    if ((rc = route())) return rc;
+    const bool grows = !workspace && !r.apart && r.record_bytes > ctx->attention_partial_bytes;
+    if (r.apart || (grows && r.shortened)) {
+        // A capture can neither allocate nor wait for an event recorded
+        // outside it.
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         SGLKV_CHECK_HIP(hipStreamIsCapturing(s, &capture));
-        if (capture != hipStreamCaptureStatusNone || !attention_tile_records(ctx)) {
-            records.apart = false;
-            p = unrouted;
-            if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length, records, &p, &r)))
-                return rc;
-        }
+        const bool captures = capture != hipStreamCaptureStatusNone;
+        if (r.apart) records.apart = !captures && attention_tile_records(ctx);
+        if (r.shortened && captures) records.shorter = 0;
+        if ((!records.apart || !records.shorter) && (rc = route())) return rc;
     }
     if (workspace) {
         if (r.record_bytes > workspace_bytes)
@@ -470,14 +504,14 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
                         "%llu-byte workspace",
                         (unsigned long long)r.record_bytes, (unsigned long long)workspace_bytes);
     } else if (!r.apart && r.record_bytes > ctx->attention_partial_bytes) {
-        if (ctx->attention_partial) {
-            SGLKV_CHECK_HIP(hipDeviceSynchronize());
-            SGLKV_CHECK_HIP(hipFree(ctx->attention_partial));
-            ctx->attention_partial = nullptr;
-            ctx->attention_partial_bytes = 0;
+        hipError_t err = attention_grow(ctx, r.record_bytes);
+        if (err == hipErrorOutOfMemory && r.shortened) {
+            (void)hipGetLastError();
+            records.shorter = 0;
+            if ((rc = route())) return rc;
+            err = attention_grow(ctx, r.record_bytes);
         }
-        SGLKV_CHECK_HIP(hipMalloc(&ctx->attention_partial, r.record_bytes));
-        ctx->attention_partial_bytes = r.record_bytes;
+        if (err != hipSuccess) return hip_fail(err, "hipMalloc");
     }
     if (p.splits > 1)
         p.partial = static_cast<float *>(workspace ? workspace : r.apart ? ctx->tile_records : ctx->attention_partial);
@@ -532,7 +566,9 @@ extern "C" int32_t sgl_rocm_kv_attention_route(sgl_rocm_kv_ctx *ctx, const sgl_k
     if (rc) return rc;
     DeviceScope scope(ctx->device);
     if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
-    if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length, {0, true}, &p, &r))) return rc;
+    if ((rc = attention_route(attention_device(ctx), plan->config, max_sequence_length,
+                              attention_records(ctx, 0), &p, &r)))
+        return rc;
     memset(out, 0, sizeof *out);
     out->body = (uint32_t)r.body;
     out->live_splits_first = p.compact != 0;

@@ -203,28 +203,31 @@ bool record_bytes(const sgl_kv_attention_plan_config &c, const sglkv_attn_params
 // order, 48 so; 9 of 739..5,919 69 and 47).
 // Batches nearer one length keep the split above (33 queries of 500..1,300:
 // 33 us either way, 34 with this one; 128 of 2,000..3,000: 239, 250).
-void split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint64_t max_len, uint64_t workspace_bytes,
+// Their records, up to 9 times those of equal splits (one MLA query of 65,536
+// tokens among 31 of 1,000: 626 MB against 68), stay within `shorter` bytes.
+// Returns whether the splits were made shorter.
+bool split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint64_t max_len, uint64_t shorter,
                   sglkv_attn_params *params, Split *s) {
     sglkv_attn_params &p = *params;
     const int which = body.which;
     if (s->splits < 2 || (which != kAttnLatent && which < kAttnStaged128) ||
         c.query_count > SGLKV_ATTN_COMPACT_QUERIES)
-        return;
+        return false;
     const uint64_t mean = ceil_div(c.sequence_slot_count, requests(c)), base = s->base, target = s->target;
     uint64_t total;  // tokens times the workgroups that share them
-    if (mean >= max_len - max_len / 3 || mul_ovf(mean, base, &total)) return;
+    if (mean >= max_len - max_len / 3 || mul_ovf(mean, base, &total)) return false;
     const bool worth = total / target >= (which == kAttnStaged64 ? 96 : 128);
     const uint64_t room = which == kAttnLatent ? target : target / 20 * 17;
     uint64_t balanced = room > base ? ceil_div(total, room - base) : s->chunk;
     const uint64_t least = which == kAttnLatent ? (max_len > 4096 ? 128 : 64) : (s->chunk < 192 ? s->chunk : 192);
     const uint64_t most = which == kAttnLatent || max_len > 32768 ? s->chunk : 512;
     balanced = balanced < least ? least : (balanced > most ? most : balanced);
-    balanced = whole_blocks(balanced, SGLKV_ATTN_TOKENS);
-    // (Never more records than the fixed workspace holds.)
     uint64_t bytes;
-    const bool fits = !workspace_bytes || (record_bytes(c, p, which == kAttnLatent, ceil_div(max_len, balanced), &bytes) &&
-                                           bytes <= workspace_bytes);
-    if (balanced < s->chunk && fits && (worth || which == kAttnLatent)) {
+    if (!record_bytes(c, p, which == kAttnLatent, 1, &bytes)) return false;
+    const uint64_t fit = ceil_div(max_len, shorter / bytes ? shorter / bytes : 1);
+    balanced = whole_blocks(balanced < fit ? fit : balanced, SGLKV_ATTN_TOKENS);
+    const bool shortened = balanced < s->chunk && (worth || which == kAttnLatent);
+    if (shortened) {
         s->chunk = balanced;
         s->splits = ceil_div(max_len, s->chunk);
     }
@@ -232,6 +235,7 @@ void split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint6
         base * s->splits <= UINT32_MAX)
         p.compact = c.layout.head_layout == SGL_KV_HND || base == c.query_count ? SGLKV_ATTN_COMPACT_HEADS_FIRST
                                                                                 : SGLKV_ATTN_COMPACT_QUERY_FIRST;
+    return shortened;
 }
 
 // The tiles of a launch with several queries per request, and whether they
@@ -346,7 +350,7 @@ int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_atten
     Split s = {0, 0, 0, 0};
     uint64_t block = SGLKV_ATTN_TOKENS;
     const TileShape shape(c, p, max_len);
-    route->apart = false;
+    route->apart = route->shortened = false;
     if (tiles_take(device, c, p, max_len) &&
         (body.which < kAttnStaged128 || shape.pays(device.cus, c.query_count * p.kv_heads))) {
         const Body single = body;
@@ -374,7 +378,7 @@ int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_atten
     } else {
         const int32_t rc = split_queries(device, c, p, body, max_len, &s);
         if (rc) return rc;
-        split_ragged(c, body, max_len, records.workspace_bytes, &p, &s);
+        route->shortened = split_ragged(c, body, max_len, records.shorter, &p, &s);
     }
     if (s.splits > 65535) {  // grid y limit
         p.compact = 0;

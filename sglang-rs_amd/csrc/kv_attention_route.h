@@ -45,6 +45,7 @@ struct AttentionRoute {
     bool half_records;        // scaled fp16 split records (SGLKV_ATTN_HPAD)
     uint64_t record_bytes;    // all split records of the launch (0: one split)
     bool apart;               // the records go to the tiles' own buffer
+    bool shortened;           // a ragged batch's splits, shorter than equal ones
     uint64_t combine_grid;
     unsigned combine_threads;
 };
@@ -54,11 +55,17 @@ int32_t attention_overflow();
 
 // Where split records can go: the caller's fixed workspace (its size, 0 if
 // there is none), else the buffer that all splitting calls of a context share,
-// or, where `apart`, the tiles' own.
+// or, where `apart`, the tiles' own. A ragged batch's splits are made shorter
+// than equal ones as far as their records fit `shorter` bytes.
 struct AttentionRecords {
     uint64_t workspace_bytes;
+    uint64_t shorter;
     bool apart;
 };
+// The most that shorter splits may take, with the no-allocation entry point's
+// workspace as without, so that both split alike; the context's buffer starts
+// at this size, so that a call never makes it grow for shorter splits.
+constexpr uint64_t kAttentionShorterBytes = SGL_KV_NOALLOC_WORKSPACE_BYTES;
 // The size of the tiles' own buffer. A launch of tiles leaves at most
 // SGLKV_ATTN_TILE_ROWS records for each workgroup that it splits into, and no
 // more of these than stay resident at once: 34 MB at dims 128 and 256 and 26 MB at

@@ -37,7 +37,7 @@ struct Routed {
     AttentionRoute r;
 };
 
-Routed route(const Call &x, const AttentionRecords &records = {0, true}) {
+Routed route(const Call &x, const AttentionRecords &records = {0, kAttentionShorterBytes, true}) {
     Routed o;
     memset(&o, 0, sizeof o);
     sgl_kv_attention_plan_config c;
@@ -128,6 +128,8 @@ void check(const Call &x, const Routed &o) {
     if (o.r.record_bytes != (splits > 1 ? x.queries * x.qheads * splits * record : 0)) fail_call("records", x, o);
 }
 
+int shortened = 0;
+
 // Records go to the buffer that all splitting calls share only where the
 // queries one by one (as many requests, so no tiles) would be split too.
 void check_apart(const Call &x, const Routed &o) {
@@ -141,13 +143,28 @@ void check_apart(const Call &x, const Routed &o) {
     const bool splits = alone.rc == SGL_KV_OK && alone.p.splits > 1;
     if (o.r.apart != (o.p.splits > 1 && !splits)) fail_call("records in the wrong buffer", x, o);
     if (o.r.record_bytes > kAttentionTileRecordBytes) fail_call("more records than the tiles' buffer holds", x, o);
-    const Routed fixed = route(x, {SGL_KV_NOALLOC_WORKSPACE_BYTES, true});
+    const Routed fixed = route(x, {SGL_KV_NOALLOC_WORKSPACE_BYTES, kAttentionShorterBytes, true});
     check(x, fixed);
     if (fixed.r.record_bytes > kAttentionTileRecordBytes) fail_call("more tile records than a workspace takes", x, fixed);
     // Without that buffer the call is made all the same, in whole tiles.
-    const Routed without = route(x, {0, false});
+    const Routed without = route(x, {0, kAttentionShorterBytes, false});
     check(x, without);
     if (without.r.apart || (!splits && without.p.splits != 1)) fail_call("records without a buffer", x, without);
+}
+
+// A ragged batch's splits take no more than the bytes they may, nor more than
+// the equal splits where these bytes are few, and the same with a workspace.
+void check_ragged(const Call &x, const Routed &o) {
+    const Routed equal = route(x, {0, 0, true});
+    check(x, equal);
+    if (equal.r.shortened || o.r.record_bytes < equal.r.record_bytes) fail_call("longer than equal splits", x, o);
+    if (o.r.shortened ? o.r.record_bytes > kAttentionShorterBytes : o.r.record_bytes != equal.r.record_bytes)
+        fail_call("records past their bound", x, o);
+    const Routed fixed = route(x, {SGL_KV_NOALLOC_WORKSPACE_BYTES, kAttentionShorterBytes, true});
+    if (fixed.p.chunk_tokens != o.p.chunk_tokens || fixed.p.splits != o.p.splits || fixed.p.compact != o.p.compact ||
+        fixed.r.body != o.r.body)
+        fail_call("another split with a workspace", x, o);
+    if (o.r.shortened) ++shortened;
 }
 
 struct Shape {
@@ -174,7 +191,9 @@ void random_calls() {
         if (rng() % 8 == 0) x.max_len = 0;
         const Routed o = route(x);
         check(x, o);
-        if (o.rc == SGL_KV_OK) check_apart(x, o);
+        if (o.rc != SGL_KV_OK) continue;
+        check_apart(x, o);
+        check_ragged(x, o);
     }
 }
 
@@ -195,6 +214,10 @@ void no_requests() {
 int main() {
     no_requests();
     random_calls();
+    if (shortened < 1000) {
+        std::fprintf(stderr, "only %d ragged batches\n", shortened);
+        return 1;
+    }
     std::puts("attention route ok");
     return 0;
 }

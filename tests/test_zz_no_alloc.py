@@ -101,6 +101,22 @@ def test_noalloc_matches_the_allocating_entry_point_twice(k, shape):
     np.testing.assert_array_equal(big.run(k, noalloc=True), big.run(k, noalloc=False))
 
 
+def test_ragged_batch_splits_alike_in_both_entry_points(k):
+    """One MLA query of 65,536 tokens among eight of 1,000: splits that fill
+    the chip would leave 245 MB of records. Both entry points stop at the
+    workspace's 128 MiB, so the results are equal bit for bit, and the
+    allocating one needs no more than the other (the call with the shortest
+    splits that fit)."""
+    rng = np.random.default_rng(99)
+    case = _Decode(rng, 64, 1, 576, 512, 128, [1000] * 4 + [65536] + [1000] * 4)
+    out = hip.DeviceBuffer(case.plan.output_required_bytes)
+    route = k.attention_route(case.plan, max_sequence_length=case.max_len, output=out, **case.bufs)
+    _say(f"noalloc: ragged MLA, {route}")
+    np.testing.assert_array_equal(case.run(k, noalloc=True), case.run(k, noalloc=False))
+    assert route.live_splits_first and route.chunk_tokens < 4096
+    assert kv.NOALLOC_WORKSPACE_BYTES * 0.95 < route.record_bytes <= kv.NOALLOC_WORKSPACE_BYTES
+
+
 def test_noalloc_calls_on_two_streams_and_two_contexts_are_ordered(k):
     """Twelve no-allocation decodes issued back to back, with no host wait,
     alternating between two streams and two contexts of one device, GQA
