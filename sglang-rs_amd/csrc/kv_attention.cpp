@@ -517,8 +517,8 @@ int32_t attention_enqueue(sgl_rocm_kv_ctx *ctx, const sgl_kv_attention_plan *pla
         p.partial = static_cast<float *>(workspace ? workspace : r.apart ? ctx->tile_records : ctx->attention_partial);
     if (r.apart) SGLKV_CHECK_HIP(hipStreamWaitEvent(s, ctx->tile_order, 0));
     void *args[] = {&p};
-    hipError_t err = hipModuleLaunchKernel(ctx->attention[r.body], (unsigned)r.grid, p.splits, 1, r.threads, 1, 1, r.lds,
-                                           s, args, nullptr);
+    hipError_t err = hipModuleLaunchKernel(p.compact ? ctx->attention_live[r.body] : ctx->attention[r.body],
+                                           (unsigned)r.grid, p.splits, 1, r.threads, 1, 1, r.lds, s, args, nullptr);
     if (err == hipSuccess && p.splits > 1)
         err = hipModuleLaunchKernel(r.half_records ? ctx->attention_combine_h : ctx->attention_combine,
                                     (unsigned)r.combine_grid, 1, 1, r.combine_threads, 1, 1, 0, s, args, nullptr);

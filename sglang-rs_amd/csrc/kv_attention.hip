@@ -134,12 +134,14 @@ struct attn_work {
 
 // The workgroup's query, split and number among the `inners` workgroups (KV
 // heads, head groups, value blocks) of that split, in a launch of queries *
-// inners (x) by splits (y). False: it has none.
+// inners (x) by splits (y) that numbers its live splits first. False: it has
+// none.
 //
 // Workgroups go round-robin over the 8 XCDs and start in order. In a plain
 // launch a grid row of a multiple of 8 gives one XCD all of a query's splits,
-// so in a ragged batch the XCDs with the longest queries finish last. Compact
-// launches (ragged batches of at most SGLKV_ATTN_COMPACT_QUERIES queries)
+// so in a ragged batch the XCDs with the longest queries finish last. Live
+// launches (ragged batches of at most SGLKV_ATTN_COMPACT_QUERIES queries; the
+// kernels named _live)
 // number the splits that have tokens, every query's first split first: the
 // empty workgroups of the grid come last, every XCD gets the same number of
 // live ones, and the host can size the chunk so that they fill the chip in one
@@ -149,17 +151,13 @@ struct attn_work {
 // different rows; with one query's heads adjacent 64 queries took 119 us at
 // dims 128 and 69 at dims 64, where this takes 115 and 63), the inners first
 // on head-major ones (116 against 119 us).
-// Only the bodies with COMPACT take compact launches (the host's rule).
-template <bool COMPACT>
+// Kernels of their own: with the search compiled into the plain ones and
+// branched around, launches that did not need it took up to 0.6 us longer
+// (traced medians, MI355X: one query over 4,096 tokens, dims 128, 9.8 us, so 9.3;
+// 144 queries of four prompts of 8..68 tokens, dims 64, 8.3 and 7.9).
 __device__ __forceinline__ bool attn_find_place(const sglkv_attn_params &p, uint32_t lane, uint32_t inners,
                                                 uint32_t &q, uint32_t &split, uint32_t &inner) {
     const uint32_t queries = gridDim.x / inners;
-    if (!COMPACT || !p.compact) {
-        q = blockIdx.x % queries;
-        inner = blockIdx.x / queries;
-        split = blockIdx.y;
-        return true;
-    }
     uint32_t n = blockIdx.y * gridDim.x + blockIdx.x;
     constexpr uint32_t U = SGLKV_ATTN_COMPACT_QUERIES / 64;
     const uint32_t chunk = static_cast<uint32_t>(p.chunk_tokens), covered = chunk * p.splits;  // (host: below 2^31)
@@ -239,19 +237,29 @@ __device__ __forceinline__ bool attn_find_place(const sglkv_attn_params &p, uint
     return true;
 }
 
-template <bool COMPACT = false>
+template <bool LIVE = false>
 __device__ __forceinline__ bool attn_decode(const sglkv_attn_params &p, uint32_t lane, attn_work *w) {
     // The KV head varies slowest: with query_count * head_groups * dv_blocks
     // a multiple of 8 every KV head of a (query, split) of a plain launch runs
     // on one XCD, and the slices of one token row meet in one L2 rather than
-    // eight.
-    uint32_t qi, split, inner;
-    if (!attn_find_place<COMPACT>(p, lane, p.kv_heads * p.head_groups * p.dv_blocks, qi, split, inner)) return false;
-    const uint32_t dblk = inner % p.dv_blocks;
-    inner /= p.dv_blocks;
-    const uint32_t hg = inner % p.head_groups;
-    const uint32_t kvh = inner / p.head_groups;
-    const uint64_t q = qi;
+    // eight. (The grid, and so every count here, is below 2^32.)
+    uint32_t q, split = blockIdx.y, dblk, hg, kvh;
+    if (LIVE) {
+        uint32_t inner;
+        if (!attn_find_place(p, lane, p.kv_heads * p.head_groups * p.dv_blocks, q, split, inner)) return false;
+        dblk = inner % p.dv_blocks;
+        inner /= p.dv_blocks;
+        hg = inner % p.head_groups;
+        kvh = inner / p.head_groups;
+    } else {
+        uint32_t bx = blockIdx.x;
+        dblk = bx % p.dv_blocks;
+        bx /= p.dv_blocks;
+        hg = bx % p.head_groups;
+        bx /= p.head_groups;
+        q = bx % static_cast<uint32_t>(p.query_count);
+        kvh = bx / static_cast<uint32_t>(p.query_count);
+    }
 
     uint64_t start = 0, len = 0;
     const bool report = lane == 0 && split == 0 && hg == 0 && dblk == 0 && kvh == 0;
@@ -1076,11 +1084,12 @@ __device__ __forceinline__ void attn_wide_body(const sglkv_attn_params &p) {
     // same rows run on one XCD when query_count * kv_heads is a multiple
     // of 8.
     const uint32_t hblocks = (p.head_groups + G::GROUPS - 1) / G::GROUPS;
-    uint32_t qi, split, inner;
-    if (!attn_find_place<false>(p, lane, p.kv_heads * hblocks, qi, split, inner)) return;
-    const uint64_t q = qi;
-    const uint32_t kvh = inner % p.kv_heads;
-    const uint32_t hb = inner / p.kv_heads;
+    uint64_t bx = blockIdx.x;
+    const uint64_t q = bx % p.query_count;
+    bx /= p.query_count;
+    const uint32_t kvh = static_cast<uint32_t>(bx % p.kv_heads);
+    const uint32_t hb = static_cast<uint32_t>(bx / p.kv_heads);
+    const uint32_t split = blockIdx.y;
     uint64_t start = 0, len = 0;
     if (!attn_metadata(p, q, tid == 0 && split == 0 && hb == 0 && kvh == 0, &start, &len)) return;
     const uint64_t t0 = static_cast<uint64_t>(split) * p.chunk_tokens;
@@ -1597,7 +1606,7 @@ __device__ __forceinline__ void attn_lat_softmax(const sglkv_attn_params &p, con
     l_part += psum;
 }
 
-template <bool EXACT>
+template <bool EXACT, bool LIVE>
 __device__ __forceinline__ void attn_latent_body(const sglkv_attn_params &p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t attn_lat_lds[];
     uint8_t *const k0 = attn_lat_lds, *const k1 = attn_lat_lds + kLatK;
@@ -1610,8 +1619,13 @@ __device__ __forceinline__ void attn_latent_body(const sglkv_attn_params &p) {
 
     // Workgroup -> (query, KV head, block of 128 query heads), split.
     const uint32_t hblocks = (p.group + SGLKV_ATTN_LATENT_HEADS - 1) / SGLKV_ATTN_LATENT_HEADS;
-    uint32_t qi, split, inner;
-    if (!attn_find_place<true>(p, lane, p.kv_heads * hblocks, qi, split, inner)) return;
+    uint32_t qi, split = blockIdx.y, inner;
+    if (LIVE) {
+        if (!attn_find_place(p, lane, p.kv_heads * hblocks, qi, split, inner)) return;
+    } else {
+        qi = blockIdx.x % static_cast<uint32_t>(p.query_count);
+        inner = blockIdx.x / static_cast<uint32_t>(p.query_count);
+    }
     const uint64_t q = qi;
     const uint32_t kvh = inner % p.kv_heads;
     const uint32_t hb = inner / p.kv_heads;
@@ -2014,7 +2028,7 @@ __device__ __forceinline__ void attn_stg_softmax_pv(const sglkv_attn_params &p, 
     }
 }
 
-template <uint32_t D>
+template <uint32_t D, bool LIVE>
 __device__ __forceinline__ void attn_staged_body(const sglkv_attn_params &p) {
     typedef attn_stg<D> S;
     extern __shared__ __attribute__((aligned(16))) uint8_t attn_stg_lds[];
@@ -2022,7 +2036,7 @@ __device__ __forceinline__ void attn_staged_body(const sglkv_attn_params &p) {
     const uint32_t lane = threadIdx.x;
     const uint32_t g = lane >> 4, r = lane & 15;
     attn_work w;
-    if (!attn_decode<true>(p, lane, &w)) return;
+    if (!attn_decode<LIVE>(p, lane, &w)) return;
     const uint32_t nb = static_cast<uint32_t>((w.t1 - w.t0 + kLatB - 1) / kLatB);  // <= SLOTS / 32 (host bound)
 
     // Queries (B operand of q.k): head r, dims 32c + 8g.
@@ -2214,7 +2228,7 @@ __device__ __forceinline__ void attn_kr_block(const sglkv_attn_params &p, uint32
     attn_stg_softmax_pv<D>(p, g, r, sc, nv, vst, st);
 }
 
-template <uint32_t D>
+template <uint32_t D, bool LIVE>
 __device__ __forceinline__ void attn_kreg_body(const sglkv_attn_params &p) {
     typedef attn_stg<D> S;
     typedef attn_kr<D> K;
@@ -2223,7 +2237,7 @@ __device__ __forceinline__ void attn_kreg_body(const sglkv_attn_params &p) {
     const uint32_t lane = threadIdx.x;
     const uint32_t g = lane >> 4, r = lane & 15;
     attn_work w;
-    if (!attn_decode<true>(p, lane, &w)) return;
+    if (!attn_decode<LIVE>(p, lane, &w)) return;
     const uint32_t nb = static_cast<uint32_t>((w.t1 - w.t0 + kLatB - 1) / kLatB);
 
     sglkv_u16x8 qf[S::KC];
@@ -2306,24 +2320,24 @@ extern "C" __global__ __launch_bounds__(512) void sglkv_paged_attention_wide128(
 // between AGPRs and VGPRs every block.
 extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
 sglkv_paged_attention_staged128(sglkv_attn_params p) {
-    attn_staged_body<128>(p);
+    attn_staged_body<128, false>(p);
 }
 
 extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
 sglkv_paged_attention_staged128k(sglkv_attn_params p) {
-    attn_kreg_body<128>(p);
+    attn_kreg_body<128, false>(p);
 }
 
 extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
 sglkv_paged_attention_staged64(sglkv_attn_params p) {
-    attn_staged_body<64>(p);
+    attn_staged_body<64, false>(p);
 }
 
 // Dims 256 (Qwen3.5's full-attention layers): 68 KiB of LDS, two
 // workgroups per CU.
 extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
 sglkv_paged_attention_staged256(sglkv_attn_params p) {
-    attn_staged_body<256>(p);
+    attn_staged_body<256, false>(p);
 }
 
 // MLA latent rows (K <= 576, V <= 512 dims), up to 128 query heads per
@@ -2332,14 +2346,45 @@ extern "C" __global__ __launch_bounds__(256) void sglkv_paged_attention_latent(s
     // Naming an accumulator register keeps the compiler's MFMA accumulators
     // in AGPRs (the 256 of o), leaving the VGPRs to the queries and scores.
     asm volatile("" ::: "a0");
-    attn_latent_body<false>(p);
+    attn_latent_body<false, false>(p);
 }
 
 // The same with each weight fed to p.v as hi + lo bf16 values, as the other
 // bodies always do (SGL_KV_ATTN_EXACT_WEIGHTS).
 extern "C" __global__ __launch_bounds__(256) void sglkv_paged_attention_latent_exact(sglkv_attn_params p) {
     asm volatile("" ::: "a0");
-    attn_latent_body<true>(p);
+    attn_latent_body<true, false>(p);
+}
+
+// The staged and latent bodies for ragged batches (attn_find_place).
+extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
+sglkv_paged_attention_staged128_live(sglkv_attn_params p) {
+    attn_staged_body<128, true>(p);
+}
+
+extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
+sglkv_paged_attention_staged128k_live(sglkv_attn_params p) {
+    attn_kreg_body<128, true>(p);
+}
+
+extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
+sglkv_paged_attention_staged64_live(sglkv_attn_params p) {
+    attn_staged_body<64, true>(p);
+}
+
+extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void
+sglkv_paged_attention_staged256_live(sglkv_attn_params p) {
+    attn_staged_body<256, true>(p);
+}
+
+extern "C" __global__ __launch_bounds__(256) void sglkv_paged_attention_latent_live(sglkv_attn_params p) {
+    asm volatile("" ::: "a0");
+    attn_latent_body<false, true>(p);
+}
+
+extern "C" __global__ __launch_bounds__(256) void sglkv_paged_attention_latent_exact_live(sglkv_attn_params p) {
+    asm volatile("" ::: "a0");
+    attn_latent_body<true, true>(p);
 }
 
 // Head dims exactly 128 (no per-dim masks) / up to 128.

@@ -144,6 +144,7 @@ struct sgl_rocm_kv_ctx {
     // staged (dims 256) / staged (dims 128, K in registers: head-major pages) /
     // tile (several queries per request) dims 128, 64, 256
     hipFunction_t attention[15];
+    hipFunction_t attention_live[15];     // the same for ragged batches, live splits first (staged and latent only)
     hipFunction_t attention_combine;
     hipFunction_t attention_combine_h;    // the latent body's scaled fp16 records
     uint32_t attention_occupancy[15];     // resident workgroups per CU of attention[i] ...

@@ -497,36 +497,30 @@ extern "C" int32_t sgl_rocm_kv_init(int32_t device, const char *code_object_path
         err = hipModuleGetFunction(&ctx->pair_slots[0], ctx->module, "sglkv_write_pair_slots_v16");
     if (err == hipSuccess)
         err = hipModuleGetFunction(&ctx->pair_slots[1], ctx->module, "sglkv_write_pair_slots_v1");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[0], ctx->module, "sglkv_paged_attention_v16");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[1], ctx->module, "sglkv_paged_attention_v2");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[2], ctx->module, "sglkv_paged_attention_pipe128");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[3], ctx->module, "sglkv_paged_attention_pipe");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[4], ctx->module, "sglkv_paged_attention_wide576");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[5], ctx->module, "sglkv_paged_attention_wide128");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[6], ctx->module, "sglkv_paged_attention_latent");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[7], ctx->module, "sglkv_paged_attention_staged128");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[8], ctx->module, "sglkv_paged_attention_staged64");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[9], ctx->module, "sglkv_paged_attention_latent_exact");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[10], ctx->module, "sglkv_paged_attention_staged256");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[11], ctx->module, "sglkv_paged_attention_staged128k");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[12], ctx->module, "sglkv_paged_attention_tile128");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[13], ctx->module, "sglkv_paged_attention_tile64");
-    if (err == hipSuccess)
-        err = hipModuleGetFunction(&ctx->attention[14], ctx->module, "sglkv_paged_attention_tile256");
+    const struct {
+        const char *plain, *live;
+    } attention_names[] = {{"sglkv_paged_attention_v16", nullptr},
+                           {"sglkv_paged_attention_v2", nullptr},
+                           {"sglkv_paged_attention_pipe128", nullptr},
+                           {"sglkv_paged_attention_pipe", nullptr},
+                           {"sglkv_paged_attention_wide576", nullptr},
+                           {"sglkv_paged_attention_wide128", nullptr},
+                           {"sglkv_paged_attention_latent", "sglkv_paged_attention_latent_live"},
+                           {"sglkv_paged_attention_staged128", "sglkv_paged_attention_staged128_live"},
+                           {"sglkv_paged_attention_staged64", "sglkv_paged_attention_staged64_live"},
+                           {"sglkv_paged_attention_latent_exact", "sglkv_paged_attention_latent_exact_live"},
+                           {"sglkv_paged_attention_staged256", "sglkv_paged_attention_staged256_live"},
+                           {"sglkv_paged_attention_staged128k", "sglkv_paged_attention_staged128k_live"},
+                           {"sglkv_paged_attention_tile128", nullptr},
+                           {"sglkv_paged_attention_tile64", nullptr},
+                           {"sglkv_paged_attention_tile256", nullptr}};
+    static_assert(sizeof attention_names / sizeof *attention_names == sizeof ctx->attention / sizeof *ctx->attention,
+                  "one name per body");
+    for (size_t i = 0; i < sizeof attention_names / sizeof *attention_names; ++i) {
+        if (err == hipSuccess) err = hipModuleGetFunction(&ctx->attention[i], ctx->module, attention_names[i].plain);
+        if (err == hipSuccess && attention_names[i].live)
+            err = hipModuleGetFunction(&ctx->attention_live[i], ctx->module, attention_names[i].live);
+    }
     if (err == hipSuccess)
         err = hipDeviceGetAttribute(&ctx->max_lds_per_block, hipDeviceAttributeMaxSharedMemoryPerBlock, device);
     if (err == hipSuccess)
