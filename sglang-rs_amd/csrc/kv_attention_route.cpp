@@ -311,8 +311,10 @@ int32_t split_tiles(const AttentionDevice &device, const sgl_kv_attention_plan_c
     sglkv_attn_params &p = *params;
     p.tile_queries = (uint32_t)shape.queries;
     p.tile_recip = UINT32_MAX / p.tile_queries + 1;
-    // Queries that come request by request make at most this many tiles.
-    const uint64_t most = c.query_count / p.tile_queries + c.request_count;
+    // Queries that come request by request make at most this many tiles (a
+    // request's queries are cut at the steps of the search).
+    const uint64_t most = c.query_count / p.tile_queries + c.request_count +
+                          (c.request_count > 1 ? (c.query_count - 1) / SGLKV_ATTN_TILE_STEP : 0);
     p.tile_slots = (uint32_t)(most < c.query_count ? most : c.query_count);
     // Later tiles of a causal prompt attend more tokens: they start
     // first, except where each request is one tile. (Several prompts'

@@ -11,12 +11,13 @@
 // outputs of 32 rows are too many registers for one wave, 64 rows, 32 per pair
 // of waves: both compute the scores, each has half the value dims). Every K and
 // V row is staged in LDS once per tile.
-//  - Tiles. A run is a maximal stretch of consecutive queries of one request;
-//    it is cut into tiles of tile_queries from its start, and tiles are
+//  - Tiles. A run is a maximal stretch of consecutive queries of one request
+//    within a step of 2,048; it is cut into tiles of tile_queries from its start, and tiles are
 //    numbered over all runs. Which queries tile t holds is found from
 //    query_request_indices by the workgroup itself (attn_tile_find), so queries of different requests never
 //    share a tile whatever their order, and no planning launch or device list
-//    is needed. The host launches tile_slots tiles per KV head, enough for
+//    is needed. Where the queries of a step do not come request by request,
+//    its tiles gather those of a request. The host launches tile_slots tiles per KV head, enough for
 //    queries that come request by request; workgroups step by tile_slots, so
 //    any other order is covered too. Later tiles of a causal prompt attend
 //    more tokens, so the tiles are taken from the last to the first.
@@ -96,19 +97,28 @@ __device__ __forceinline__ const sglkv_attn_params &attn_tile_params() {
     return *(const sglkv_attn_params *)k;
 }
 
-// Queries [q0, q0 + nq) of tile `want`, or false if there are fewer tiles
-// (uniform over the workgroup). `masks`: 256 bytes of LDS; `seen_requests`: 8
-// KiB, the step's request indices, from which the tile's own request and end
-// are read without another memory latency. 2,048 queries a step: each wave
+constexpr uint32_t kTileGathered = 0xFFFFFFFFu;  // q0 of a tile whose queries are listed
+
+// The nq queries of tile `want`, or false if there are fewer tiles (uniform
+// over the workgroup): queries [q0, q0 + nq), or members[0 .. nq) where q0 is
+// kTileGathered. `masks`: 256 bytes of LDS, the list (128 words) behind them;
+// `seen_requests`: 17 KiB, first the step's request indices, from which the
+// tile's own request and end are read without another memory latency.
+// SGLKV_ATTN_TILE_STEP queries a step: each wave
 // ballots where runs start in 8 stretches of 64 queries (its loads all in
 // flight at once: stepping through 128 queries at a time by one wave, each
 // step a memory latency, took most of a short tile's time), then lane l of
 // every wave takes stretch l, counts the tiles that start in it and sums over
-// the lanes.
+// the lanes. A run ends with its step.
+// A step with more runs than there are requests holds queries of one request
+// apart from each other. Its tiles gather the queries of one request wherever
+// they are in the step: with a tile for each run, 200 queries of each of four
+// prompts in turn were 800 tiles of one query and took 495 us (dims 64), so 14.
 __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint32_t want, uint32_t w, uint32_t lane,
                                                uint64_t *masks, uint32_t *seen_requests, uint32_t *q0, uint32_t *nq,
                                                uint32_t *request) {
-    constexpr uint32_t U = 8, STEP = 4 * U * 64;
+    constexpr uint32_t U = 8, STEP = SGLKV_ATTN_TILE_STEP;
+    static_assert(STEP == 4 * U * 64, "a stretch of 64 queries per load");
     const uint32_t count = static_cast<uint32_t>(p.query_count);  // host: at most SGLKV_ATTN_TILE_QUERIES_MAX
     const uint32_t *req = p.query_request_indices;
     // ceil(x / tile_queries) for x up to 2^24 (the host's reciprocal is exact there)
@@ -129,9 +139,8 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
         }
         return tiles;
     };
-    uint32_t seen = 0, run = 0, first = 0, base = 0;
-    bool found = false;
-    for (; base < count; base += STEP) {
+    uint32_t seen = 0;
+    for (uint32_t base = 0; base < count; base += STEP) {
         uint32_t cur[U], before[U];
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
@@ -143,7 +152,7 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
         __syncthreads();  // the table and stage that the masks and indices overlay are no longer read
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
-            const uint64_t starts = __ballot(cur[u] != before[u]) | (base + w + u == 0 ? 1 : 0);
+            const uint64_t starts = __ballot(cur[u] != before[u]) | (w + u == 0 ? 1 : 0);
             seen_requests[64 * (U * w + u) + lane] = cur[u];
             if (lane == 0) masks[U * w + u] = starts;
         }
@@ -151,15 +160,64 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
         const uint64_t starts = lane < 4 * U ? masks[lane] : 0;
         const uint32_t from = base + 64 * lane;
         const uint32_t n = lane >= 4 * U || from >= count ? 0 : (count - from < 64 ? count - from : 64);
+        uint32_t runs = __popcll(starts);
+#pragma unroll
+        for (uint32_t d = 1; d < 32; d <<= 1) runs += __shfl_xor(runs, d);
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(runs) > p.request_count, 0)) {
+            // The step's queries of each request (below 2,048 of them; bad
+            // indices count as one more), the tiles that they make, in the
+            // requests' order, and the tile's own queries in theirs.
+            uint32_t *const counts = seen_requests + STEP, bad = p.request_count;
+            for (uint32_t i = 64 * w + lane; i <= bad; i += 256) counts[i] = 0;
+            __syncthreads();
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u)
+                if (base + 64 * (U * w + u) + lane < count) atomicAdd(&counts[cur[u] < bad ? cur[u] : bad], 1u);
+            __syncthreads();
+            for (uint32_t r0 = 0; r0 <= bad; r0 += 64) {
+                const uint32_t r = r0 + lane, own = r <= bad ? counts[r] : 0, t = tiles_to(own);
+                uint32_t sum = t;
+#pragma unroll
+                for (uint32_t d = 1; d < 64; d <<= 1) {
+                    const uint32_t x = __shfl_up(sum, d);
+                    sum += lane >= d ? x : 0u;
+                }
+                const uint64_t here = __ballot(want - seen < sum);  // (want >= seen)
+                if (here) {
+                    const int l = __builtin_ctzll(here);
+                    const uint32_t skip = (want - seen - __shfl(sum - t, l)) * p.tile_queries;
+                    const uint32_t left = __shfl(own, l) - skip;
+                    uint32_t *const members = reinterpret_cast<uint32_t *>(masks + 4 * U);
+                    uint32_t rank = 0;
+                    // (Every wave writes the whole list.)
+                    for (uint32_t i = lane; base + i - lane < count && i < STEP; i += 64) {
+                        const uint32_t x = seen_requests[i];
+                        const bool is = base + i < count && (x < bad ? x : bad) == r0 + l;
+                        const uint64_t m = __ballot(is);
+                        const uint32_t k = rank - skip +
+                                           __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0));
+                        if (is && k < p.tile_queries) members[k] = base + i;
+                        rank += __popcll(m);
+                    }
+                    *q0 = kTileGathered;
+                    *nq = __builtin_amdgcn_readfirstlane(left < p.tile_queries ? left : p.tile_queries);
+                    *request = r0 + l;
+                    return true;
+                }
+                seen += __builtin_amdgcn_readfirstlane(__shfl(sum, 63));
+            }
+            continue;
+        }
         // Start of the last run at or before the stretch's end: a running
-        // maximum over the lanes (and what came before).
-        uint32_t last = starts ? from + 63 - static_cast<uint32_t>(__builtin_clzll(starts)) : run;
+        // maximum over the lanes.
+        uint32_t last = starts ? from + 63 - static_cast<uint32_t>(__builtin_clzll(starts)) : 0;
 #pragma unroll
         for (uint32_t d = 1; d < 64; d <<= 1) {
             const uint32_t x = __shfl_up(last, d);
             last = lane >= d && x > last ? x : last;
         }
-        const uint32_t x = __shfl_up(last, 1), in = lane ? x : run;
+        const uint32_t in = __shfl_up(last, 1);  // (lane 0's stretch begins with a start)
         uint32_t unused;
         const uint32_t mine = walk(from, n, starts, in, 0xFFFFFFFFu, &unused);
         uint32_t sum = mine;
@@ -169,39 +227,32 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
             sum += lane >= d ? x : 0u;
         }
         const uint64_t here = __ballot(want - seen < sum);  // (want >= seen)
-        if (here) {
-            const int l = __builtin_ctzll(here);
-            const uint32_t k = want - seen - __shfl(sum - mine, l);
-            const uint64_t bits = static_cast<uint64_t>(__shfl(static_cast<uint32_t>(starts >> 32), l)) << 32 |
-                                  __shfl(static_cast<uint32_t>(starts), l);
-            walk(base + 64 * l, __shfl(n, l), bits, __shfl(in, l), k, &first);
-            found = true;
-            break;
+        if (!here) {
+            seen += __shfl(sum, 63);
+            continue;
         }
-        seen += __shfl(sum, 63);
-        run = __shfl(last, 63);
+        const int l = __builtin_ctzll(here);
+        const uint32_t k = want - seen - __shfl(sum - mine, l);
+        const uint64_t bits = static_cast<uint64_t>(__shfl(static_cast<uint32_t>(starts >> 32), l)) << 32 |
+                              __shfl(static_cast<uint32_t>(starts), l);
+        uint32_t first = 0;
+        walk(base + 64 * l, __shfl(n, l), bits, __shfl(in, l), k, &first);
+        first = __builtin_amdgcn_readfirstlane(first);
+        // The tile ends with its run, its step or after tile_queries (at most
+        // 128): how many of the step's queries from `first` on are of its
+        // request.
+        const uint32_t end = count - base < STEP ? count - base : STEP, i = first - base + lane, j = i + 64;
+        const uint32_t ri = seen_requests[i < end ? i : end - 1], rj = seen_requests[j < end ? j : end - 1];
+        const uint32_t own = __builtin_amdgcn_readfirstlane(ri);
+        const uint64_t oi = ~__ballot(i < end && ri == own), oj = ~__ballot(j < end && rj == own);
+        const uint32_t len = oi ? static_cast<uint32_t>(__builtin_ctzll(oi))
+                                : 64 + (oj ? static_cast<uint32_t>(__builtin_ctzll(oj)) : 64u);
+        *q0 = first;
+        *nq = len < p.tile_queries ? len : p.tile_queries;
+        *request = own;
+        return true;
     }
-    if (!found) return false;
-    first = __builtin_amdgcn_readfirstlane(first);
-    // The tile ends with its run or after tile_queries (at most 128): how
-    // many of the queries from `first` on are of its request.
-    const uint32_t i = first + lane, j = i + 64;
-    uint32_t ri, rj;
-    if (first + 128 <= base + STEP) {
-        ri = seen_requests[i - base];
-        rj = seen_requests[j - base];
-    } else {
-        ri = req[i < count ? i : count - 1];
-        rj = req[j < count ? j : count - 1];
-    }
-    const uint32_t own = __builtin_amdgcn_readfirstlane(ri);
-    const uint64_t oi = ~__ballot(i < count && ri == own), oj = ~__ballot(j < count && rj == own);
-    const uint32_t len = oi ? static_cast<uint32_t>(__builtin_ctzll(oi))
-                            : 64 + (oj ? static_cast<uint32_t>(__builtin_ctzll(oj)) : 64u);
-    *q0 = first;
-    *nq = len < p.tile_queries ? len : p.tile_queries;
-    *request = own;
-    return true;
+    return false;
 }
 
 // Four loads: lane l's 16 bytes of load i from a[i] to LDS at at + 1024 i +
@@ -502,16 +553,16 @@ __device__ __forceinline__ void attn_tile_row(const sglkv_attn_params &p, uint32
     *head = row - *query * p.group;
 }
 
-// The row's output (one split), or its split record (rows of the combine
+// The output of the row of query `query` (one split), or its split record (rows of the combine
 // kernel's layout). Lanes l and l + 32 hold the row's dims 8i + 4h .. +3.
 // Plain stores: the two lanes' pieces of a line meet in L2.
 template <uint32_t D>
-__device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint32_t q0, uint32_t kvh, uint32_t split, uint32_t w,
+__device__ __forceinline__ void attn_tile_write(const sglkv_attn_params &p, uint32_t query, uint32_t kvh, uint32_t split, uint32_t w,
                                                 uint32_t lane, const attn_tile_state<D> &st) {
     typedef attn_tl<D> T;
     uint32_t rq, rh;
     attn_tile_row<D>(p, w, lane, &rq, &rh);
-    const uint64_t qrow = (static_cast<uint64_t>(q0) + rq) * p.query_heads + kvh * p.group + rh;
+    const uint64_t qrow = static_cast<uint64_t>(query) * p.query_heads + kvh * p.group + rh;
     const uint32_t part = w % T::SHARE, h = lane >> 5;
     const float l_tot = st.l_part + __shfl_xor(st.l_part, 32);
     if (p.splits == 1) {
@@ -587,11 +638,14 @@ __device__ __forceinline__ void attn_tile_body() {
         // depends on the tile alone is loaded at once (from request 0 and
         // the tile's first query where the lane or the request has none).
         const bool mine = rq < nq;
-        const uint64_t qrow = (static_cast<uint64_t>(q0) + (mine ? rq : 0)) * p.query_heads + kvh * p.group + rh;
+        // (A listed query is read here, before the list's LDS is used again.)
+        const uint32_t member = mine ? rq : 0;
+        const uint32_t query = q0 == kTileGathered ? reinterpret_cast<const uint32_t *>(table)[64 + member] : q0 + member;
+        const uint64_t qrow = static_cast<uint64_t>(query) * p.query_heads + kvh * p.group + rh;
         const uint32_t known = req < p.request_count ? req : 0;
         const uint64_t start = p.request_slot_offsets[known], end = p.request_slot_offsets[known + 1];
-        const uint64_t n = p.query_sequence_lengths[q0 + (mine ? rq : 0)];
-        const uint32_t own_req = p.query_request_indices[q0 + (mine ? rq : 0)];
+        const uint64_t n = p.query_sequence_lengths[query];
+        const uint32_t own_req = p.query_request_indices[query];
         // Queries (B operand of q.k): row l % 32, dims 16c + 8(l/32).
         sglkv_u16x8 qf[T::KC];
 #pragma unroll
@@ -666,12 +720,12 @@ __device__ __forceinline__ void attn_tile_body() {
                 __syncthreads();
                 apart = __builtin_amdgcn_readfirstlane(table[0] | table[1] | table[2] | table[3]) != 0;
                 if (!apart) {
-                    if (own > t0) attn_tile_write<D>(attn_tile_params(), q0, kvh, split, w, lane, st);
+                    if (own > t0) attn_tile_write<D>(attn_tile_params(), query, kvh, split, w, lane, st);
                     break;
                 }
                 longest = 0xFFFFFFFFu;
             } else if (own > t0) {
-                attn_tile_write<D>(attn_tile_params(), q0, kvh, split, w, lane, st);
+                attn_tile_write<D>(attn_tile_params(), query, kvh, split, w, lane, st);
             }
             longest = tile_longest(longest);
             if (t0 >= longest) break;

@@ -307,6 +307,7 @@ static inline sglkv_combine_place sglkv_combine_place_of(uint32_t thread, uint32
 #define SGLKV_ATTN_TILE_BLOCK(d) ((d) > 128u ? 32u : 64u) /* tokens per block */
 #define SGLKV_ATTN_TILE_SLOTS(d) ((d) > 64u ? 4096u : 2048u)
 #define SGLKV_ATTN_TILE_LDS_BYTES(d) (8u * (d) * SGLKV_ATTN_TILE_BLOCK(d) + 4u * SGLKV_ATTN_TILE_SLOTS(d))
+#define SGLKV_ATTN_TILE_STEP 2048u /* queries that the tile search looks at together: no tile crosses a step */
 #define SGLKV_ATTN_TILE_QUERIES_MAX (1u << 24) /* queries the tile search indexes */
 
 typedef struct sglkv_attn_params {

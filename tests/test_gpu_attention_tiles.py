@@ -42,6 +42,31 @@ def _requests(rng, spans, slot_count):
     return qri, qsl, rso, slots
 
 
+class _Call:
+    """Device buffers of one call, for launches into outputs of their own."""
+
+    def __init__(self, c, q, qri, qsl, rso, slots, max_len):
+        self.plan = kv.PagedAttentionPlan.for_layer(c.layout, c.layer, len(qri), len(rso) - 1, len(slots), c.qh,
+                                                    1.0 / math.sqrt(c.dk), kv.HND if c.hnd else kv.NHD)
+        arrays = dict(queries=q, query_request_indices=np.asarray(qri, np.uint32),
+                      query_sequence_lengths=np.asarray(qsl, np.uint64),
+                      request_slot_offsets=np.asarray(rso, np.uint64), sequence_slots=np.asarray(slots, np.uint64))
+        self.bufs = {n: hip.DeviceBuffer.from_array(a) for n, a in arrays.items()}
+        self.bufs["pool"], self.max_len = c.pool, max_len
+
+    def output(self):
+        out = hip.DeviceBuffer(self.plan.output_required_bytes)
+        out.fill(0xFF)
+        return out
+
+    def run(self, k, out, stream=None):
+        k.paged_attention_async(self.plan, max_sequence_length=self.max_len, stream=stream, output=out, **self.bufs)
+
+    def route(self, k):
+        out = self.output()
+        return k.attention_route(self.plan, max_sequence_length=self.max_len, output=out, **self.bufs)
+
+
 @pytest.mark.parametrize("H,qh,d,P,hnd,spans", [
     (2, 8, 128, 16, False, [(0, 1), (0, 2), (0, 31), (0, 32), (0, 33), (0, 63), (0, 64), (0, 65)]),
     (2, 8, 128, 64, True, [(0, 300), (127, 3), (64, 64), (63, 66)]),
@@ -81,6 +106,67 @@ def test_queries_in_any_order(k, d):
     _say(f"tiles in any order, d={d}, {len(qri)} queries")
     got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=900)
     _check(got, want, c)
+
+
+@pytest.mark.parametrize("H,qh,d,spans,shuffle", [
+    (8, 32, 64, [(0, 200)] * 4, False),          # four prompts in turn: gathered tiles of 32
+    (8, 32, 128, [(0, 64)] * 8, False),
+    (1, 8, 128, [(30, 300), (0, 700), (5, 1300), (0, 3)], True),   # over the search's step of 2,048 queries
+    (2, 8, 256, [(1500, 5)] * 24, False),         # drafts, position by position
+    (1, 4, 64, [(600, 40 + i % 7) for i in range(60)], True),
+    (4, 4, 64, [(0, 2500), (0, 90), (0, 20)], False),  # 128 a tile; a step of one request alone
+])
+def test_interleaved_queries(k, H, qh, d, spans, shuffle):
+    """Queries of several requests in turn (query j of every request before
+    query j + 1 of any), or in a random order: every step of the search then
+    has more runs than there are requests, and its tiles gather a request's
+    queries."""
+    rng = np.random.default_rng(d + qh + len(spans))
+    c = _Case(rng, P=16, L=1, H=H, dk=d, dv=d, qh=qh, pages=sum(c + n for c, n in spans) // 16 + 3, layer=0)
+    qri, qsl, rso, slots = _requests(rng, spans, c.layout.slot_count)
+    turn = np.concatenate([np.arange(n) for _, n in spans])
+    order = rng.permutation(len(qri)) if shuffle else np.argsort(turn, kind="stable")
+    qri, qsl = qri[order], qsl[order]
+    q = _bf16_normal(rng, len(qri) * qh * d).reshape(len(qri), qh, d)
+    call = _Call(c, q, qri, qsl, rso, slots, int(qsl.max()))
+    assert call.route(k).body == f"tile{d}"
+    _say(f"tiles of gathered queries H={H} qh={qh} d={d} queries={len(qri)} shuffle={shuffle}")
+    got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=int(qsl.max()))
+    _check(got, want, c)
+
+
+def test_gathered_tiles_report_bad_requests(k):
+    """A bad request index among interleaved queries raises the reference's
+    request bit and leaves every other query's result as it is."""
+    rng = np.random.default_rng(8)
+    c = _Case(rng, P=16, L=1, H=8, dk=64, dv=64, qh=32, pages=60, layer=0)
+    qri, qsl, rso, slots = _requests(rng, [(0, 200)] * 4, c.layout.slot_count)
+    order = np.argsort(np.tile(np.arange(200), 4), kind="stable")
+    qri, qsl = qri[order], qsl[order]
+    q = _bf16_normal(rng, 800 * 32 * 64).reshape(800, 32, 64)
+    outs = []
+    for bad in (False, True):
+        index = qri.copy()
+        if bad:
+            index[[5, 300]] = [4, 1 << 30]
+        call = _Call(c, q, index, qsl, rso, slots, 200)
+        assert call.route(k).body == "tile64"
+        outs.append(call.output())
+        _say(f"tiles of gathered queries, two bad indices: {bad}")
+        call.run(k, outs[-1])
+        if bad:
+            with pytest.raises(kv.KvError) as e:
+                k.check_errors()
+            assert e.value.variant == "DeviceMetadataInvalid" and e.value.fields[0] == 1
+        else:
+            k.check_errors()
+    good, got = (o.download(dtype=np.uint16).reshape(800, 32, 64) for o in outs)
+    keep = np.delete(np.arange(800), [5, 300])
+    # (A tile that loses a query passes the maxima of the others alone, so
+    # last bits may differ: two results within the bound of _check of one value.)
+    a, b = (oracle.bf16_to_f32(x[keep]).astype(np.float64) for x in (good, got))
+    assert (np.abs(a - b) <= 2 * (2.0 ** -8 * np.abs(a) + 5.5 * 2.0 ** -12)).all()
+    assert (got[[5, 300]] == 0xFFFF).all()
 
 
 @pytest.mark.parametrize("bits", [0x7F80, 0xFF80, 0x7FC0])  # inf, -inf, NaN
@@ -133,31 +219,6 @@ def test_bad_slot_is_reported(k):
     with pytest.raises(kv.KvError) as e:
         c.run(k, q, np.zeros(64, int), 100 + np.arange(64), [0, 200], slots, 0.1, max_len=200)
     assert e.value.variant == "DeviceMetadataInvalid" and e.value.fields[0] == 4
-
-
-class _Call:
-    """Device buffers of one call, for launches into outputs of their own."""
-
-    def __init__(self, c, q, qri, qsl, rso, slots, max_len):
-        self.plan = kv.PagedAttentionPlan.for_layer(c.layout, c.layer, len(qri), len(rso) - 1, len(slots), c.qh,
-                                                    1.0 / math.sqrt(c.dk), kv.HND if c.hnd else kv.NHD)
-        arrays = dict(queries=q, query_request_indices=np.asarray(qri, np.uint32),
-                      query_sequence_lengths=np.asarray(qsl, np.uint64),
-                      request_slot_offsets=np.asarray(rso, np.uint64), sequence_slots=np.asarray(slots, np.uint64))
-        self.bufs = {n: hip.DeviceBuffer.from_array(a) for n, a in arrays.items()}
-        self.bufs["pool"], self.max_len = c.pool, max_len
-
-    def output(self):
-        out = hip.DeviceBuffer(self.plan.output_required_bytes)
-        out.fill(0xFF)
-        return out
-
-    def run(self, k, out, stream=None):
-        k.paged_attention_async(self.plan, max_sequence_length=self.max_len, stream=stream, output=out, **self.bufs)
-
-    def route(self, k):
-        out = self.output()
-        return k.attention_route(self.plan, max_sequence_length=self.max_len, output=out, **self.bufs)
 
 
 def _chunk_call(seed, H, qh, d, cached, queries):
