@@ -238,17 +238,21 @@ bool split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint6
     return shortened;
 }
 
-// The tiles of a launch with several queries per request, and whether they
-// are the faster way.
+// The tiles of a launch with several queries per request.
 struct TileShape {
-    uint64_t queries, per_request, live, max_len, dims, mean;
+    uint64_t queries, per_request, slots, live, max_len;
 
     TileShape(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p, uint64_t longest)
         : queries(p.group && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) ? SGLKV_ATTN_TILE_ROWS(p.dk) / p.group : 1),
           // (the queries shared evenly among the requests)
-          per_request(ceil_div(ceil_div(c.query_count, requests(c)), queries)),
-          live(per_request * requests(c) * p.kv_heads), max_len(longest), dims(p.dk),
-          mean(ceil_div(c.sequence_slot_count, requests(c))) {}
+          per_request(ceil_div(ceil_div(c.query_count, requests(c)), queries)), max_len(longest) {
+        // Queries that come request by request make at most this many tiles (a
+        // request's queries are cut at the steps of the search).
+        slots = c.query_count / queries + requests(c) +
+                (requests(c) > 1 ? (c.query_count - 1) / SGLKV_ATTN_TILE_STEP : 0);
+        if (slots > c.query_count) slots = c.query_count;
+        live = per_request * requests(c) * p.kv_heads;
+    }
 
     // Splits that fill `target` resident workgroups: of 256 tokens or more,
     // or of 128 where a request is one tile (few queries, so the records that
@@ -258,34 +262,6 @@ struct TileShape {
     uint64_t splits(uint64_t target) const {
         const uint64_t want = live >= target ? 1 : target / live, least = per_request > 1 ? 256 : 128;
         return want < max_len / least ? want : (max_len >= 2 * least ? max_len / least : 1);
-    }
-
-    // Whether the tiles are estimated to take less time than the staged
-    // bodies, whose work items are one query's. Times in units of 50 ns, from
-    // measurements on MI355X: the staged bodies take about 8 us, 6 more once
-    // they split (and merge: where twice the work items fit the resident slots,
-    // or a sequence is longer than a slot table), and 50 ns for each token that a resident
-    // workgroup's share comes to (100 past 128; half of that at dims 64, whose
-    // workgroups are twice as many); a tile takes about 11 us to its first
-    // block, 5 more if split, and per block 0.8, 1.5 or 1.0 us (dims 64, 128;
-    // 256, whose blocks are half as long) where other tiles of the request
-    // have brought the rows into L2, 2.2 us where it reads them first. Tiles
-    // and staged measured: 64 queries of one prompt (dims 128) 13.9 and 12.0
-    // us, 4 x 64 12.8 and 17.9, 160 15.2 and 19.1, 4 x 160 16 and 51; 4 x 2
-    // queries of up to 1,000 tokens 22 and 15, 20 x 5 30 and 57 (over 8 KV
-    // heads; over one 27 and 18).
-    bool pays(uint64_t cus, uint64_t items) const {
-        const uint64_t lds = 160u * 1024u;
-        const uint64_t staged_slots = cus * (lds / SGLKV_ATTN_STAGED_LDS_BYTES(dims));
-        uint64_t share;  // tokens per resident workgroup
-        if (mul_ovf(items, mean, &share)) return true;
-        share = share / staged_slots / (dims == 64 ? 2 : 1);
-        const bool cuts = (max_len > 64 && items <= staged_slots / 2) || max_len > SGLKV_ATTN_STAGED_SLOTS;
-        const uint64_t staged = 160 + (cuts ? 120 : 0) + share + (share > 128 ? share - 128 : 0);
-        const uint64_t cut = splits(cus * (lds / SGLKV_ATTN_TILE_LDS_BYTES(dims)));
-        const uint64_t blocks = ceil_div(ceil_div(max_len, cut), SGLKV_ATTN_TILE_BLOCK(dims));
-        const uint64_t block = per_request == 1 ? 44 : dims == 64 ? 16 : dims == 128 ? 30 : 20;
-        return 220 + blocks * block + (cut > 1 ? 100 : 0) < staged;
     }
 };
 
@@ -305,17 +281,70 @@ bool tiles_take(const AttentionDevice &device, const sgl_kv_attention_plan_confi
                           SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= device.max_lds;
 }
 
+// Whether the tiles are estimated to take less time than `body`, whose work
+// items are one query's, by a tenth. Both estimates are straight lines through
+// 420 random calls on MI355X (1 to 48 requests: prompts, chunks of prompts
+// over a cached prefix, drafts; 14 shapes of heads), each run both ways; their
+// coefficients are us.
+//  - A per-query body: its start; a merge, if split; each 32-token block of a
+//    workgroup's chain; the blocks that a resident workgroup has beyond its
+//    first chain; each round of work items past the first. Never less than
+//    the rows that all queries read, at 4.9 TB/s (64 x 4 queries over 1,100
+//    tokens, dims 64: 114 us, tiles 52).
+//  - Tiles: their start; with several requests the search, by the runs that a
+//    stretch of 64 queries holds; a merge, if split; each block of a chain; the
+//    blocks beyond it; start and search again for each round past the first.
+//    Never less than each row read once.
+// Queries attend the average request's tokens, less half its queries. Over
+// these calls and 420 others the way chosen takes 0.72 of the per-query
+// bodies' time (geometric mean) and 2 % more than the faster of both; 13 of
+// the 840 take over a tenth longer than one query at a time, at most 28 %. A
+// batch of one prompt and many decodes, which looks like one of drafts, is
+// beyond what the counts tell.
+bool tiles_pay(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p, const TileShape &shape,
+               const Body &body, const Split &single, uint64_t tile_target) {
+    const struct {
+        double start, merge, block, beyond, round;
+    } staged[] = {{8.1, 1.7, 1.05, 1.3, 4.6}, {7.2, 1.4, 1.65, 1.9, 6.5}, {8.7, 3.1, 2.0, 2.8, 9.3}},
+      wide[] = {{7.4, 2.4, 1.35, 1.8, 7.6}, {7.1, 3.3, 1.3, 1.1, 15.2}, {8.8, 2.3, 2.6, 3.8, 8.7}};
+    const struct {
+        double start, search, run, merge, block, beyond;
+    } tile[] = {{4.0, 3.5, 0.33, 4.0, 1.6, 2.5}, {6.0, 2.8, 0.28, 4.0, 2.05, 3.0}, {6.5, 3.3, 0.34, 4.0, 1.5, 3.0}};
+    const int d = p.dk == 64 ? 0 : p.dk == 128 ? 1 : 2;
+    const double per = (double)c.query_count / c.request_count, mean = (double)c.sequence_slot_count / c.request_count,
+                 attended = mean - (mean < per ? mean : per) / 2;
+    auto past = [](double x, double y) { return x > y ? x - y : 0.0; };
+
+    const auto &q = body.which < kAttnStaged128 ? wide[d] : staged[d];
+    const double rounds = (double)single.base / single.target,
+                 chain = (double)(single.chunk < shape.max_len ? single.chunk : shape.max_len) / SGLKV_ATTN_TOKENS;
+    const double row = 2.0 * (p.dk + p.dv) / 4.9e6;  // us to read a token's K and V of one head
+    double alone = q.start + (single.splits > 1 ? q.merge : 0) + q.block * chain +
+                   q.beyond * past(rounds * attended / SGLKV_ATTN_TOKENS, chain) + q.round * past(rounds, 1);
+    alone = alone > single.base * attended * row ? alone : single.base * attended * row;
+
+    const auto &t = tile[d];
+    const double size = SGLKV_ATTN_TILE_BLOCK(p.dk), requests = (double)c.request_count;
+    double runs = c.query_count > 64 ? 64 / per : requests;  // of a stretch
+    runs = runs < 1 ? 1 : runs > requests ? requests : runs;
+    const uint64_t splits = shape.splits(tile_target);
+    const double blocks = (double)ceil_div(ceil_div(shape.max_len, splits), (uint64_t)size);
+    const double start = t.start + (c.request_count > 1 ? t.search + t.run * runs : 0),
+                 tile_rounds = (double)shape.live / tile_target;
+    double tiled = start * (1 + past(tile_rounds, 1)) + (splits > 1 ? t.merge : 0) + t.block * blocks +
+                   t.beyond * past(tile_rounds * attended / size, blocks);
+    const double once = c.sequence_slot_count * (double)p.kv_heads * row;
+    tiled = tiled > once ? tiled : once;
+    return 1.1 * tiled < alone;
+}
+
 // Splits for a launch of tiles.
-int32_t split_tiles(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, const TileShape &shape,
-                    const Body &body, uint64_t max_len, sglkv_attn_params *params, Split *s) {
+int32_t split_tiles(const AttentionDevice &device, const TileShape &shape, const Body &body, uint64_t max_len,
+                    sglkv_attn_params *params, Split *s) {
     sglkv_attn_params &p = *params;
     p.tile_queries = (uint32_t)shape.queries;
     p.tile_recip = UINT32_MAX / p.tile_queries + 1;
-    // Queries that come request by request make at most this many tiles (a
-    // request's queries are cut at the steps of the search).
-    const uint64_t most = c.query_count / p.tile_queries + c.request_count +
-                          (c.request_count > 1 ? (c.query_count - 1) / SGLKV_ATTN_TILE_STEP : 0);
-    p.tile_slots = (uint32_t)(most < c.query_count ? most : c.query_count);
+    p.tile_slots = (uint32_t)shape.slots;
     // Later tiles of a causal prompt attend more tokens: they start
     // first, except where each request is one tile. (Several prompts'
     // last tiles in turn were no faster: 4 of 2,048 tokens 266 us against
@@ -351,24 +380,28 @@ int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_atten
     if (body.which >= kAttnStaged128) p.dv_blocks = 1;
     Split s = {0, 0, 0, 0};
     uint64_t block = SGLKV_ATTN_TOKENS;
-    const TileShape shape(c, p, max_len);
     route->apart = route->shortened = false;
-    if (tiles_take(device, c, p, max_len) &&
-        (body.which < kAttnStaged128 || shape.pays(device.cus, c.query_count * p.kv_heads))) {
-        const Body single = body;
-        body = {p.dk == 128 ? kAttnTile128 : p.dk == 64 ? kAttnTile64 : kAttnTile256, 256,
-                SGLKV_ATTN_TILE_LDS_BYTES(p.dk)};
+    const Body tile = {p.dk == 128 ? kAttnTile128 : p.dk == 64 ? kAttnTile64 : kAttnTile256, 256,
+                       SGLKV_ATTN_TILE_LDS_BYTES(p.dk)};
+    const TileShape shape(c, p, max_len);
+    bool tiles = tiles_take(device, c, p, max_len);
+    int32_t rc = split_queries(device, c, p, body, max_len, &s);
+    if (tiles && rc == SGL_KV_OK) {
+        const uint64_t target = device.resident(device.context, tile.which, tile.threads, tile.lds) * device.cus;
+        if (!target) return SGL_KV_MODULE;
+        tiles = tiles_pay(c, p, shape, body, s, target);
+    }
+    if (tiles) {
+        const bool splits_alone = rc == SGL_KV_OK && s.splits > 1;
+        body = tile;
         block = SGLKV_ATTN_TILE_BLOCK(p.dk);
-        const int32_t rc = split_tiles(device, c, shape, body, max_len, &p, &s);
-        if (rc) return rc;
+        if ((rc = split_tiles(device, shape, body, max_len, &p, &s))) return rc;
         // The calls of a context that split share one buffer, so a caller
         // issues them on one stream. Where the per-query body would not split,
         // the caller need not: those records go to the tiles' own buffer,
         // whose calls the library orders itself, or the tiles stay whole
         // (where there is no such buffer, and under graph capture).
-        Split alone = {0, 0, 0, 0};
-        if (s.splits > 1 && !records.workspace_bytes &&
-            (split_queries(device, c, p, single, max_len, &alone) != SGL_KV_OK || alone.splits == 1)) {
+        if (s.splits > 1 && !records.workspace_bytes && !splits_alone) {
             uint64_t bytes;
             route->apart = records.apart && record_bytes(c, p, false, s.splits, &bytes) &&
                            bytes <= kAttentionTileRecordBytes;
@@ -378,7 +411,6 @@ int32_t sglkv::attention_route(const AttentionDevice &device, const sgl_kv_atten
             }
         }
     } else {
-        const int32_t rc = split_queries(device, c, p, body, max_len, &s);
         if (rc) return rc;
         route->shortened = split_ragged(c, body, max_len, records.shorter, &p, &s);
     }
