@@ -251,7 +251,15 @@ struct TileShape {
         slots = c.query_count / queries + requests(c) +
                 (requests(c) > 1 ? (c.query_count - 1) / SGLKV_ATTN_TILE_STEP : 0);
         if (slots > c.query_count) slots = c.query_count;
+        // Workgroups with tokens: as many as even shares make if the requests
+        // have as many queries each, nearly all where one has most of them (a
+        // prompt among decodes). Half way between, since the host cannot tell:
+        // sized for even shares, the mixed batches of 20 took a second round
+        // and 10 % longer (7 queries a KV head, dims 64: 512 queries of a
+        // prompt and 63 decodes over 2,000 tokens 72.7 us, so 55.4), while
+        // the 50 even ones are as fast (0.95 to 1.11 of it).
         live = per_request * requests(c) * p.kv_heads;
+        if (requests(c) > 1) live = (live + slots * p.kv_heads) / 2;
     }
 
     // Splits that fill `target` resident workgroups: of 256 tokens or more,
