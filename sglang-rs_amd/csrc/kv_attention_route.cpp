@@ -185,7 +185,8 @@ bool record_bytes(const sgl_kv_attention_plan_config &c, const sglkv_attn_params
 // twentieths of the staged bodies'): at least 64 tokens (128 for long
 // sequences, whose merge grows) and at most the equal-length chunk for
 // the latent body, between 192 and 512 for the staged ones, whose larger
-// batches take several rounds anyway (past 32,768 tokens up to the
+// batches take several rounds anyway (where the equal chunk takes one, that;
+// past 32,768 tokens up to the
 // equal-length chunk: 64 splits of the longest are enough, and more only
 // add workgroups without tokens: one of 131,072 tokens among 63 of 1,000
 // 248 us at 512 a split, 181 so; dims 64, one of 65,536, 81 and 67).
@@ -220,8 +221,17 @@ bool split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint6
     const uint64_t room = which == kAttnLatent ? target : target / 20 * 17;
     uint64_t balanced = room > base ? ceil_div(total, room - base) : s->chunk;
     const uint64_t least = which == kAttnLatent ? (max_len > 4096 ? 128 : 64) : (s->chunk < 192 ? s->chunk : 192);
-    const uint64_t most = which == kAttnLatent || max_len > 32768 ? s->chunk : 512;
-    balanced = balanced < least ? least : (balanced > most ? most : balanced);
+    // Workgroups with tokens at a chunk of k, each sequence's last one half full.
+    auto live = [&](uint64_t k) { return mean < k / 2 ? base : base * (mean + k / 2) / k; };
+    // Shorter than 512 helps no more where that takes a second round and the
+    // equal chunk does not: 57 queries of 650 or 6,566 tokens (dims 256) 84.7 us a
+    // layer at 512, 74.9 at 1,024; 42 of up to 14,923 90.4 and 75.7; 84 of up to
+    // 5,813 (dims 128, head-major) 155.7 and 147.2. (Just past one round 512 is
+    // still the better: 238 of 126 or 1,262 98 and 113.)
+    const bool capped = which != kAttnLatent && max_len <= 32768;
+    const bool second = capped && live(512) > target + target / 4 && live(s->chunk) <= target;
+    const uint64_t most = capped && !second ? 512 : s->chunk;
+    balanced = second ? most : balanced < least ? least : (balanced > most ? most : balanced);
     uint64_t bytes;
     if (!record_bytes(c, p, which == kAttnLatent, 1, &bytes)) return false;
     const uint64_t fit = ceil_div(max_len, shorter / bytes ? shorter / bytes : 1);
