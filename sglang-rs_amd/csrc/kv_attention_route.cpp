@@ -250,17 +250,28 @@ bool split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint6
 
 // The tiles of a launch with several queries per request.
 struct TileShape {
-    uint64_t queries, per_request, slots, live, max_len;
+    uint64_t queries, per_request, slots, step_slots, live, max_len;
 
     TileShape(const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p, uint64_t longest)
         : queries(p.group && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) ? SGLKV_ATTN_TILE_ROWS(p.dk) / p.group : 1),
           // (the queries shared evenly among the requests)
           per_request(ceil_div(ceil_div(c.query_count, requests(c)), queries)), max_len(longest) {
-        // Queries that come request by request make at most this many tiles (a
-        // request's queries are cut at the steps of the search).
-        slots = c.query_count / queries + requests(c) +
-                (requests(c) > 1 ? (c.query_count - 1) / SGLKV_ATTN_TILE_STEP : 0);
-        if (slots > c.query_count) slots = c.query_count;
+        // Queries that come request by request make at most this many tiles. Past
+        // one step of the search each step has its workgroups, for its share
+        // of the requests.
+        step_slots = 0;
+        const uint64_t steps = (c.query_count - 1) / SGLKV_ATTN_TILE_STEP + 1;
+        auto most = [&](uint64_t count, uint64_t runs) {
+            const uint64_t n = count / queries + runs;
+            return n < count ? n : count;
+        };
+        if (requests(c) == 1 || steps == 1) {
+            slots = most(c.query_count, requests(c));
+        } else {
+            const uint64_t runs = ceil_div(requests(c), steps) + 1;
+            step_slots = most(SGLKV_ATTN_TILE_STEP, runs);
+            slots = (steps - 1) * step_slots + most(c.query_count - (steps - 1) * SGLKV_ATTN_TILE_STEP, runs);
+        }
         // Workgroups with tokens: as many as even shares make if the requests
         // have as many queries each, nearly all where one has most of them (a
         // prompt among decodes). Half way between, since the host cannot tell:
@@ -363,6 +374,7 @@ int32_t split_tiles(const AttentionDevice &device, const TileShape &shape, const
     p.tile_queries = (uint32_t)shape.queries;
     p.tile_recip = UINT32_MAX / p.tile_queries + 1;
     p.tile_slots = (uint32_t)shape.slots;
+    p.tile_step_slots = (uint32_t)shape.step_slots;
     // Later tiles of a causal prompt attend more tokens: they start
     // first, except where each request is one tile. (Several prompts'
     // last tiles in turn were no faster: 4 of 2,048 tokens 266 us against

@@ -106,13 +106,16 @@ constexpr uint32_t kTileWalk = 6;
 
 constexpr uint32_t kTileGathered = 0xFFFFFFFFu;  // q0 of a tile whose queries are listed
 
-// The nq queries of tile `want`, or false if there are fewer tiles (uniform
-// over the workgroup): queries [q0, q0 + nq), or members[0 .. nq) where q0 is
+// The nq queries of tile `want` of the step of queries from `base` on, or false
+// if it has fewer tiles (uniform over the workgroup): queries [q0, q0 + nq), or members[0 .. nq) where q0 is
 // kTileGathered. `masks`: 512 bytes of LDS, the list (128 words) behind the
 // first 256;
 // `seen_requests`: 17 KiB, first the step's request indices, from which the
 // tile's own request and end are read without another memory latency.
-// SGLKV_ATTN_TILE_STEP queries a step: each wave
+// SGLKV_ATTN_TILE_STEP queries a step, whose tiles are numbered by themselves (numbered
+// over all steps, each workgroup looked through those before its own: 1,024
+// queries of each of 128 prompts, 7 a KV head of dims 64, 3,310 us, so 574; 200
+// of each of 5,000 190 ms, so 2.2): each wave
 // ballots where runs start in 8 stretches of 64 queries (its loads all in
 // flight at once: stepping through 128 queries at a time by one wave, each
 // step a memory latency, took most of a short tile's time), then lane l of
@@ -122,9 +125,10 @@ constexpr uint32_t kTileGathered = 0xFFFFFFFFu;  // q0 of a tile whose queries a
 // apart from each other. Its tiles gather the queries of one request wherever
 // they are in the step: with a tile for each run, 200 queries of each of four
 // prompts in turn were 800 tiles of one query and took 495 us (dims 64), so 14.
-__device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint32_t want, uint32_t w, uint32_t lane,
-                                               uint64_t *masks, uint32_t *seen_requests, uint32_t *q0, uint32_t *nq,
+__device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint32_t base, uint32_t want, uint32_t w,
+                                               uint32_t lane, uint64_t *masks, uint32_t *seen_requests, uint32_t *q0, uint32_t *nq,
                                                uint32_t *request) {
+    asm volatile("" : "+v"(lane));  // (what it computes from the lane is not held across tiles)
     constexpr uint32_t U = 8, STEP = SGLKV_ATTN_TILE_STEP;
     static_assert(STEP == 4 * U * 64, "a stretch of 64 queries per load");
     const uint32_t count = static_cast<uint32_t>(p.query_count);  // host: at most SGLKV_ATTN_TILE_QUERIES_MAX
@@ -147,150 +151,144 @@ __device__ __forceinline__ bool attn_tile_find(const sglkv_attn_params &p, uint3
         }
         return tiles;
     };
-    uint32_t seen = 0;
-    for (uint32_t base = 0; base < count; base += STEP) {
-        uint32_t cur[U], before[U];
+    uint32_t cur[U], before[U];
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
-            // (Past the last query both are that query: no start.)
-            const uint32_t i = base + 64 * (U * w + u) + lane, at = i < count ? i : count;
-            cur[u] = req[i < count - 1 ? i : count - 1];
-            before[u] = req[(at > 1 ? at : 1) - 1];
+    for (uint32_t u = 0; u < U; ++u) {
+        // (Past the last query both are that query: no start.)
+        const uint32_t i = base + 64 * (U * w + u) + lane, at = i < count ? i : count;
+        cur[u] = req[i < count - 1 ? i : count - 1];
+        before[u] = req[(at > 1 ? at : 1) - 1];
+    }
+    __syncthreads();  // the table and stage that the masks and indices overlay are no longer read
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+        const uint64_t starts = __ballot(cur[u] != before[u]) | (w + u == 0 ? 1 : 0);
+        seen_requests[64 * (U * w + u) + lane] = cur[u];
+        if (lane == 0) masks[U * w + u] = starts;
+    }
+    __syncthreads();
+    const uint64_t starts = lane < 4 * U ? masks[lane] : 0;
+    const uint32_t from = base + 64 * lane;
+    uint32_t runs = __popcll(starts);
+#pragma unroll
+    for (uint32_t d = 1; d < 32; d <<= 1) runs += __shfl_xor(runs, d);
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(runs) > p.request_count, 0)) {
+        // The step's queries of each request (below 2,048 of them; bad
+        // indices count as one more), the tiles that they make, in the
+        // requests' order, and the tile's own queries in theirs.
+        uint32_t *const counts = seen_requests + STEP, bad = p.request_count;
+        for (uint32_t i = 64 * w + lane; i <= bad; i += 256) counts[i] = 0;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (base + 64 * (U * w + u) + lane < count) atomicAdd(&counts[cur[u] < bad ? cur[u] : bad], 1u);
+        __syncthreads();
+        uint32_t seen = 0;
+        for (uint32_t r0 = 0; r0 <= bad; r0 += 64) {
+            const uint32_t r = r0 + lane, own = r <= bad ? counts[r] : 0, t = tiles_to(own);
+            uint32_t sum = t;
+#pragma unroll
+            for (uint32_t d = 1; d < 64; d <<= 1) {
+                const uint32_t x = __shfl_up(sum, d);
+                sum += lane >= d ? x : 0u;
+            }
+            const uint64_t here = __ballot(want - seen < sum);  // (want >= seen)
+            if (here) {
+                const int l = __builtin_ctzll(here);
+                const uint32_t skip = (want - seen - __shfl(sum - t, l)) * p.tile_queries;
+                const uint32_t left = __shfl(own, l) - skip;
+                uint32_t *const members = reinterpret_cast<uint32_t *>(masks + 4 * U);
+                uint32_t rank = 0;
+                // (Every wave writes the whole list.)
+                for (uint32_t i = lane; base + i - lane < count && i < STEP; i += 64) {
+                    const uint32_t x = seen_requests[i];
+                    const bool is = base + i < count && (x < bad ? x : bad) == r0 + l;
+                    const uint64_t m = __ballot(is);
+                    const uint32_t k = rank - skip +
+                                       __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0));
+                    if (is && k < p.tile_queries) members[k] = base + i;
+                    rank += __popcll(m);
+                }
+                *q0 = kTileGathered;
+                *nq = __builtin_amdgcn_readfirstlane(left < p.tile_queries ? left : p.tile_queries);
+                *request = r0 + l;
+                return true;
+            }
+            seen += __builtin_amdgcn_readfirstlane(__shfl(sum, 63));
         }
-        __syncthreads();  // the table and stage that the masks and indices overlay are no longer read
+        return false;
+    }
+    // Start of the last run at or before the stretch's end: a running
+    // maximum over the lanes.
+    uint32_t last = starts ? from + 63 - static_cast<uint32_t>(__builtin_clzll(starts)) : 0;
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
-            const uint64_t starts = __ballot(cur[u] != before[u]) | (w + u == 0 ? 1 : 0);
-            seen_requests[64 * (U * w + u) + lane] = cur[u];
-            if (lane == 0) masks[U * w + u] = starts;
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+        const uint32_t x = __shfl_up(last, d);
+        last = lane >= d && x > last ? x : last;
+    }
+    const uint32_t in = __shfl_up(last, 1);  // (lane 0's stretch begins with a start)
+    const uint32_t n = lane >= 4 * U || from >= count ? 0 : (count - from < 64 ? count - from : 64);
+    // Few runs a stretch (prompts, chunks): lane l walks the runs of
+    // stretch l. Many (drafts, decodes): all 64 queries of a stretch at
+    // once, a tile starting at each multiple of tile_queries from its
+    // run's start; wave w takes stretches w, w + 4, ....
+    const bool dense = __ballot(__popcll(starts) > kTileWalk) != 0;
+    uint64_t tiles = 0;
+    uint32_t mine, unused;
+    if (dense) {
+        for (uint32_t x = w; x < 4 * U && base + 64 * x < count; x += 4) {
+            const uint32_t i = base + 64 * x + lane;
+            const uint32_t high = __builtin_amdgcn_readlane(static_cast<uint32_t>(starts >> 32), x),
+                           low = __builtin_amdgcn_readlane(static_cast<uint32_t>(starts), x);  // (readlane is signed)
+            const uint64_t m = static_cast<uint64_t>(high) << 32 | low;
+            const uint32_t carried = __builtin_amdgcn_readlane(in, x);
+            const uint64_t upto = m & ((2ull << lane) - 1);
+            const uint32_t run = upto ? base + 64 * x + 63 - static_cast<uint32_t>(__builtin_clzll(upto)) : carried;
+            const uint64_t t = __ballot(i < count && tiles_to(i - run) * p.tile_queries == i - run);
+            if (lane == 0) masks[4 * U + x] = t;
         }
         __syncthreads();
-        const uint64_t starts = lane < 4 * U ? masks[lane] : 0;
-        const uint32_t from = base + 64 * lane;
-        uint32_t runs = __popcll(starts);
-#pragma unroll
-        for (uint32_t d = 1; d < 32; d <<= 1) runs += __shfl_xor(runs, d);
-        if (__builtin_expect(__builtin_amdgcn_readfirstlane(runs) > p.request_count, 0)) {
-            // The step's queries of each request (below 2,048 of them; bad
-            // indices count as one more), the tiles that they make, in the
-            // requests' order, and the tile's own queries in theirs.
-            uint32_t *const counts = seen_requests + STEP, bad = p.request_count;
-            for (uint32_t i = 64 * w + lane; i <= bad; i += 256) counts[i] = 0;
-            __syncthreads();
-#pragma unroll
-            for (uint32_t u = 0; u < U; ++u)
-                if (base + 64 * (U * w + u) + lane < count) atomicAdd(&counts[cur[u] < bad ? cur[u] : bad], 1u);
-            __syncthreads();
-            for (uint32_t r0 = 0; r0 <= bad; r0 += 64) {
-                const uint32_t r = r0 + lane, own = r <= bad ? counts[r] : 0, t = tiles_to(own);
-                uint32_t sum = t;
-#pragma unroll
-                for (uint32_t d = 1; d < 64; d <<= 1) {
-                    const uint32_t x = __shfl_up(sum, d);
-                    sum += lane >= d ? x : 0u;
-                }
-                const uint64_t here = __ballot(want - seen < sum);  // (want >= seen)
-                if (here) {
-                    const int l = __builtin_ctzll(here);
-                    const uint32_t skip = (want - seen - __shfl(sum - t, l)) * p.tile_queries;
-                    const uint32_t left = __shfl(own, l) - skip;
-                    uint32_t *const members = reinterpret_cast<uint32_t *>(masks + 4 * U);
-                    uint32_t rank = 0;
-                    // (Every wave writes the whole list.)
-                    for (uint32_t i = lane; base + i - lane < count && i < STEP; i += 64) {
-                        const uint32_t x = seen_requests[i];
-                        const bool is = base + i < count && (x < bad ? x : bad) == r0 + l;
-                        const uint64_t m = __ballot(is);
-                        const uint32_t k = rank - skip +
-                                           __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0));
-                        if (is && k < p.tile_queries) members[k] = base + i;
-                        rank += __popcll(m);
-                    }
-                    *q0 = kTileGathered;
-                    *nq = __builtin_amdgcn_readfirstlane(left < p.tile_queries ? left : p.tile_queries);
-                    *request = r0 + l;
-                    return true;
-                }
-                seen += __builtin_amdgcn_readfirstlane(__shfl(sum, 63));
-            }
-            continue;
-        }
-        // Start of the last run at or before the stretch's end: a running
-        // maximum over the lanes.
-        uint32_t last = starts ? from + 63 - static_cast<uint32_t>(__builtin_clzll(starts)) : 0;
-#pragma unroll
-        for (uint32_t d = 1; d < 64; d <<= 1) {
-            const uint32_t x = __shfl_up(last, d);
-            last = lane >= d && x > last ? x : last;
-        }
-        const uint32_t in = __shfl_up(last, 1);  // (lane 0's stretch begins with a start)
-        const uint32_t n = lane >= 4 * U || from >= count ? 0 : (count - from < 64 ? count - from : 64);
-        // Few runs a stretch (prompts, chunks): lane l walks the runs of
-        // stretch l. Many (drafts, decodes): all 64 queries of a stretch at
-        // once, a tile starting at each multiple of tile_queries from its
-        // run's start; wave w takes stretches w, w + 4, ....
-        const bool dense = __ballot(__popcll(starts) > kTileWalk) != 0;
-        uint64_t tiles = 0;
-        uint32_t mine, unused;
-        if (dense) {
-            for (uint32_t x = w; x < 4 * U && base + 64 * x < count; x += 4) {
-                const uint32_t i = base + 64 * x + lane;
-                const uint32_t high = __builtin_amdgcn_readlane(static_cast<uint32_t>(starts >> 32), x),
-                               low = __builtin_amdgcn_readlane(static_cast<uint32_t>(starts), x);  // (readlane is signed)
-                const uint64_t m = static_cast<uint64_t>(high) << 32 | low;
-                const uint32_t carried = __builtin_amdgcn_readlane(in, x);
-                const uint64_t upto = m & ((2ull << lane) - 1);
-                const uint32_t run = upto ? base + 64 * x + 63 - static_cast<uint32_t>(__builtin_clzll(upto)) : carried;
-                const uint64_t t = __ballot(i < count && tiles_to(i - run) * p.tile_queries == i - run);
-                if (lane == 0) masks[4 * U + x] = t;
-            }
-            __syncthreads();
-            tiles = n ? masks[4 * U + lane] : 0;
-            mine = __popcll(tiles);
-        } else {
-            mine = walk(from, n, starts, in, 0xFFFFFFFFu, &unused);
-        }
-        uint32_t sum = mine;
-#pragma unroll
-        for (uint32_t d = 1; d < 64; d <<= 1) {
-            const uint32_t x = __shfl_up(sum, d);
-            sum += lane >= d ? x : 0u;
-        }
-        const uint64_t here = __ballot(want - seen < sum);  // (want >= seen)
-        if (!here) {
-            seen += __shfl(sum, 63);
-            continue;
-        }
-        const int l = __builtin_ctzll(here);
-        const uint32_t k = want - seen - __shfl(sum - mine, l);
-        const uint64_t from_l = dense ? tiles : starts;
-        const uint64_t bits = static_cast<uint64_t>(__shfl(static_cast<uint32_t>(from_l >> 32), l)) << 32 |
-                              __shfl(static_cast<uint32_t>(from_l), l);
-        uint32_t first = 0;
-        if (dense) {
-            const uint32_t below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(bits >> 32),
-                                                             __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bits), 0));
-            first = base + 64 * l + __builtin_ctzll(__ballot(below == k && ((bits >> lane) & 1)));
-        } else {
-            walk(base + 64 * l, __shfl(n, l), bits, __shfl(in, l), k, &first);
-        }
-        first = __builtin_amdgcn_readfirstlane(first);
-        // The tile ends with its run, its step or after tile_queries (at most
-        // 128): how many of the step's queries from `first` on are of its
-        // request.
-        const uint32_t end = count - base < STEP ? count - base : STEP, i = first - base + lane, j = i + 64;
-        const uint32_t ri = seen_requests[i < end ? i : end - 1], rj = seen_requests[j < end ? j : end - 1];
-        const uint32_t own = __builtin_amdgcn_readfirstlane(ri);
-        const uint64_t oi = ~__ballot(i < end && ri == own), oj = ~__ballot(j < end && rj == own);
-        const uint32_t len = oi ? static_cast<uint32_t>(__builtin_ctzll(oi))
-                                : 64 + (oj ? static_cast<uint32_t>(__builtin_ctzll(oj)) : 64u);
-        *q0 = first;
-        *nq = len < p.tile_queries ? len : p.tile_queries;
-        *request = own;
-        return true;
+        tiles = n ? masks[4 * U + lane] : 0;
+        mine = __popcll(tiles);
+    } else {
+        mine = walk(from, n, starts, in, 0xFFFFFFFFu, &unused);
     }
-    return false;
+    uint32_t sum = mine;
+#pragma unroll
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+        const uint32_t x = __shfl_up(sum, d);
+        sum += lane >= d ? x : 0u;
+    }
+    const uint64_t here = __ballot(want < sum);
+    if (!here) return false;
+    const int l = __builtin_ctzll(here);
+    const uint32_t k = want - __shfl(sum - mine, l);
+    const uint64_t from_l = dense ? tiles : starts;
+    const uint64_t bits = static_cast<uint64_t>(__shfl(static_cast<uint32_t>(from_l >> 32), l)) << 32 |
+                          __shfl(static_cast<uint32_t>(from_l), l);
+    uint32_t first = 0;
+    if (dense) {
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(bits >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bits), 0));
+        first = base + 64 * l + __builtin_ctzll(__ballot(below == k && ((bits >> lane) & 1)));
+    } else {
+        walk(base + 64 * l, __shfl(n, l), bits, __shfl(in, l), k, &first);
+    }
+    first = __builtin_amdgcn_readfirstlane(first);
+    // The tile ends with its run, its step or after tile_queries (at most
+    // 128): how many of the step's queries from `first` on are of its
+    // request.
+    const uint32_t end = count - base < STEP ? count - base : STEP, i = first - base + lane, j = i + 64;
+    const uint32_t ri = seen_requests[i < end ? i : end - 1], rj = seen_requests[j < end ? j : end - 1];
+    const uint32_t own = __builtin_amdgcn_readfirstlane(ri);
+    const uint64_t oi = ~__ballot(i < end && ri == own), oj = ~__ballot(j < end && rj == own);
+    const uint32_t len = oi ? static_cast<uint32_t>(__builtin_ctzll(oi))
+                            : 64 + (oj ? static_cast<uint32_t>(__builtin_ctzll(oj)) : 64u);
+    *q0 = first;
+    *nq = len < p.tile_queries ? len : p.tile_queries;
+    *request = own;
+    return true;
 }
 
 // Four loads: lane l's 16 bytes of load i from a[i] to LDS at at + 1024 i +
@@ -656,19 +654,27 @@ __device__ __forceinline__ void attn_tile_body() {
     // of any other index is refused row by row): no search. Otherwise the
     // tiles of each request's run.
     const uint32_t count = static_cast<uint32_t>(p.query_count);
-    auto find = [&](uint32_t tile, uint32_t *q0, uint32_t *nq, uint32_t *req) {
+    auto find = [&](uint32_t base, uint32_t tile, uint32_t *q0, uint32_t *nq, uint32_t *req) {
         const sglkv_attn_params &p = attn_tile_params();
         if (p.request_count > 1)
-            return attn_tile_find(p, tile, w, lane, reinterpret_cast<uint64_t *>(table),
+            return attn_tile_find(p, base, tile, w, lane, reinterpret_cast<uint64_t *>(table),
                                   reinterpret_cast<uint32_t *>(attn_tile_lds), q0, nq, req);
         *q0 = tile * p.tile_queries;
         *nq = *q0 < count && count - *q0 < p.tile_queries ? count - *q0 : p.tile_queries;
         *req = 0;
         return *q0 < count;
     };
-    uint32_t q0, nq, req;
-    for (uint32_t tile = attn_tile_order(p, blockIdx.x / p.kv_heads); find(tile, &q0, &nq, &req);
-         tile += p.tile_slots) {
+    // The workgroup's step (the first ones have tile_step_slots workgroups each,
+    // the last one the rest) and its tiles there.
+    uint32_t q0, nq, req, tile = attn_tile_order(p, blockIdx.x / p.kv_heads), base = 0, stride = p.tile_slots;
+    if (p.tile_step_slots) {
+        const uint32_t last = (count - 1) / SGLKV_ATTN_TILE_STEP,
+                       own = __builtin_amdgcn_readfirstlane(tile / p.tile_step_slots), step = own < last ? own : last;
+        tile -= step * p.tile_step_slots;
+        stride = step < last ? p.tile_step_slots : p.tile_slots - last * p.tile_step_slots;
+        base = step * SGLKV_ATTN_TILE_STEP;
+    }
+    for (; find(base, tile, &q0, &nq, &req); tile += stride) {
         const sglkv_attn_params &p = attn_tile_params();
         uint32_t rq, rh;
         attn_tile_row<D>(p, w, lane, &rq, &rh);

@@ -349,7 +349,7 @@ typedef struct sglkv_attn_params {
     uint32_t tile_slots;                  /* workgroups per KV head and split */
     uint32_t tile_backward;               /* they take the tiles from the last to the first */
     uint32_t tile_fold;                   /* past this many, from the other end (0: never) */
-    uint32_t reserved2;
+    uint32_t tile_step_slots;             /* workgroups of a step of queries but the last (0: one step) */
 } sglkv_attn_params;
 
 /* Both tensors of one layer for `count` slots in one launch (key and value
