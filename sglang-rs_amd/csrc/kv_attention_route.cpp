@@ -226,10 +226,11 @@ bool split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint6
     // Shorter than 512 helps no more where that takes a second round and the
     // equal chunk does not: 57 queries of 650 or 6,566 tokens (dims 256) 84.7 us a
     // layer at 512, 74.9 at 1,024; 42 of up to 14,923 90.4 and 75.7; 84 of up to
-    // 5,813 (dims 128, head-major) 155.7 and 147.2. (Just past one round 512 is
-    // still the better: 238 of 126 or 1,262 98 and 113.)
+    // 5,813 (dims 128, head-major) 155.7 and 147.2; 54 of up to 3,838 spread evenly
+    // (dims 256) 78.1 and 69.7. (Just past one round batches of two lengths would
+    // still gain, 238 of 126 or 1,262 tokens 98 and 113, of 118 without numbers.)
     const bool capped = which != kAttnLatent && max_len <= 32768;
-    const bool second = capped && live(512) > target + target / 4 && live(s->chunk) <= target;
+    const bool second = capped && live(512) > target && live(s->chunk) <= target;
     const uint64_t most = capped && !second ? 512 : s->chunk;
     balanced = second ? most : balanced < least ? least : (balanced > most ? most : balanced);
     uint64_t bytes;
