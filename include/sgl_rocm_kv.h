@@ -20,7 +20,10 @@
  *    variant's fields. No exception, panic or abort crosses the ABI.
  *  - All buffers are borrowed: the caller owns every device allocation and
  *    passes plain device pointers with their byte lengths. The context owns
- *    only the loaded module and a 4-byte device error flag.
+ *    the loaded module, a small device block of error words, 192 bytes of
+ *    pinned host words that synchronous calls and check_errors report
+ *    through, and, once attention calls split sequences, their record
+ *    buffers (sgl_rocm_kv_paged_attention).
  *  - Streams are explicit (hipStream_t passed as void*; NULL is the null
  *    stream). The pair scatter/gather drop-ins synchronise the stream and
  *    read the error flag like the reference; the per-layer transfer calls are

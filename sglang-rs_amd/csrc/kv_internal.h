@@ -56,7 +56,7 @@ struct Launch {
 };
 
 // Replaces the device error word a validated launch raises (default: the
-// context's copy word).
+// context's copy word), or has it raise a pinned host word instead.
 inline void set_launch_flag(Launch &l, uint32_t *flag, uint32_t *host_flag = nullptr) {
     l.params.flag = flag;
     l.realign.flag = flag;
@@ -156,11 +156,11 @@ struct sgl_rocm_kv_ctx {
     // consumer's read-and-clear never takes another's bits.
     uint32_t *flag;                 // asynchronous copies, span resolution, page requests
     uint32_t *attn_flag;            // asynchronous paged attention
-    uint32_t *pair_flag;            // the synchronous pair scatter/gather drop-ins
     uint32_t *sync_attn_flag;       // the synchronous paged attention
     // Pinned host words that the device writes (separate lines), so that a
     // synchronous call reads its result after the stream's wait instead of
-    // through a blocking copy: a bad slot of the pair scatter/gather, and two
+    // through a blocking copy: a bad slot of the pair scatter/gather (their
+    // only error word), and two
     // words each that sglkv_take_flags hands check_errors and the synchronous
     // attention.
     uint32_t *host_words;

@@ -135,11 +135,12 @@ __device__ __forceinline__ void sglkv_pool_row(const sglkv_side &s, uint32_t row
                                                uint32_t *host_flag, uint64_t *off0, uint64_t *off1) {
     const uint64_t slot = s.slots[row];
     if (slot >= s.slot_count) {
-        atomicOr(flag, SGLKV_FLAG_SLOT);
-        // (A plain store: the only bit that a copy raises, and an atomic on
-        // host memory would need the host link's support.)
+        // (A plain store to the host word: the only bit that a copy raises, and
+        // an atomic on host memory would need the host link's support.)
         if (host_flag)
             __hip_atomic_store(host_flag, SGLKV_FLAG_SLOT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        else
+            atomicOr(flag, SGLKV_FLAG_SLOT);
         *off0 = *off1 = SGLKV_INVALID_OFFSET;
         return;
     }

@@ -83,7 +83,7 @@ typedef struct sglkv_copy_params {
     sglkv_side src;
     sglkv_side dst;
     uint32_t *flag;         /* device error word (OR of SGLKV_FLAG_*) */
-    uint32_t *host_flag;    /* or null: a bad slot sets this host word too */
+    uint32_t *host_flag;    /* a bad slot sets this host word instead (null: `flag`) */
     float *scale_src;       /* optional per-layer scales copied bit-exactly; layer y's */
     float *scale_dst;       /* scale_count floats follow layer y - 1's */
     uint32_t scale_count;   /* floats to copy per layer (0: none) */

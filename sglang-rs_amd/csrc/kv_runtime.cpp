@@ -430,11 +430,10 @@ int32_t pair_copy(sgl_rocm_kv_ctx *ctx, const sgl_kv_pair_copy_plan *plan,
     // These drop-ins own an error word, as the reference's kernels object
     // owns its flag (cuda_kv_kernels.rs:421, 550-551): clearing and reading
     // it never touches the bits of the asynchronous calls.
-    // The word is a pinned host one (the kernel also raises the device word,
-    // which nobody reads): with a memset before the launch and a blocking
-    // 4-byte copy after the wait, a call of 64 rows took 28.7 us, against
-    // 15.1 us (from Python, all told).
-    set_launch_flag(l, ctx->pair_flag, ctx->host_pair());
+    // The word is a pinned host one: with a device word, a memset before the
+    // launch and a blocking 4-byte copy after the wait, a call of 64 rows took
+    // 28.7 us, against 15.1 us (from Python, all told).
+    set_launch_flag(l, nullptr, ctx->host_pair());
 
     __atomic_store_n(ctx->host_pair(), 0u, __ATOMIC_RELEASE);
     if ((rc = submit_launch(ctx, l, stream))) return rc;
@@ -542,8 +541,8 @@ extern "C" int32_t sgl_rocm_kv_init(int32_t device, const char *code_object_path
     if (err == hipSuccess && (ctx->rows_per_thread == 0 || ctx->rows_per_thread > ctx->max_tile_rows ||
                               ctx->realign_rows_per_thread == 0 || ctx->realign_rows_per_thread > 32))
         err = hipErrorInvalidImage;
-    // One small block: the error words at offsets 0, 64, 128 and 256
-    // (separate lines), the zero row at 320.
+    // One small block: the error words at offsets 0, 64 and 256 (separate
+    // lines), the zero row at 320.
     constexpr size_t kFlagBlock = 320 + SGLKV_ZERO_ROW_BYTES;
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void **>(&ctx->flag), kFlagBlock);
     if (err == hipSuccess) err = hipMemset(ctx->flag, 0, kFlagBlock);
@@ -553,7 +552,6 @@ extern "C" int32_t sgl_rocm_kv_init(int32_t device, const char *code_object_path
     if (err == hipSuccess) memset(ctx->host_words, 0, kHostWords);
     if (err == hipSuccess) {
         ctx->attn_flag = ctx->flag + 16;
-        ctx->pair_flag = ctx->flag + 32;
         ctx->sync_attn_flag = ctx->flag + 64;
         ctx->zero_row = reinterpret_cast<const uint8_t *>(ctx->flag) + 320;
     }
