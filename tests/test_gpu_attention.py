@@ -154,6 +154,18 @@ class _Case:
         return got, want
 
 
+    def route(self, k, queries, qri, qsl, rso, slots, max_len):
+        """What a call with these arguments launches."""
+        plan = kv.PagedAttentionPlan.for_layer(self.layout, self.layer, len(qri), len(rso) - 1, len(slots), self.qh,
+                                               1.0 / math.sqrt(self.dk), kv.HND if self.hnd else kv.NHD)
+        arrays = dict(queries=queries, query_request_indices=np.asarray(qri, np.uint32),
+                      query_sequence_lengths=np.asarray(qsl, np.uint64),
+                      request_slot_offsets=np.asarray(rso, np.uint64), sequence_slots=np.asarray(slots, np.uint64))
+        bufs = {n: hip.DeviceBuffer.from_array(a) for n, a in arrays.items()}
+        return k.attention_route(plan, max_sequence_length=max_len, pool=self.pool,
+                                 output=hip.DeviceBuffer(plan.output_required_bytes), **bufs)
+
+
 def _random_batch(rng, requests, max_len, slot_count, min_len=1):
     lens = rng.integers(min_len, max_len + 1, size=requests)
     rso = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
@@ -247,16 +259,20 @@ def test_long_sequence_is_split_and_combined(k):
     _check(got2, want, c, 'no length hint')
 
 
-@pytest.mark.parametrize("dk,dv,qh,H", [(128, 128, 32, 8), (64, 64, 16, 2), (256, 256, 8, 2),
-                                        (576, 512, 128, 1)])
-def test_split_records_are_each_counted_once(k, dk, dv, qh, H):
+@pytest.mark.parametrize("shared,body,dk,dv,qh,H", [
+    (False, "staged128", 128, 128, 32, 8), (False, "staged64", 64, 64, 16, 2), (False, "staged256", 256, 256, 8, 2),
+    (False, "latent_exact", 576, 512, 128, 1), (True, "tile128", 128, 128, 32, 8), (True, "tile64", 64, 64, 16, 2),
+    (True, "tile256", 256, 256, 8, 2), (True, "latent_exact", 576, 512, 128, 1)])
+def test_split_records_are_each_counted_once(k, shared, body, dk, dv, qh, H):
     """Values that are constant over 256-token blocks (+-4 plus a little
     noise, a random sign per block) make each split's share of the output
     O(1): a split record that the combine dropped or merged twice would move
     the output by about 4 x that split's weight, far past the error bound.
-    24 queries over one 20,000-token request take every count of splits
+    24 queries over 20,000 tokens take every count of splits
     from 1 to all of them (so every remainder of the combine's groups of
-    eight), on the staged bodies (dims 128, 64, 256) and the latent MLA body."""
+    eight), each of a request of its own over the same slots (the staged
+    bodies, dims 128, 64, 256, and the latent MLA body) or all of one request
+    (the tile bodies)."""
     rng = np.random.default_rng(dk + 31)
     n = 20000
     c = _Case(rng, P=64, L=1, H=H, dk=dk, dv=dv, qh=qh, pages=-(-n // 64) + 4, layer=0)
@@ -276,7 +292,10 @@ def test_split_records_are_each_counted_once(k, dk, dv, qh, H):
     qsl = np.linspace(1, n, nq).astype(np.int64)
     q = _bf16_normal(rng, nq * qh * dk).reshape(nq, qh, dk)
     _say(f"split records counted once: dk={dk} dv={dv} qh={qh}, {nq} queries up to {n} tokens")
-    got, want = c.run(k, q, np.zeros(nq, int), qsl, [0, n], slots, 1.0 / math.sqrt(dk), max_len=n)
+    qri, rso = (np.zeros(nq, int), [0, n]) if shared else (np.arange(nq), n * np.arange(nq + 1))
+    own = slots if shared else np.tile(slots, nq)
+    assert c.route(k, q, qri, qsl, rso, own, n).body == body
+    got, want = c.run(k, q, qri, qsl, rso, own, 1.0 / math.sqrt(dk), max_len=n)
     _check(got, want, c)
 
 

@@ -1,12 +1,14 @@
-"""GPU tests of the paged attention's tile bodies (launches with at least two
+"""GPU tests of the paged attention's tile bodies (launches with several
 queries per request on average: prefill, chunked prefill, drafted tokens)
 against the float64 oracle, under the bound that tests/test_gpu_attention.py
 derives: the outputs' own bf16 rounding plus 2^-12 sum_i w_i |v_i| for the
 fp32 sums (the tile bodies keep hi + lo weights and fp32 split records).
 
-A tile holds up to 128 (query, query head) rows of one request, its tokens
-come in blocks of 64, and the slot table covers 2,048 (dims 64) or 4,096
-tokens, so the sizes below sit at those edges.
+A tile holds up to 128 (query, query head) rows of one request (64 at dims
+256), its tokens come in blocks of 64 (32), the slot table covers 2,048 (dims
+64) or 4,096 tokens, and the search looks at 2,048 queries at a time, so the
+sizes below sit at those edges. Whether a call takes the tile bodies is the
+host's estimate; every test asks which body its call takes.
 """
 import ctypes
 import math
@@ -67,26 +69,59 @@ class _Call:
         return k.attention_route(self.plan, max_sequence_length=self.max_len, output=out, **self.bufs)
 
 
-@pytest.mark.parametrize("H,qh,d,P,hnd,spans", [
-    (2, 8, 128, 16, False, [(0, 1), (0, 2), (0, 31), (0, 32), (0, 33), (0, 63), (0, 64), (0, 65)]),
-    (2, 8, 128, 64, True, [(0, 300), (127, 3), (64, 64), (63, 66)]),
-    (8, 32, 128, 64, False, [(700, 5), (40, 5), (1999, 5), (3, 5)]),     # drafted tokens
-    (2, 14, 64, 16, False, [(0, 129), (2000, 150), (5, 2)]),              # groups of 7, past the slot table
-    (2, 14, 64, 1, True, [(0, 40), (0, 18), (0, 19), (1, 1)]),
-    (1, 64, 128, 64, False, [(4090, 9), (0, 3)]),                         # groups of 64: two queries a tile
-    (4, 4, 64, 64, False, [(0, 200), (0, 128), (77, 127)]),               # one head a group: 128 queries a tile
-    (2, 8, 256, 64, False, [(0, 70), (500, 5), (31, 33)]),
-    (1, 16, 256, 16, True, [(100, 40), (0, 9)]),
-    (1, 48, 128, 1, False, [(0, 21), (64, 2)]),                           # two queries a tile, 32 idle rows
+@pytest.mark.parametrize("body,H,qh,d,P,hnd,spans", [
+    # too few or too short for tiles: the per-query bodies, several queries per request
+    ("staged128", 2, 8, 128, 16, False, [(0, 1), (0, 2), (0, 31), (0, 32), (0, 33), (0, 63), (0, 64), (0, 65)]),
+    ("staged128k", 2, 8, 128, 64, True, [(0, 300), (127, 3), (64, 64), (63, 66)]),
+    ("staged64", 2, 14, 64, 1, True, [(0, 40), (0, 18), (0, 19), (1, 1)]),
+    ("staged64", 4, 4, 64, 64, False, [(0, 200), (0, 128), (77, 127)]),
+    ("staged256", 2, 8, 256, 64, False, [(0, 70), (500, 5), (31, 33)]),
+    ("staged256", 1, 16, 256, 16, True, [(100, 40), (0, 9)]),
+    ("wide128", 1, 64, 128, 64, False, [(4090, 9), (0, 3)]),
+    ("wide128", 1, 48, 128, 1, False, [(0, 21), (64, 2)]),
+    # tiles
+    ("tile128", 8, 32, 128, 16, False, [(0, 1), (0, 2), (0, 31), (0, 32), (0, 33), (0, 63), (0, 64), (0, 65)]),
+    ("tile128", 8, 32, 128, 64, True, [(0, 300), (127, 3), (64, 64), (63, 66)]),
+    ("tile128", 8, 32, 128, 64, False, [(700, 5), (40, 5), (1999, 5), (3, 5)]),    # drafted tokens, split
+    ("tile64", 2, 14, 64, 16, False, [(0, 129), (2000, 150), (5, 2)]),              # groups of 7, split
+    ("tile64", 8, 56, 64, 1, True, [(0, 140), (0, 118), (0, 119), (1, 1)]),
+    ("tile64", 16, 16, 64, 64, False, [(0, 200), (0, 128), (77, 127)]),             # one head a group: 128 queries a tile
+    ("tile128", 1, 64, 128, 64, False, [(90, 200)]),                                # groups of 64: two queries a tile
+    ("tile128", 1, 48, 128, 1, False, [(90, 200)]),                                 # two queries a tile, 32 idle rows
+    ("tile256", 4, 16, 256, 64, False, [(0, 70), (500, 5), (31, 33)]),
+    ("tile256", 2, 32, 256, 16, True, [(1000, 70), (0, 39)]),                       # groups of 16, split
+    ("tile256", 1, 32, 256, 64, False, [(300, 60), (0, 39)]),                       # groups of 32: two queries a tile
+    ("tile64", 2, 14, 64, 16, False, [(0, 1500), (0, 900), (0, 2)]),                # a run cut at the search's step
+    ("tile128", 2, 8, 128, 16, True, [(0, 700)] * 2 + [(300, 2)] * 400),            # both ways of the search, two steps
+    ("tile64", 48, 96, 64, 16, False, [(0, 511)]),                                  # 384 whole tiles: folded over 256 CUs
 ])
-def test_causal_queries(k, H, qh, d, P, hnd, spans):
+def test_causal_queries(k, body, H, qh, d, P, hnd, spans):
     rng = np.random.default_rng(d + qh + len(spans))
     pages = -(-sum(c + n for c, n in spans) // P) + 3
     c = _Case(rng, P=P, L=2, H=H, dk=d, dv=d, qh=qh, pages=pages, layer=1, hnd=hnd)
     qri, qsl, rso, slots = _requests(rng, spans, c.layout.slot_count)
     q = _bf16_normal(rng, len(qri) * qh * d).reshape(len(qri), qh, d)
-    _say(f"tiles H={H} qh={qh} d={d} P={P} hnd={hnd} queries={len(qri)}")
+    _say(f"{body} H={H} qh={qh} d={d} P={P} hnd={hnd} queries={len(qri)}")
+    assert c.route(k, q, qri, qsl, rso, slots, int(qsl.max())).body == body
     got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=int(qsl.max()))
+    _check(got, want, c)
+
+
+@pytest.mark.parametrize("d,length", [(64, 2152), (128, 4202), (256, 4152)])
+def test_splits_longer_than_the_slot_table(k, d, length):
+    """60 requests of two queries each over the same slots: enough tiles that
+    none is split, so each fills its slot table again on the way."""
+    rng = np.random.default_rng(d + 7)
+    c = _Case(rng, P=16, L=1, H=8, dk=d, dv=d, qh=8, pages=length // 16 + 2, layer=0)
+    own = rng.choice(c.layout.slot_count, size=length, replace=False).astype(np.uint64)
+    qri, qsl = np.repeat(np.arange(60), 2), np.tile([length - 1, length], 60)
+    qsl[8:24] -= 3 * np.arange(16)
+    rso, slots = np.arange(61, dtype=np.uint64) * np.uint64(length), np.tile(own, 60)
+    q = _bf16_normal(rng, 120 * 8 * d).reshape(120, 8, d)
+    route = c.route(k, q, qri, qsl, rso, slots, length)
+    assert route.body == f"tile{d}" and route.splits == 1 and route.chunk_tokens > (2048 if d == 64 else 4096)
+    _say(f"tiles past the slot table, d={d}, {length} tokens")
+    got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=length)
     _check(got, want, c)
 
 
@@ -95,15 +130,17 @@ def test_queries_in_any_order(k, d):
     """Runs of one request cut by others, decreasing and repeated lengths,
     and far more tiles than queries that come request by request make."""
     rng = np.random.default_rng(d)
-    c = _Case(rng, P=16, L=1, H=2, dk=d, dv=d, qh=8, pages=120, layer=0)
+    H = 4 if d == 256 else 8
+    c = _Case(rng, P=16, L=1, H=H, dk=d, dv=d, qh=4 * H, pages=120, layer=0)
     lens = np.array([900, 333, 64])
     rso = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
     slots = rng.choice(c.layout.slot_count, size=int(rso[-1]), replace=False).astype(np.uint64)
     qri = np.concatenate([np.arange(90) % 3, np.zeros(70, int), rng.integers(0, 3, 64), np.full(3, 2)])
     qsl = np.array([rng.integers(1, lens[r] + 1) for r in qri])
     qsl[90:160] = np.sort(qsl[90:160])[::-1]
-    q = _bf16_normal(rng, len(qri) * 8 * d).reshape(len(qri), 8, d)
+    q = _bf16_normal(rng, len(qri) * 4 * H * d).reshape(len(qri), 4 * H, d)
     _say(f"tiles in any order, d={d}, {len(qri)} queries")
+    assert c.route(k, q, qri, qsl, rso, slots, 900).body == f"tile{d}"
     got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=900)
     _check(got, want, c)
 
@@ -175,7 +212,8 @@ def test_values_past_a_query_are_not_seen(k, d, bits):
     """Tokens 50 and 180 of a causal prompt hold infinite or NaN keys and
     values: queries that do not attend them are as without them."""
     rng = np.random.default_rng(d + bits)
-    c = _Case(rng, P=16, L=1, H=1, dk=d, dv=d, qh=4, pages=20, layer=0)
+    H = 4 if d == 256 else 8
+    c = _Case(rng, P=16, L=1, H=H, dk=d, dv=d, qh=4 * H, pages=20, layer=0)
     qri, qsl, rso, slots = _requests(rng, [(0, 200)], c.layout.slot_count)
     pool16 = c.pool_h.view(np.uint16)
     for token in (50, 180):
@@ -184,8 +222,9 @@ def test_values_past_a_query_are_not_seen(k, d, bits):
             at, end = c.layout.tensor_token_byte_range(page, 0, tensor, pos)
             pool16[at // 2 + (token % 7):end // 2:5] = bits
     c.pool.upload(c.pool_h)
-    q = _bf16_normal(rng, 200 * 4 * d).reshape(200, 4, d)
+    q = _bf16_normal(rng, 200 * 4 * H * d).reshape(200, 4 * H, d)
     _say(f"tiles with values of 0x{bits:x} past some queries, d={d}")
+    assert c.route(k, q, qri, qsl, rso, slots, 200).body == f"tile{d}"
     with np.errstate(all="ignore"):
         got, want = c.run(k, q, qri, qsl, rso, slots, 1.0 / math.sqrt(d), max_len=200)
     c.absw = c.absw[:50]
@@ -193,32 +232,39 @@ def test_values_past_a_query_are_not_seen(k, d, bits):
     _check(got[:50], want[:50], c)
 
 
-@pytest.mark.parametrize("qri,qsl,flag", [([0] * 40 + [7] + [1] * 40, None, 1), (None, 0, 2), (None, 1000, 2)])
-def test_bad_metadata_is_reported(k, qri, qsl, flag):
-    """A request index past the requests, and lengths of 0 or past the
-    request's slots, raise the reference's flag bits from inside a tile."""
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("what,flag", [("index", 1), ("empty", 2), ("long", 2), ("slot", 4)])
+def test_bad_metadata_is_reported(k, d, what, flag):
+    """A request index past the requests, lengths of 0 or past the request's
+    slots, and a slot past the pool raise the reference's flag bits from
+    inside a tile; the other queries' outputs are written (all but those
+    that attend the bad slot)."""
     rng = np.random.default_rng(9)
-    c = _Case(rng, P=16, L=1, H=2, dk=128, dv=128, qh=8, pages=20, layer=0)
-    slots = rng.choice(c.layout.slot_count, size=200, replace=False).astype(np.uint64)
-    index = np.array(qri if qri else [0] * 40 + [1] * 41)
-    lengths = np.full(81, 60)
-    if qsl is not None:
-        lengths[33] = qsl
-    q = _bf16_normal(rng, 81 * 8 * 128).reshape(81, 8, 128)
+    H = 4 if d == 256 else 8
+    c = _Case(rng, P=16, L=1, H=H, dk=d, dv=d, qh=4 * H, pages=50, layer=0)
+    slots = rng.choice(c.layout.slot_count, size=600, replace=False).astype(np.uint64)
+    index, lengths = np.repeat([0, 1], 130), np.full(260, 160)
+    keep = np.ones(260, bool)
+    if what == "index":
+        index[50] = 7
+    elif what == "slot":
+        slots[70] = c.layout.slot_count
+        keep[:130] = False
+    else:
+        lengths[50] = 0 if what == "empty" else 301
+    if what != "slot":
+        keep[50] = False
+    q = _bf16_normal(rng, 260 * 4 * H * d).reshape(260, 4 * H, d)
+    call = _Call(c, q, index, lengths, [0, 300, 600], slots, 600)
+    assert call.route(k).body == f"tile{d}"
+    out = call.output()
+    _say(f"tiles with a bad {what}, d={d}")
+    call.run(k, out)
     with pytest.raises(kv.KvError) as e:
-        c.run(k, q, index, lengths, [0, 100, 200], slots, 0.1, max_len=2000)
+        k.check_errors()
     assert e.value.variant == "DeviceMetadataInvalid" and e.value.fields[0] == flag
-
-
-def test_bad_slot_is_reported(k):
-    rng = np.random.default_rng(10)
-    c = _Case(rng, P=16, L=1, H=2, dk=128, dv=128, qh=8, pages=20, layer=0)
-    slots = rng.choice(c.layout.slot_count, size=200, replace=False).astype(np.uint64)
-    slots[70] = c.layout.slot_count
-    q = _bf16_normal(rng, 64 * 8 * 128).reshape(64, 8, 128)
-    with pytest.raises(kv.KvError) as e:
-        c.run(k, q, np.zeros(64, int), 100 + np.arange(64), [0, 200], slots, 0.1, max_len=200)
-    assert e.value.variant == "DeviceMetadataInvalid" and e.value.fields[0] == 4
+    written = (out.download(dtype=np.uint16).reshape(260, -1) != 0xFFFF).all(axis=1)
+    assert written[keep].all() and (what == "slot" or not written[50])
 
 
 def _chunk_call(seed, H, qh, d, cached, queries):
@@ -315,3 +361,21 @@ def test_captured_call_is_not_split(k):
     hip.check(h.hipGraphDestroy(graph), "hipGraphDestroy")
     stream.destroy()
     ctx.close()
+
+
+def test_no_allocation_entry_point_splits_alike(k):
+    """Tiles through the no-allocation entry point: the same splits, bit for
+    bit the same result, for a chunk whose queries alone would not be split
+    and for one whose queries would."""
+    for call in (_chunk_call(5, 8, 32, 128, 600, 384), _chunk_call(6, 2, 14, 64, 3000, 100),
+                 _chunk_call(7, 2, 8, 256, 2000, 60)):
+        route = call.route(k)
+        assert route.body.startswith("tile") and route.splits > 1
+        outs = [call.output() for _ in range(2)]
+        _say(f"tiles through the no-allocation entry point: {route}")
+        call.run(k, outs[0])
+        k.paged_attention_async_noalloc(call.plan, max_sequence_length=call.max_len, output=outs[1], **call.bufs)
+        k.check_errors()
+        a, b = (o.download(dtype=np.uint16) for o in outs)
+        assert not np.all(a == 0xFFFF)
+        np.testing.assert_array_equal(a, b)
