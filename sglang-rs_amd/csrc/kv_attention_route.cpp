@@ -179,17 +179,18 @@ bool record_bytes(const sgl_kv_attention_plan_config &c, const sglkv_attn_params
 // the split above is sized for equal lengths, so most queries leave their
 // last splits empty and the chip part idle. With enough work (128 tokens a
 // resident slot, 96 of the shorter dims-64 ones: 24 queries of 62..999 at
-// dims 128, 100 a slot, took 21.1 us so and 20.5 without) the launch numbers the splits that have tokens first (compact).
+// dims 128, 100 a slot, took 21.1 us so and 20.5 without) the launch numbers
+// the splits that have tokens first (compact).
 // Its chunk is the shortest whose live workgroups, at most total / chunk +
 // queries of each query's, fit the resident slots in one round (seventeen
 // twentieths of the staged bodies'): at least 64 tokens (128 for long
 // sequences, whose merge grows) and at most the equal-length chunk for
 // the latent body, between 192 and 512 for the staged ones, whose larger
 // batches take several rounds anyway (where the equal chunk takes one, that;
-// past 32,768 tokens up to the
-// equal-length chunk: 64 splits of the longest are enough, and more only
-// add workgroups without tokens: one of 131,072 tokens among 63 of 1,000
-// 248 us at 512 a split, 181 so; dims 64, one of 65,536, 81 and 67).
+// past 32,768 tokens up to the equal-length chunk: 64 splits of the longest
+// are enough, and more only add workgroups without tokens: one of 131,072
+// tokens among 63 of 1,000 248 us at 512 a split, 181 so; dims 64, one of
+// 65,536, 81 and 67).
 // Measured on MI355X, per layer, before -> after:
 //  - latent, 32 queries of 1,000..8,192 tokens (1,024 -> 672 a split) 125
 //    -> 102 us, 23 of 955..7,643 93 -> 78, 7 of 100..900 (256 -> 64) 43 ->
@@ -205,7 +206,11 @@ bool record_bytes(const sgl_kv_attention_plan_config &c, const sglkv_attn_params
 // Batches nearer one length keep the split above (33 queries of 500..1,300:
 // 33 us either way, 34 with this one; 128 of 2,000..3,000: 239, 250).
 // Their records, up to 9 times those of equal splits (one MLA query of 65,536
-// tokens among 31 of 1,000: 626 MB against 68), stay within `shorter` bytes.
+// tokens among 31 of 1,000: 626 MB against 68), stay within `shorter` bytes,
+// 128 MiB; the chunk is then the shortest that does. That is slower where one
+// MLA sequence is far the longest: 64 queries, one of 30,000 among 1,000s, 195
+// us a layer so, 88 with records of any size (357 with equal splits); 16, one
+// of 20,000, 54 and 44 (126).
 // Returns whether the splits were made shorter.
 bool split_ragged(const sgl_kv_attention_plan_config &c, const Body &body, uint64_t max_len, uint64_t shorter,
                   sglkv_attn_params *params, Split *s) {
@@ -302,13 +307,13 @@ struct TileShape {
 // at least two queries), count tokens in 32 bits and write 8-byte pieces.
 bool tiles_take(const AttentionDevice &device, const sgl_kv_attention_plan_config &c, const sglkv_attn_params &p,
                 uint64_t max_len) {
-    return fast_rows(c, p) && p.dk == p.dv && (p.dk == 64 || p.dk == 128 || p.dk == 256) && reinterpret_cast<uint64_t>(p.queries) % 16 == 0 &&
-                          reinterpret_cast<uint64_t>(p.output) % 8 == 0 && p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) / 2 &&
-                          p.key_token_stride == p.value_token_stride && p.key_token_stride < (1u << 24) &&
-                          c.layout.page_size <= (1u << 24) && c.request_count > 0 && c.query_count / 2 >= c.request_count &&
-                          c.query_count <= SGLKV_ATTN_TILE_QUERIES_MAX &&
-                          c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
-                          SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= device.max_lds;
+    return fast_rows(c, p) && p.dk == p.dv && (p.dk == 64 || p.dk == 128 || p.dk == 256) &&
+           reinterpret_cast<uint64_t>(p.queries) % 16 == 0 && reinterpret_cast<uint64_t>(p.output) % 8 == 0 &&
+           p.group <= SGLKV_ATTN_TILE_ROWS(p.dk) / 2 && p.key_token_stride == p.value_token_stride &&
+           p.key_token_stride < (1u << 24) && c.layout.page_size <= (1u << 24) && c.request_count > 0 &&
+           c.query_count / 2 >= c.request_count && c.query_count <= SGLKV_ATTN_TILE_QUERIES_MAX &&
+           c.query_count <= UINT32_MAX / 512 / p.kv_heads && max_len <= (1u << 30) &&
+           SGLKV_ATTN_TILE_LDS_BYTES(p.dk) <= device.max_lds;
 }
 
 // Whether the tiles are estimated to take less time than `body`, whose work

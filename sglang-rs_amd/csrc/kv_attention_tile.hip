@@ -11,16 +11,19 @@
 // outputs of 32 rows are too many registers for one wave, 64 rows, 32 per pair
 // of waves: both compute the scores, each has half the value dims). Every K and
 // V row is staged in LDS once per tile.
-//  - Tiles. A run is a maximal stretch of consecutive queries of one request
-//    within a step of 2,048; it is cut into tiles of tile_queries from its start, and tiles are
-//    numbered over all runs. Which queries tile t holds is found from
-//    query_request_indices by the workgroup itself (attn_tile_find), so queries of different requests never
-//    share a tile whatever their order, and no planning launch or device list
-//    is needed. Where the queries of a step do not come request by request,
-//    its tiles gather those of a request. The host launches tile_slots tiles per KV head, enough for
-//    queries that come request by request; workgroups step by tile_slots, so
-//    any other order is covered too. Later tiles of a causal prompt attend
-//    more tokens, so the tiles are taken from the last to the first.
+//  - Tiles. The queries are taken in steps of 2,048, each with its own
+//    workgroups (tile_step_slots; the rest of tile_slots for the last step). A
+//    run is a maximal stretch of consecutive queries of one request within a
+//    step; it is cut into tiles of tile_queries from its start, and a step's
+//    tiles are numbered over its runs. Which queries tile t holds is found from
+//    query_request_indices by the workgroup itself (attn_tile_find), so queries
+//    of different requests never share a tile whatever their order, and no
+//    planning launch or device list is needed. Where the queries of a step do
+//    not come request by request, its tiles gather those of a request. The host
+//    launches enough workgroups for queries that come request by request; those
+//    of a step go on by their number, so any other order is covered too. Later
+//    tiles of a causal prompt attend more tokens, so the tiles are taken from
+//    the last to the first.
 //  - q.k: S[token][row] = K (A operand) x Q^T (B operand) with
 //    v_mfma_f32_32x32x16_bf16, the queries in registers. Lane l holds row
 //    l % 32's scores of tokens 8(i/4) + 4(l/32) + i%4, i < 16, of each
@@ -40,17 +43,24 @@
 //    (16 bytes) pc of token t's K row sits at pc ^ kswz(t), of its V row at
 //    pc ^ vswz(t), chosen so that the 16 tokens of a q.k read, and the four
 //    tokens of a half-wave's transposing read, land in distinct banks.
-// What bounds it: the matrix products (48 per 64-token block and wave at dims
-// 128, 32 of them p.v's, hi and lo) and the softmax's vector instructions (about
-// as long), on two waves per SIMD; for short prompts the chain of loads before
-// the first block (about 6 us). Measured on MI355X, per layer, against the
-// per-query bodies:
+// What bounds it, by SQ counters, on two waves per SIMD (dims 64: three):
+//  - long causal prompts, dims 128: a wave's products (48 per 64-token block, 32
+//    of them p.v's, hi and lo) and its softmax follow each other, so neither
+//    pipe is full: matrix cores busy 39 % of the SIMD cycles, vector issue 48 %;
+//    a quarter of a wave's time at the block barrier, no LDS bank conflicts;
+//  - a chunk over a long prefix, dims 64: 26 % and 52 %, a third of the time
+//    waiting for rows;
+//  - a few queries a request, dims 256: waiting for rows, 56 % of a wave's time
+//    (one block in flight, and waves without a row only load).
+// Short calls take the chain of loads before the first block: 4.0 to 6.5 us
+// (fitted, by dims) and 3 us of search where there are several requests.
+// Measured on MI355X, per layer, against the per-query bodies:
 //   causal prompts of 300..2,048 tokens (5,206 queries, 32 heads over 8, dims
-//   128): 1,744 -> 129 us (517 TFLOP/s of q.k and p.v; 688 where 2,048 queries
+//   128): 1,755 -> 125 us (532 TFLOP/s of q.k and p.v; 688 where 2,048 queries
 //   each attend 6,144..8,192 tokens);
 //   384 queries over 6,144 tokens (14 heads over 2, dims 64): 112 -> 33 us;
 //   5 queries of each of 24 requests of 200..3,000 tokens (8 heads over 2, dims
-//   256): 109 -> 41 us.
+//   256): 110 -> 38 us.
 // Of these, the search for the tile's queries in steps of 2,048 (not 128
 // at a time) took the prompts from 185 to 135 us, and products at raised wave
 // priority with the next step's weights scheduled between them 388 -> 350 us on
@@ -107,20 +117,19 @@ constexpr uint32_t kTileWalk = 6;
 constexpr uint32_t kTileGathered = 0xFFFFFFFFu;  // q0 of a tile whose queries are listed
 
 // The nq queries of tile `want` of the step of queries from `base` on, or false
-// if it has fewer tiles (uniform over the workgroup): queries [q0, q0 + nq), or members[0 .. nq) where q0 is
-// kTileGathered. `masks`: 512 bytes of LDS, the list (128 words) behind the
-// first 256;
-// `seen_requests`: 17 KiB, first the step's request indices, from which the
-// tile's own request and end are read without another memory latency.
-// SGLKV_ATTN_TILE_STEP queries a step, whose tiles are numbered by themselves (numbered
-// over all steps, each workgroup looked through those before its own: 1,024
-// queries of each of 128 prompts, 7 a KV head of dims 64, 3,310 us, so 574; 200
-// of each of 5,000 190 ms, so 2.2): each wave
-// ballots where runs start in 8 stretches of 64 queries (its loads all in
-// flight at once: stepping through 128 queries at a time by one wave, each
-// step a memory latency, took most of a short tile's time), then lane l of
-// every wave takes the tiles that start in stretch l and sums over the lanes. A
-// run ends with its step.
+// if it has fewer tiles (uniform over the workgroup): queries [q0, q0 + nq), or
+// those listed where q0 is kTileGathered. `masks`: 512 bytes of LDS, the list
+// (128 words) behind the first 256; `seen_requests`: 17 KiB, first the step's
+// request indices, from which the tile's own request and end are read without
+// another memory latency.
+// The SGLKV_ATTN_TILE_STEP queries of a step have tiles numbered by themselves
+// (numbered over all steps, each workgroup looked through those before its own:
+// 1,024 queries of each of 128 prompts, 7 a KV head of dims 64, 3,310 us, so
+// 574; 200 of each of 5,000 190 ms, so 2.2). Each wave ballots where runs start
+// in 8 stretches of 64 queries (its loads all in flight at once: stepping
+// through 128 queries at a time by one wave, each step a memory latency, took
+// most of a short tile's time), then lane l of every wave takes the tiles that
+// start in stretch l and sums over the lanes. A run ends with its step.
 // A step with more runs than there are requests holds queries of one request
 // apart from each other. Its tiles gather the queries of one request wherever
 // they are in the step: with a tile for each run, 200 queries of each of four
@@ -721,6 +730,8 @@ __device__ __forceinline__ void attn_tile_body() {
         // length. So when a wave whose rows end apart holds an output that is
         // not finite, the rows are done again, one length a round from the
         // longest down: no row then meets a token that it does not attend.
+        // That costs a pass per length: up to tile_queries (at most 128) passes
+        // more for a tile of a causal prompt that reaches such a value.
         auto wave_reduce = [&](uint32_t v, bool most) {
 #pragma unroll
             for (uint32_t d = 1; d < 32; d <<= 1) {
